@@ -32,8 +32,10 @@
 // largest items start first. Tiles that need more than one chunk write unnormalised fp32
 // partials (O, m, l) and a merge kernel combines them (log-sum-exp weights).
 //
-// VALU path (fp32 and any other head_dim): one wave per (row, q-head), a 64-key chunk per
-// step, one key per lane for the scores and the PV sum over the chunk per output dimension.
+// fp32 path (fp32 tensors, head_dim 64 or 128): the fp32 matrix cores, sb_attn_f32.h.
+//
+// VALU path (any other head_dim, alignment or scale): one wave per (row, q-head), a 64-key chunk
+// per step, one key per lane for the scores and the PV sum over the chunk per output dimension.
 
 #include "sb_common.h"
 
@@ -180,6 +182,7 @@ struct AttnArgs {
   int head_dim;
   float scale;
   float scale_log2;           // scale * log2(e)
+  float scale_log2_lo;        // fp32 kernel: what scale_log2 rounds off
   int ksplit;                 // keys per work item after a row tile's first chunk
                               // (multiple of kTileKeys)
   int ksplit_first;           // keys of a row tile's first chunk (multiple of kTileKeys)
@@ -474,16 +477,6 @@ __host__ __device__ inline KeySplit key_split(int64_t n_tiles, int64_t num_kv_he
   const int64_t chunks = (kv_len + ks - 1) / ks;
   return KeySplit{static_cast<int>(ks), static_cast<int>(chunks < 1 ? 1 : chunks)};
 }
-// The device-derived split of a dense call (device_split), from its row-tile count.
-__device__ __forceinline__ void apply_device_split(AttnArgs& a, int64_t n_tiles_live) {
-  if (!a.device_split) return;
-  const KeySplit sp = key_split(n_tiles_live, a.num_kv_heads, a.kv_len, 1, false);
-  a.ksplit = sp.ksplit;
-  a.ksplit_first = sp.ksplit;
-  a.max_chunks = sp.max_chunks;
-  a.n_tiles = n_tiles_live;
-}
-
 // Work-item decode shared by the attention and merge kernels.
 struct Item {
   int kvh;
@@ -504,6 +497,24 @@ __device__ __forceinline__ Item decode_item(const AttnArgs& a, int64_t n_tiles_l
   it.chunk = static_cast<int>(min(rest / n_tiles_live, static_cast<int64_t>(0x7fffffff)));
   it.tile = n_tiles_live - 1 - tile_rev;
   return it;
+}
+
+}  // namespace sb
+
+#include "sb_attn_f32.h"
+
+namespace sb {
+
+// The device-derived split of a dense call (device_split), from its row-tile count.
+template <bool F32>
+__device__ __forceinline__ void apply_device_split(AttnArgs& a, int64_t n_tiles_live) {
+  if (!a.device_split) return;
+  const KeySplit sp = F32 ? key_split_f32(n_tiles_live, a.num_kv_heads, a.kv_len, a.head_dim)
+                          : key_split(n_tiles_live, a.num_kv_heads, a.kv_len, 1, false);
+  a.ksplit = sp.ksplit;
+  a.ksplit_first = sp.ksplit;
+  a.max_chunks = sp.max_chunks;
+  a.n_tiles = n_tiles_live;
 }
 
 // Key-row addressing, fixed per instantiation so that the tile loop carries no branch on it
@@ -551,7 +562,7 @@ attn_mfma_kernel(const AttnBatch batch) {
   const int64_t rows_kv = n_rows * a.group;
   const int64_t n_tiles_live = (rows_kv + TR - 1) / TR;
   if (n_tiles_live <= 0) return;  // no rows (uniform)
-  apply_device_split(a, n_tiles_live);
+  apply_device_split<false>(a, n_tiles_live);
   const Item item = decode_item(a, n_tiles_live, item_b);
   if (item.tile < 0 || item.chunk >= a.max_chunks) return;  // uniform, before any barrier
   const int kvh = item.kvh;
@@ -1198,7 +1209,7 @@ template <int DT, int D>
 __device__ __forceinline__ void merge_unit(const AttnArgs& a, int64_t mb, int64_t n_tiles_live,
                                            int64_t rows_kv, int* red) {
   const int tid = threadIdx.x;
-  const int TR = a.tile_rows;  // 128 or 256
+  const int TR = a.tile_rows;  // 64 (fp32), 128 or 256
   const int parts = TR / 32;
   const int kvh = static_cast<int>(mb % a.num_kv_heads);
   const int64_t rest = mb / a.num_kv_heads;
@@ -1236,28 +1247,36 @@ __device__ __forceinline__ void merge_unit(const AttnArgs& a, int64_t mb, int64_
   float acc[DPT];
 #pragma unroll
   for (int e = 0; e < DPT; ++e) acc[e] = 0.f;
-  float lsum = 0.f;
-  if (nchunks <= kMergeBatch) {
-    // Every chunk's (m, l) and values requested at once: one round trip to memory.
+  float lsum = 0.f, mmax = -INFINITY;
+  // Batches of kMergeBatch chunks: a batch's (m, l) and values are requested at once (one round
+  // trip to memory), then added relative to the largest m so far.
+  for (int c0 = 0; c0 < nchunks; c0 += kMergeBatch) {
     float2 ml[kMergeBatch];
     float4 v[kMergeBatch][DPT / 4];
 #pragma unroll
     for (int ch = 0; ch < kMergeBatch; ++ch) {
-      if (ch < nchunks) {
-        const int64_t slot = (base + ch) * TR + row_in_tile;
+      if (c0 + ch < nchunks) {
+        const int64_t slot = (base + c0 + ch) * TR + row_in_tile;
         ml[ch] = *reinterpret_cast<const float2*>(a.part_ml + slot * 2);
 #pragma unroll
         for (int q = 0; q < DPT / 4; ++q)
           v[ch][q] = *reinterpret_cast<const float4*>(a.part_o + slot * D + d_begin + 4 * q);
       }
     }
-    float mmax = -INFINITY;
+    float mnew = mmax;
 #pragma unroll
     for (int ch = 0; ch < kMergeBatch; ++ch)
-      if (ch < nchunks) mmax = fmaxf(mmax, ml[ch].x);
+      if (c0 + ch < nchunks) mnew = fmaxf(mnew, ml[ch].x);
+    if (c0 > 0 && mnew > mmax && mmax != -INFINITY) {
+      const float alpha = __builtin_amdgcn_exp2f(mmax - mnew);
+      lsum *= alpha;
+#pragma unroll
+      for (int e = 0; e < DPT; ++e) acc[e] *= alpha;
+    }
+    mmax = mnew;
 #pragma unroll
     for (int ch = 0; ch < kMergeBatch; ++ch) {
-      if (ch >= nchunks || ml[ch].x == -INFINITY) continue;
+      if (c0 + ch >= nchunks || ml[ch].x == -INFINITY) continue;
       const float w = __builtin_amdgcn_exp2f(ml[ch].x - mmax);
       lsum += w * ml[ch].y;
 #pragma unroll
@@ -1268,39 +1287,21 @@ __device__ __forceinline__ void merge_unit(const AttnArgs& a, int64_t mb, int64_
         acc[4 * q + 3] += w * v[ch][q].w;
       }
     }
-  } else {
-    float mmax = -INFINITY;
-    for (int ch = 0; ch < nchunks; ++ch)
-      mmax = fmaxf(mmax, a.part_ml[((base + ch) * TR + row_in_tile) * 2]);
-    // Each chunk's DPT values are loaded together (one 16-byte load per four), then weighted.
-    for (int ch = 0; ch < nchunks; ++ch) {
-      const int64_t slot = (base + ch) * TR + row_in_tile;
-      const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + slot * 2);
-      if (ml.x == -INFINITY) continue;
-      const float w = __builtin_amdgcn_exp2f(ml.x - mmax);
-      lsum += w * ml.y;
-      float4 v[DPT / 4];
-#pragma unroll
-      for (int q = 0; q < DPT / 4; ++q)
-        v[q] = *reinterpret_cast<const float4*>(a.part_o + slot * D + d_begin + 4 * q);
-#pragma unroll
-      for (int q = 0; q < DPT / 4; ++q) {
-        acc[4 * q] += w * v[q].x;
-        acc[4 * q + 1] += w * v[q].y;
-        acc[4 * q + 2] += w * v[q].z;
-        acc[4 * q + 3] += w * v[q].w;
-      }
-    }
   }
   const float inv = 1.f / lsum;
   char* op = a.o + qrow * a.o_s_row + qh * a.o_s_head;
 #pragma unroll
   for (int q = 0; q < DPT / 4; ++q) {
-    const uint32_t w0 = static_cast<uint32_t>(Mma<DT>::cvt1(acc[4 * q] * inv)) |
-                        (static_cast<uint32_t>(Mma<DT>::cvt1(acc[4 * q + 1] * inv)) << 16);
-    const uint32_t w1 = static_cast<uint32_t>(Mma<DT>::cvt1(acc[4 * q + 2] * inv)) |
-                        (static_cast<uint32_t>(Mma<DT>::cvt1(acc[4 * q + 3] * inv)) << 16);
-    *reinterpret_cast<uint2*>(op + (d_begin + 4 * q) * 2) = make_uint2(w0, w1);
+    if constexpr (DT == SB_DTYPE_F32) {
+      *reinterpret_cast<float4*>(op + (d_begin + 4 * q) * 4) = make_float4(
+          acc[4 * q] / lsum, acc[4 * q + 1] / lsum, acc[4 * q + 2] / lsum, acc[4 * q + 3] / lsum);
+    } else {
+      const uint32_t w0 = static_cast<uint32_t>(Mma<DT>::cvt1(acc[4 * q] * inv)) |
+                          (static_cast<uint32_t>(Mma<DT>::cvt1(acc[4 * q + 1] * inv)) << 16);
+      const uint32_t w1 = static_cast<uint32_t>(Mma<DT>::cvt1(acc[4 * q + 2] * inv)) |
+                          (static_cast<uint32_t>(Mma<DT>::cvt1(acc[4 * q + 3] * inv)) << 16);
+      *reinterpret_cast<uint2*>(op + (d_begin + 4 * q) * 2) = make_uint2(w0, w1);
+    }
   }
 }
 
@@ -1319,7 +1320,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnBatch batch) 
     merge_unit<DT, D>(a, mb, n_tiles_live, rows_kv, red);
     return;
   }
-  apply_device_split(a, n_tiles_live);
+  apply_device_split<DT == SB_DTYPE_F32>(a, n_tiles_live);
   const int64_t units = n_tiles_live * a.num_kv_heads * (TR / 32);
   for (int64_t u = mb; u < units; u += gridDim.x) {
     merge_unit<DT, D>(a, u, n_tiles_live, rows_kv, red);
@@ -1445,6 +1446,11 @@ bool mfma_path(int32_t dtype, int64_t head_dim) {
          (head_dim == 64 || head_dim == 128);
 }
 
+// fp32 tensors on the fp32 matrix cores (given 16-byte alignment and a positive scale).
+bool f32_path(int32_t dtype, int64_t head_dim) {
+  return dtype == SB_DTYPE_F32 && (head_dim == 64 || head_dim == 128);
+}
+
 // A host-planned launch of the single-request paged attention (sb_partial_attention_paged_plan):
 // the key split (first chunk, later chunks) and the dispatch order of the work items.
 struct OrderPlan {
@@ -1466,16 +1472,17 @@ struct Plan {
 
 Plan make_plan(int64_t rows_upper, int64_t group, int64_t num_kv_heads, int64_t kv_len,
                int64_t head_dim, int64_t block_size, bool paged,
-               const OrderPlan* op = nullptr) {
+               const OrderPlan* op = nullptr, bool f32 = false) {
   Plan pl{};
-  pl.tile_rows = kWaveRows * kRowGroups * kWaves;
+  pl.tile_rows = f32 ? kF32Rows : kWaveRows * kRowGroups * kWaves;
   pl.n_tiles = (rows_upper * group + pl.tile_rows - 1) / pl.tile_rows;
   if (op) {
     pl.ksplit = op->ks_rest;
     pl.ksplit_first = op->ks_first;
     pl.max_chunks = op->max_chunks;
   } else {
-    const KeySplit sp = key_split(pl.n_tiles, num_kv_heads, kv_len, block_size, paged);
+    const KeySplit sp = f32 ? key_split_f32(pl.n_tiles, num_kv_heads, kv_len, head_dim)
+                            : key_split(pl.n_tiles, num_kv_heads, kv_len, block_size, paged);
     pl.ksplit = sp.ksplit;
     pl.ksplit_first = sp.ksplit;
     pl.max_chunks = sp.max_chunks;
@@ -1495,15 +1502,66 @@ struct DeviceSplitBounds {
   int64_t part_rows;  // flattened rows of split-key partials (O rows, then m/l pairs)
 };
 DeviceSplitBounds device_split_bounds(int64_t n_tiles_upper, int64_t num_kv_heads,
-                                      int64_t kv_len, int tile_rows) {
+                                      int64_t kv_len, int tile_rows, int64_t head_dim,
+                                      bool f32) {
   DeviceSplitBounds b{0, 0};
   for (int64_t t = 1; t <= n_tiles_upper; ++t) {
-    const KeySplit sp = key_split(t, num_kv_heads, kv_len, 1, false);
+    const KeySplit sp = f32 ? key_split_f32(t, num_kv_heads, kv_len, head_dim)
+                            : key_split(t, num_kv_heads, kv_len, 1, false);
     b.items = std::max<int64_t>(b.items, t * num_kv_heads * sp.max_chunks);
     if (sp.max_chunks > 1)
       b.part_rows = std::max<int64_t>(b.part_rows, num_kv_heads * t * sp.max_chunks * tile_rows);
   }
   return b;
+}
+
+// The fp32 kernel. Callers that sized no workspace for it (a launch plan is empty for fp32, and
+// a caller may hold a smaller fixed buffer) run unsplit.
+int launch_attention_f32(const char* fn, AttnArgs a, int64_t rows_upper, void* workspace,
+                         int64_t workspace_bytes, hipStream_t st) {
+  const Plan pl = make_plan(rows_upper, a.group, a.num_kv_heads, a.kv_len, a.head_dim,
+                            a.block_size, a.paged != 0, nullptr, true);
+  const double c = static_cast<double>(a.scale) * 1.4426950408889634;
+  a.scale_log2 = static_cast<float>(c);
+  a.scale_log2_lo = static_cast<float>(c - static_cast<double>(a.scale_log2));
+  a.n_tiles = pl.n_tiles;
+  a.tile_rows = pl.tile_rows;
+  a.ksplit = a.ksplit_first = pl.ksplit;
+  a.max_chunks = pl.max_chunks;
+  a.item_order = nullptr;
+  int64_t part_rows =
+      pl.part_bytes > 0 ? a.num_kv_heads * pl.n_tiles * pl.max_chunks * pl.tile_rows : 0;
+  int64_t gx = pl.n_tiles * a.num_kv_heads * pl.max_chunks;
+  if (a.device_split) {
+    const DeviceSplitBounds b =
+        device_split_bounds(pl.n_tiles, a.num_kv_heads, a.kv_len, pl.tile_rows, a.head_dim, true);
+    part_rows = b.part_rows;
+    gx = b.items;
+  }
+  if (part_rows > 0 && (!workspace || workspace_bytes < part_rows * (a.head_dim + 2) * 4)) {
+    a.device_split = 0;
+    a.ksplit = a.ksplit_first = static_cast<int>((a.kv_len + 63) / 64 * 64);
+    a.max_chunks = 1;
+    part_rows = 0;
+    gx = pl.n_tiles * a.num_kv_heads;
+  }
+  if (part_rows > 0) {
+    a.part_o = static_cast<float*>(workspace);
+    a.part_ml = a.part_o + part_rows * static_cast<int64_t>(a.head_dim);
+  }
+  if (gx > 0x7fffffff) return fail(fn, "grid too large");
+  const dim3 grid(static_cast<unsigned>(gx));
+  int64_t mx = pl.n_tiles * a.num_kv_heads * (pl.tile_rows / 32);
+  if (a.device_split) mx = std::min<int64_t>(mx, kMergeStrideGrid);
+  if (mx > 0x7fffffff) return fail(fn, "grid too large");
+  const dim3 mgrid(static_cast<unsigned>(mx));
+  AttnBatch one{};
+  one.a = a;
+#define SB_F32_CASE(D)                                                                        if (a.head_dim == D) {                                                                        if (a.paged)                                                                                  SB_LAUNCH("attn_f32", (attn_f32_kernel<SB_DTYPE_F32, D, true>), grid,                                 dim3(kF32Threads), st, a);                                                      else                                                                                          SB_LAUNCH("attn_f32", (attn_f32_kernel<SB_DTYPE_F32, D, false>), grid,                                dim3(kF32Threads), st, a);                                                      if (part_rows > 0 && a.device_split)                                                          SB_LAUNCH("attn_merge", (attn_merge_kernel<SB_DTYPE_F32, D, true>), mgrid, dim3(256),                 st, one);                                                                       else if (part_rows > 0)                                                                       SB_LAUNCH("attn_merge", (attn_merge_kernel<SB_DTYPE_F32, D, false>), mgrid, dim3(256),                 st, one);                                                                       return check_launch(fn);                                                                  }
+  SB_F32_CASE(64)
+  SB_F32_CASE(128)
+#undef SB_F32_CASE
+  return fail(fn, "internal: no fp32 kernel for this head_dim");
 }
 
 int launch_attention(const char* fn, AttnArgs a, int32_t dtype, int64_t rows_upper,
@@ -1528,7 +1586,7 @@ int launch_attention(const char* fn, AttnArgs a, int32_t dtype, int64_t rows_upp
     if (a.device_split) {
       // The kernels split by the device row count: cover every count that can occur.
       const DeviceSplitBounds b =
-          device_split_bounds(pl.n_tiles, a.num_kv_heads, a.kv_len, pl.tile_rows);
+          device_split_bounds(pl.n_tiles, a.num_kv_heads, a.kv_len, pl.tile_rows, a.head_dim, false);
       part_rows = b.part_rows;
       gx = b.items;
     }
@@ -1562,6 +1620,8 @@ int launch_attention(const char* fn, AttnArgs a, int32_t dtype, int64_t rows_upp
     SB_ATT_CASE(SB_DTYPE_F16, 64)
 #undef SB_ATT_CASE
   }
+  if (f32_path(dtype, a.head_dim) && aligned16 && a.scale_log2 > 0.f && a.kv_len <= 0x7fffff00)
+    return launch_attention_f32(fn, a, rows_upper, workspace, workspace_bytes, st);
   if (a.head_dim > kValuMaxDim) return fail(fn, "head_dim above 512 is not supported");
   if (rows_upper > 0x7fffffff) return fail(fn, "too many rows");
   dim3 grid(static_cast<unsigned>(rows_upper), static_cast<unsigned>(a.num_kv_heads * a.group));
@@ -1636,7 +1696,7 @@ int launch_attention_varlen(const char* fn, AttnArgs a, int32_t dtype, int64_t n
   const VarlenPlan pl = make_varlen_plan(num_reqs, rows, blocks, a.block_size, a.group,
                                          a.num_kv_heads, a.head_dim);
   if (!(mfma_path(dtype, a.head_dim) && aligned16 && a.scale_log2 > 0.f)) {
-    // VALU path: one launch per request.
+    // fp32 and VALU paths: one launch per request.
     for (int r : pl.order) {
       AttnArgs b = a;
       b.positions = a.positions + pl.row_begin[r];
@@ -1719,8 +1779,10 @@ int log2_exact(int64_t v) {
 
 int64_t part_bytes_for(int32_t dtype, int64_t rows_upper, int64_t group, int64_t num_kv_heads,
                        int64_t kv_len, int64_t head_dim, int64_t block_size, bool paged) {
-  if (!mfma_path(dtype, head_dim)) return 0;
-  return make_plan(rows_upper, group, num_kv_heads, kv_len, head_dim, block_size, paged)
+  const bool f32 = f32_path(dtype, head_dim);
+  if (!f32 && !mfma_path(dtype, head_dim)) return 0;
+  return make_plan(rows_upper, group, num_kv_heads, kv_len, head_dim, block_size, paged, nullptr,
+                   f32)
       .part_bytes;
 }
 
@@ -1837,10 +1899,11 @@ extern "C" int64_t sb_partial_prefill_attention_workspace_size(int64_t num_heads
   // positions (S) + count, rounded to 256 bytes, then the split-key partials of the largest
   // split the device row count can select.
   const int64_t idx = ((seq_len + 1) * 4 + 255) / 256 * 256;
-  if (!mfma_path(dtype, head_dim) || num_heads <= 0 || seq_len <= 0) return idx;
-  const int tile_rows = kWaveRows * kRowGroups * kWaves;
-  const DeviceSplitBounds b =
-      device_split_bounds((seq_len + tile_rows - 1) / tile_rows, num_heads, seq_len, tile_rows);
+  const bool f32 = f32_path(dtype, head_dim);
+  if ((!f32 && !mfma_path(dtype, head_dim)) || num_heads <= 0 || seq_len <= 0) return idx;
+  const int tile_rows = f32 ? kF32Rows : kWaveRows * kRowGroups * kWaves;
+  const DeviceSplitBounds b = device_split_bounds((seq_len + tile_rows - 1) / tile_rows, num_heads,
+                                                  seq_len, tile_rows, head_dim, f32);
   return idx + b.part_rows * (head_dim + 2) * 4;
 }
 
@@ -2120,6 +2183,15 @@ extern "C" int64_t sb_partial_attention_paged_varlen_workspace_size(
       num_q_heads % num_kv_heads != 0 || block_size <= 0)
     return 0;
   const int64_t group = num_q_heads / num_kv_heads;
+  if (f32_path(dtype, head_dim)) {  // one launch per request over one workspace
+    int64_t most = 0;
+    for (int64_t r = 0; r < num_reqs; ++r)
+      if (rows_per_req[r] > 0 && blocks_per_req[r] > 0)
+        most = std::max(most, part_bytes_for(dtype, rows_per_req[r], group, num_kv_heads,
+                                             blocks_per_req[r] * block_size, head_dim, block_size,
+                                             true));
+    return most;
+  }
   if (!mfma_path(dtype, head_dim)) return 0;
   return make_varlen_plan(num_reqs, rows_per_req, blocks_per_req, block_size, group,
                           num_kv_heads, head_dim)
@@ -2231,7 +2303,8 @@ extern "C" int sb_partial_attention_paged_noalloc(
   if (num_blocks_per_seq <= 0) return fail(fn, "empty block table or pool");
   const int64_t need = sb_partial_attention_paged_workspace_size(
       num_rows, num_q_heads, num_kv_heads, head_dim, block_size, num_blocks_per_seq, dtype);
-  if (need > kNoAllocScratchBytes)
+  // (fp32 partials past the array's size: the call runs unsplit)
+  if (need > kNoAllocScratchBytes && dtype != SB_DTYPE_F32)
     return fail(fn, "this call needs " + std::to_string(need) +
                         " bytes of split-key partials; the no-allocation entry holds at most " +
                         std::to_string(kNoAllocScratchBytes) +
@@ -2250,6 +2323,7 @@ extern "C" int sb_partial_attention_paged_noalloc(
   a.num_rows = num_rows;
   a.nb_per_seq = num_blocks_per_seq;
   a.kv_len = num_blocks_per_seq * block_size;
-  return launch_attention(fn, a, dtype, num_rows, aligned16, ws, need,
+  return launch_attention(fn, a, dtype, num_rows, aligned16, ws,
+                          std::min(need, kNoAllocScratchBytes),
                           static_cast<hipStream_t>(stream));
 }

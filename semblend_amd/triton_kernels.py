@@ -539,6 +539,7 @@ def partial_prefill_attention_paged(
                             bt.shape[0], q.dtype):
             raise ValueError("plan was made for another shape (rows, heads, head_dim, block "
                              "size, block-table length or dtype)")
+    if plan is not None and plan.max_chunks > 0:  # (an empty plan: no MFMA launch to order)
         ws_bytes = _lib.size_query("sb_partial_attention_paged_planned_workspace_size",
                                    num_rows, num_q_heads, num_kv_heads, head_dim,
                                    plan.max_chunks, dt)

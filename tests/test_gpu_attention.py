@@ -289,3 +289,72 @@ def test_paged_gqa_planned_unsorted_and_fp32(dev):
     with pytest.raises(ValueError, match="another shape"):
         tk.partial_prefill_attention_paged(q.to(dev)[:10], kv.to(dev), bt.to(dev),
                                            pos.to(dev)[:10], plan=plan)
+
+
+# ---- fp32 on the fp32 matrix cores (head_dim 64 and 128) ----
+
+@pytest.mark.parametrize("hq,hkv,d,seq,rows,bs", [
+    (14, 2, 64, 65, 1, 16),       # one row, one key past a 64-key tile
+    (14, 2, 64, 64, 9, 16),       # 63 flattened rows: one short of a row tile
+    (32, 8, 128, 700, 17, 16),    # 68 flattened rows: a second row tile of 4
+    (28, 4, 128, 33, 33, 24),     # every row; blocks that are no power of two
+    (4, 4, 128, 4096, 3, 32),     # few rows of a long context: many key chunks
+    (4, 4, 64, 700, 700, 16),     # no GQA, every row
+    (64, 16, 64, 2000, 1100, 16)])  # enough row tiles to run unsplit
+def test_paged_fp32_tiles_and_splits(dev, hq, hkv, d, seq, rows, bs):
+    """Row tiles of 64, key tiles of 4096 / head_dim and the key split at their edges; a call
+    whose caller sized no workspace (an empty launch plan through the C entry) runs unsplit."""
+    q, kv, bt, pos = _paged_case(hq, hkv, d, seq, rows, torch.float32, 400 + d + rows, bs=bs)
+    qd, kvd, btd, posd = q.to(dev), kv.to(dev), bt.to(dev), pos.to(dev)
+    want = ref.partial_attention_paged(q, kv, bt, pos)
+    got = tk.partial_prefill_attention_paged(qd, kvd, btd, posd)
+    # two orders of summing d products and up to seq weighted values: a few 2^-24 of |out| <= 1
+    assert float((got.cpu() - want).abs().max()) <= 5e-6 * max(1.0, float(want.abs().max()))
+    out = torch.full_like(qd, float("nan"))
+    from semblend_amd import _lib
+    _lib.call("sb_partial_attention_paged_planned", out.data_ptr(), qd.data_ptr(),
+              kvd.data_ptr(), btd.data_ptr(), posd.data_ptr(), None, 0, 0, 0, 0, None, 0,
+              q.shape[0], hq, hkv, d, bs, kv.shape[0], bt.shape[0], 1.0 / math.sqrt(d),
+              _lib.strides(qd), _lib.strides(out), _lib.strides(kvd), _lib.dtype_code(qd),
+              _lib.stream_handle(dev))
+    assert float((out.cpu() - want).abs().max()) <= 5e-6 * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_fp32_masked_keys_never_reach_a_row(dev, d):
+    """NaN and infinite K / V at positions past a row (but inside its key tile) leave the row as
+    it is without them; a row that does attend them takes the same non-finite elements."""
+    h, s = 2, 200
+    q, k, v = (randn((h, s, d), torch.float32, 430 + i) for i in range(3))
+    v[0, 100, 3], v[1, 150, 5] = float("nan"), float("inf")
+    k[0, 120, 1], v[0, 199] = float("nan"), float("-inf")
+    for rows in ([90, 99, 100, 119, 120, 149, 150, 198, 199], [60, 110]):
+        mask = torch.zeros(s, dtype=torch.bool)
+        mask[rows] = True
+        got = tk.partial_prefill_attention(q.to(dev), k.to(dev), v.to(dev), mask.to(dev)).cpu()
+        for hh in range(h):
+            for p in rows:
+                w = torch.softmax((k[hh, :p + 1].double() @ q[hh, p].double()) / math.sqrt(d), 0)
+                want = (w[:, None] * v[hh, :p + 1].double()).sum(0)
+                fin = torch.isfinite(want)
+                assert torch.equal(torch.isnan(got[hh, p]), torch.isnan(want)), (hh, p)
+                assert torch.equal(torch.isfinite(got[hh, p]), fin), (hh, p)
+                assert float((got[hh, p].double() - want)[fin].abs().max().nan_to_num(0)
+                             if fin.any() else 0) <= 1e-5
+
+
+def test_fp32_rising_scores_and_strided_inputs(dev):
+    """Scores that rise along the context move the row maximum in every tile; query and cache
+    are views with a wider head stride."""
+    hq, hkv, d, ctx = 8, 2, 64, 1500
+    kv = randn((100, 2, hkv, 16, 2 * d), torch.float32, 440)[..., :d]
+    kv[:, 0] *= torch.linspace(0.2, 8.0, 100)[:, None, None, None]
+    bt = torch.arange(94, dtype=torch.int32)
+    pos = recompute_set(ctx, 130, 441, chunk=16)
+    q = randn((pos.shape[0], hq, 2 * d), torch.float32, 442)[..., :d]
+    big = torch.zeros((100, 2, hkv, 16, 2 * d), device=dev)
+    big[..., :d] = kv.to(dev)
+    bq = torch.zeros((pos.shape[0], hq, 2 * d), device=dev)
+    bq[..., :d] = q.to(dev)
+    got = tk.partial_prefill_attention_paged(bq[..., :d], big[..., :d], bt.to(dev), pos.to(dev))
+    assert_attn_close(got, ref.partial_attention_paged(q, kv, bt, pos))
