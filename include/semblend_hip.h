@@ -115,6 +115,60 @@ int sb_masked_qkv_projection(void* out, const void* hidden, const void* weight, 
                              int64_t out_features, int64_t hidden_stride, int64_t weight_stride,
                              int64_t out_stride, int32_t dtype, void* stream);
 
+/* The dense form for rows compacted by the caller: positions (device int32, seq_len entries and
+ * then their count, as sb_prefill_index writes them) name the hidden rows to multiply and the
+ * rows of `out` to write; other rows of `out` are left as they are. Same shapes and alignment as
+ * sb_masked_qkv_projection. */
+int sb_qkv_projection_rows(void* out, const void* hidden, const void* weight, const void* bias,
+                           const int32_t* positions, int64_t seq_len, int64_t hidden_dim,
+                           int64_t out_features, int64_t hidden_stride, int64_t weight_stride,
+                           int64_t out_stride, int32_t dtype, void* stream);
+
+/* ------------------------------------------------------------------------------------------
+ * Stages of the single-layer partial prefill (semblend_core/triton_kernels.py:769-923)
+ * ---------------------------------------------------------------------------------------- */
+
+/* index[t] (t < seq_len) = -2 where compute_mask[t], else the donor row of the last pair with
+ * target_pos == t and 0 <= donor_pos < donor_seq_len, else -1; positions[0..count) = the
+ * computed positions ascending, positions[seq_len] = their count (seq_len + 1 entries). */
+int sb_prefill_index(const uint8_t* compute_mask, const int32_t* donor_pos,
+                     const int32_t* target_pos, int64_t num_pairs, int64_t seq_len,
+                     int64_t donor_seq_len, int32_t* index, int32_t* positions, void* stream);
+
+/* The target cache [num_layers, 2, num_heads, seq_len, head_dim] (contiguous), every row written
+ * once: the donor's row index[t] (d_strides[5] = layer, kv, head, seq, dim), the new K / V of
+ * qkv row t ([seq_len, 3, num_heads, head_dim], row stride qkv_stride) in every layer where
+ * index[t] == -2, zeros where it is -1. Rows are 16 bytes times a power of two, 16-byte
+ * aligned. */
+int sb_prefill_assemble(void* cache, const void* donor, const void* qkv, const int32_t* index,
+                        int64_t num_layers, int64_t num_heads, int64_t seq_len,
+                        int64_t head_dim, const int64_t* d_strides, int64_t qkv_stride,
+                        int32_t dtype, void* stream);
+
+/* Causal attention of the rows listed in `positions` (as above) with Q, K and V [num_heads,
+ * seq_len, head_dim] of any dtype, fp32 products, weights and sums, and fp32 output (strides
+ * head, seq, dim in elements); other output rows are left as they are. head_dim 64 or 128,
+ * scale > 0, rows aligned to four elements. `workspace` holds split-key partials:
+ * sb_partial_prefill_attention_workspace_size(..., SB_DTYPE_F32) bytes are enough, and with less
+ * the call runs unsplit. */
+int sb_partial_attention_rows_f32(float* out, const void* q, const void* k, const void* v,
+                                  const int32_t* positions, void* workspace,
+                                  int64_t workspace_bytes, int64_t num_heads, int64_t seq_len,
+                                  int64_t head_dim, float scale, const int64_t* q_strides,
+                                  const int64_t* k_strides, const int64_t* v_strides,
+                                  const int64_t* o_strides, int32_t dtype, void* stream);
+
+/* out[p] = attn[p] . W^T (+ bias) in fp32, rounded to dtype, for the positions listed in
+ * `positions`; zeros in the rows where compute_mask is 0. attn [seq_len, in_features] fp32,
+ * W [out_features, in_features] and out [seq_len, out_features] of dtype, bias fp32 or NULL;
+ * in_features a multiple of 16, out_features of 4, rows aligned to four elements. */
+int sb_prefill_output_projection(void* out, const float* attn, const void* weight,
+                                 const float* bias, const uint8_t* compute_mask,
+                                 const int32_t* positions, int64_t seq_len, int64_t in_features,
+                                 int64_t out_features, int64_t attn_stride,
+                                 int64_t weight_stride, int64_t out_stride, int32_t dtype,
+                                 void* stream);
+
 /* Compacted GQA QKV projection fused with the new K/V write: for each row n the hidden row
  * p = positions[n] is projected with W [(Hq + 2 Hkv) * D, hidden_dim] (+ bias), features
  * laid out Q | K | V. With inv_freq (device fp32 [D/2]), Q and K are rotated by p with the

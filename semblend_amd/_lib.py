@@ -99,6 +99,15 @@ SIGNATURES: dict[str, list] = {
     "sb_qkv_gather_rows": [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _i32, _vp],
     "sb_qkv_epilogue_paged": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp,
                               _vp, _i64, _i64, _i64, _i64, _i64, _i64p, _i32, _vp],
+    "sb_qkv_projection_rows": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64,
+                               _i32, _vp],
+    "sb_prefill_index": [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp],
+    "sb_prefill_assemble": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64p, _i64, _i32,
+                            _vp],
+    "sb_partial_attention_rows_f32": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64,
+                                      _f32, _i64p, _i64p, _i64p, _i64p, _i32, _vp],
+    "sb_prefill_output_projection": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64,
+                                     _i64, _i64, _i32, _vp],
     "sb_device_copy": [_vp, _vp, _i64, _vp],
     "sb_kernel_timing_enable": [_i32],
     "sb_kernel_timing_read": [ctypes.c_char_p, ctypes.POINTER(ctypes.c_double), _i64p],

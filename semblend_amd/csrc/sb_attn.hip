@@ -1515,10 +1515,12 @@ DeviceSplitBounds device_split_bounds(int64_t n_tiles_upper, int64_t num_kv_head
   return b;
 }
 
-// The fp32 kernel. Callers that sized no workspace for it (a launch plan is empty for fp32, and
+// The fp32 kernel, on tensors of `in_dtype` (fp16 / bf16 elements are widened as they are staged:
+// the same results as on fp32 copies of them). Callers that sized no workspace for it (a launch plan is empty for fp32, and
 // a caller may hold a smaller fixed buffer) run unsplit.
 int launch_attention_f32(const char* fn, AttnArgs a, int64_t rows_upper, void* workspace,
-                         int64_t workspace_bytes, hipStream_t st) {
+                         int64_t workspace_bytes, hipStream_t st,
+                         int32_t in_dtype = SB_DTYPE_F32) {
   const Plan pl = make_plan(rows_upper, a.group, a.num_kv_heads, a.kv_len, a.head_dim,
                             a.block_size, a.paged != 0, nullptr, true);
   const double c = static_cast<double>(a.scale) * 1.4426950408889634;
@@ -1557,11 +1559,27 @@ int launch_attention_f32(const char* fn, AttnArgs a, int64_t rows_upper, void* w
   const dim3 mgrid(static_cast<unsigned>(mx));
   AttnBatch one{};
   one.a = a;
-#define SB_F32_CASE(D)                                                                        if (a.head_dim == D) {                                                                        if (a.paged)                                                                                  SB_LAUNCH("attn_f32", (attn_f32_kernel<SB_DTYPE_F32, D, true>), grid,                                 dim3(kF32Threads), st, a);                                                      else                                                                                          SB_LAUNCH("attn_f32", (attn_f32_kernel<SB_DTYPE_F32, D, false>), grid,                                dim3(kF32Threads), st, a);                                                      if (part_rows > 0 && a.device_split)                                                          SB_LAUNCH("attn_merge", (attn_merge_kernel<SB_DTYPE_F32, D, true>), mgrid, dim3(256),                 st, one);                                                                       else if (part_rows > 0)                                                                       SB_LAUNCH("attn_merge", (attn_merge_kernel<SB_DTYPE_F32, D, false>), mgrid, dim3(256),                 st, one);                                                                       return check_launch(fn);                                                                  }
-  SB_F32_CASE(64)
-  SB_F32_CASE(128)
+#define SB_F32_CASE(IT, D, PAGED)                                                         \
+  if (in_dtype == IT && a.head_dim == D && (a.paged != 0) == PAGED) {                     \
+    SB_LAUNCH("attn_f32", (attn_f32_kernel<IT, D, PAGED>), grid, dim3(kF32Threads), st, a); \
+    if (part_rows > 0 && a.device_split)                                                  \
+      SB_LAUNCH("attn_merge", (attn_merge_kernel<SB_DTYPE_F32, D, true>), mgrid,          \
+                dim3(256), st, one);                                                      \
+    else if (part_rows > 0)                                                               \
+      SB_LAUNCH("attn_merge", (attn_merge_kernel<SB_DTYPE_F32, D, false>), mgrid,         \
+                dim3(256), st, one);                                                      \
+    return check_launch(fn);                                                              \
+  }
+  SB_F32_CASE(SB_DTYPE_F32, 64, true)
+  SB_F32_CASE(SB_DTYPE_F32, 128, true)
+  SB_F32_CASE(SB_DTYPE_F32, 64, false)
+  SB_F32_CASE(SB_DTYPE_F32, 128, false)
+  SB_F32_CASE(SB_DTYPE_F16, 64, false)
+  SB_F32_CASE(SB_DTYPE_F16, 128, false)
+  SB_F32_CASE(SB_DTYPE_BF16, 64, false)
+  SB_F32_CASE(SB_DTYPE_BF16, 128, false)
 #undef SB_F32_CASE
-  return fail(fn, "internal: no fp32 kernel for this head_dim");
+  return fail(fn, "internal: no fp32 kernel for this head_dim and dtype");
 }
 
 int launch_attention(const char* fn, AttnArgs a, int32_t dtype, int64_t rows_upper,
@@ -1985,6 +2003,61 @@ extern "C" int sb_partial_prefill_attention(void* out, const void* q, const void
   return launch_attention(fn, a, dtype, seq_len, aligned16,
                           static_cast<char*>(workspace) + idx_bytes,
                           workspace_bytes - idx_bytes, st);
+}
+
+// Dense attention of compacted rows in fp32 arithmetic with fp32 output, Q / K / V in any dtype.
+extern "C" int sb_partial_attention_rows_f32(float* out, const void* q, const void* k,
+                                             const void* v, const int32_t* positions,
+                                             void* workspace, int64_t workspace_bytes,
+                                             int64_t num_heads, int64_t seq_len,
+                                             int64_t head_dim, float scale, const int64_t* qs,
+                                             const int64_t* ks, const int64_t* vs,
+                                             const int64_t* os, int32_t dtype, void* stream) {
+  const char* fn = "sb_partial_attention_rows_f32";
+  clear_error();
+  if (num_heads == 0 || seq_len == 0) return SB_OK;
+  if (elem_size(dtype) == 0) return fail(fn, "invalid dtype");
+  if (!out || !q || !k || !v || !positions || !qs || !ks || !vs || !os)
+    return fail(fn, "null pointer argument");
+  if (num_heads < 0 || seq_len < 0 || seq_len > 0x7fffff00) return fail(fn, "invalid sizes");
+  if (!f32_path(SB_DTYPE_F32, head_dim)) return fail(fn, "head_dim must be 64 or 128");
+  if (!(scale * 1.4426950408889634f > 0.f)) return fail(fn, "scale must be positive");
+  if (qs[2] != 1 || ks[2] != 1 || vs[2] != 1 || os[2] != 1)
+    return fail(fn, "head_dim must be contiguous (stride 1)");
+  const int64_t es = elem_size(dtype);
+  if (vec_bytes({reinterpret_cast<int64_t>(q), reinterpret_cast<int64_t>(k),
+                 reinterpret_cast<int64_t>(v), qs[0] * es, qs[1] * es, ks[0] * es, ks[1] * es,
+                 vs[0] * es, vs[1] * es}) < 4 * es ||
+      vec_bytes({reinterpret_cast<int64_t>(out), os[0] * 4, os[1] * 4}) < 16)
+    return fail(fn, "rows must be aligned to four elements");
+  AttnArgs a{};
+  a.q = static_cast<const char*>(q);
+  a.o = reinterpret_cast<char*>(out);
+  a.q_s_row = qs[1] * es;
+  a.q_s_head = qs[0] * es;
+  a.o_s_row = os[1] * 4;
+  a.o_s_head = os[0] * 4;
+  a.q_by_position = 1;
+  a.positions = positions;
+  a.count_ptr = positions + seq_len;
+  a.num_rows = seq_len;
+  a.k = static_cast<const char*>(k);
+  a.v = static_cast<const char*>(v);
+  a.k_s_head = ks[0] * es;
+  a.v_s_head = vs[0] * es;
+  a.k_s_seq = ks[1] * es;
+  a.v_s_seq = vs[1] * es;
+  a.block_size = 1;
+  a.bs_log2 = -1;
+  a.kv_len = seq_len;
+  a.num_kv_heads = static_cast<int>(num_heads);
+  a.group = 1;
+  a.head_dim = static_cast<int>(head_dim);
+  a.scale = scale;
+  a.scale_log2 = scale * 1.4426950408889634f;
+  a.device_split = 1;  // the row count is known on the device only
+  return launch_attention_f32(fn, a, seq_len, workspace, workspace_bytes,
+                              static_cast<hipStream_t>(stream), dtype);
 }
 
 extern "C" int64_t sb_partial_attention_paged_workspace_size(int64_t num_rows,

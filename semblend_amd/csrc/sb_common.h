@@ -189,10 +189,9 @@ __device__ __forceinline__ void sincos_rn(float x, float* s, float* c) {
 // into ascending positions (+ count) in one workgroup, and write zeros into the output rows
 // whose mask entry is 0 (rows of [heads, seq, ...] under byte strides).
 // ---------------------------------------------------------------------------------------
-template <int kUnused = 0>
-__global__ __launch_bounds__(1024) void mask_compact_kernel(const uint8_t* mask, int64_t n,
-                                                            int32_t* pos_out,
-                                                            int32_t* count_out) {
+// One workgroup of 1024 threads (mask_compact_kernel, or a workgroup of a larger launch).
+__device__ __forceinline__ void mask_compact_unit(const uint8_t* mask, int64_t n,
+                                                  int32_t* pos_out, int32_t* count_out) {
   // Each thread takes 16 consecutive mask bytes per round (one 16-byte load when the mask is
   // 16-byte aligned), so a round covers 16384 positions; a wave scan of the per-thread
   // counts and the per-wave totals in LDS give every thread its output offset.
@@ -243,6 +242,13 @@ __global__ __launch_bounds__(1024) void mask_compact_kernel(const uint8_t* mask,
     __syncthreads();
   }
   if (tid == 0) *count_out = base;
+}
+
+template <int kUnused = 0>
+__global__ __launch_bounds__(1024) void mask_compact_kernel(const uint8_t* mask, int64_t n,
+                                                            int32_t* pos_out,
+                                                            int32_t* count_out) {
+  mask_compact_unit(mask, n, pos_out, count_out);
 }
 
 template <int VB>

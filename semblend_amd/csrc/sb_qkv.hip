@@ -812,6 +812,21 @@ int launch_qkv_epilogue(const char* fn, const QkvArgs& a, const float* proj, int
   return check_launch(fn);
 }
 
+// The dense form over compacted positions [seq_len] followed by their count (device).
+int launch_qkv_dense(const char* fn, QkvArgs a, const int32_t* positions, void* out,
+                     int64_t out_stride, int32_t dtype, hipStream_t st) {
+  a.positions = positions;
+  a.count = positions + a.seq_len;
+  a.num_rows = a.seq_len;
+  a.q_features = a.num_features;  // every feature goes to the dense row; no RoPE
+  a.kv_features = 0;
+  a.head_dim = 8;
+  a.out = static_cast<char*>(out);
+  a.o_s_row = out_stride * 2;
+  return launch_qkv<QKV_DENSE>(fn, a, dtype, st,
+                               qkv_plan(a.num_rows, a.num_features, a.k_steps, false));
+}
+
 // Workspace of the split form: the RoPE table first, then (split product) the slices.
 constexpr int64_t kQkvWsAlign = 256;
 int64_t qkv_table_bytes(int64_t num_rows, int64_t head_dim, bool rope) {
@@ -1032,13 +1047,28 @@ extern "C" int sb_masked_qkv_projection(void* out, const void* hidden, const voi
             seq_len, pos, pos + seq_len);
   rc = check_launch(fn);
   if (rc) return rc;
-  a.positions = pos;
-  a.count = pos + seq_len;
-  a.num_rows = seq_len;
-  a.q_features = out_features;  // every feature goes to the dense row; no RoPE
-  a.kv_features = 0;
-  a.head_dim = 8;
-  a.out = static_cast<char*>(out);
-  a.o_s_row = out_stride * 2;
-  return launch_qkv<QKV_DENSE>(fn, a, dtype, st, qkv_plan(a.num_rows, a.num_features, a.k_steps, false));
+  return launch_qkv_dense(fn, a, pos, out, out_stride, dtype, st);
+}
+
+// The dense form for rows the caller has compacted: positions[0..count) with the count at
+// positions[seq_len] (both on the device); other rows of `out` are left as they are.
+extern "C" int sb_qkv_projection_rows(void* out, const void* hidden, const void* weight,
+                                      const void* bias, const int32_t* positions,
+                                      int64_t seq_len, int64_t hidden_dim,
+                                      int64_t out_features, int64_t hidden_stride,
+                                      int64_t weight_stride, int64_t out_stride, int32_t dtype,
+                                      void* stream) {
+  const char* fn = "sb_qkv_projection_rows";
+  clear_error();
+  if (seq_len == 0) return SB_OK;
+  if (seq_len < 0) return fail(fn, "invalid sizes");
+  if (!out || !positions) return fail(fn, "null pointer argument");
+  QkvArgs a{};
+  const int rc = qkv_common(fn, &a, hidden, weight, bias, seq_len, hidden_dim, out_features,
+                            hidden_stride, weight_stride, dtype);
+  if (rc) return rc;
+  if (reinterpret_cast<uintptr_t>(out) % 16 || (out_stride * 2) % 16)
+    return fail(fn, "output rows must be 16-byte aligned");
+  return launch_qkv_dense(fn, a, positions, out, out_stride, dtype,
+                          static_cast<hipStream_t>(stream));
 }

@@ -745,8 +745,152 @@ def partial_prefill(
         cast to the input dtype, with reuse rows zeroed;
     (5) the new K/V are written into the compute rows of EVERY layer of the target cache.
     Attention uses layer 0 only, as in the reference.
+
+    head_dim 64 or 128 with one dtype throughout runs as six launches that touch the cache once
+    (``_prefill_stages``); other calls, and calls that record gradients, compose the stages
+    from this module's functions and torch (``_prefill_composed``), with the same results.
     """
     dev = _lib.require_device(hidden_states, donor_kv, qkv_weight, output_projection)
+    args = (hidden_states, donor_kv, qkv_weight, output_projection, donor_positions,
+            target_positions, compute_mask, num_heads, head_dim, qkv_bias, output_bias, scale)
+    if _prefill_stages_ok(*args):
+        return _prefill_stages(dev, *args)
+    return _prefill_composed(dev, *args)
+
+
+def _prefill_stages_ok(hidden_states, donor_kv, qkv_weight, output_projection, donor_positions,
+                       target_positions, compute_mask, num_heads, head_dim, qkv_bias,
+                       output_bias, scale) -> bool:
+    """Whether a call fits the kernels of :func:`_prefill_stages` (shapes, dtypes, alignment)
+    and records no gradient. A call that does not is composed, or rejected there."""
+    dt = hidden_states.dtype
+    if head_dim not in (64, 128) or dt not in _lib.SB_DTYPE or num_heads < 1:
+        return False
+    if donor_kv.dtype != dt or qkv_weight.dtype != dt or output_projection.dtype != dt:
+        return False
+    if hidden_states.dim() != 2 or donor_kv.dim() != 5 or output_projection.dim() != 2:
+        return False
+    seq_len, hidden = hidden_states.shape
+    feats = num_heads * head_dim
+    layers = donor_kv.shape[0]
+    es = hidden_states.element_size()
+    if (seq_len < 1 or not 1 <= layers <= 32767 or seq_len > 1 << 20
+            or tuple(qkv_weight.shape) != (3 * feats, hidden)
+            or tuple(donor_kv.shape[1:3]) != (2, num_heads) or donor_kv.shape[4] != head_dim
+            or donor_kv.stride(4) != 1 or donor_kv.data_ptr() % 16
+            or any(s * es % 16 for s in donor_kv.stride()[:4])):
+        return False
+    if (output_projection.shape[1] != feats or output_projection.shape[0] % 4
+            or output_projection.stride(1) != 1 or output_projection.data_ptr() % 16
+            or output_projection.stride(0) * es % 16):
+        return False
+    for b, n in ((qkv_bias, 3 * feats), (output_bias, output_projection.shape[0])):
+        if b is not None and (tuple(b.shape) != (n,) or not b.is_cuda):
+            return False
+    if not isinstance(compute_mask, torch.Tensor) or tuple(compute_mask.shape) != (seq_len,):
+        return False
+    if len(donor_positions) != len(target_positions):
+        return False
+    if scale is not None and not float(scale) * 1.4426950408889634 > 1e-37:
+        return False
+    return not (torch.is_grad_enabled() and any(
+        t is not None and t.requires_grad
+        for t in (hidden_states, donor_kv, qkv_weight, output_projection, qkv_bias, output_bias)))
+
+
+def _prefill_stages(dev, hidden_states, donor_kv, qkv_weight, output_projection,
+                    donor_positions, target_positions, compute_mask, num_heads, head_dim,
+                    qkv_bias, output_bias, scale) -> PartialPrefillResult:
+    """:func:`partial_prefill` on its own kernels: projection of the computed rows, the cache
+    assembled in one pass (donor rows, new K/V, zeros), fp32 attention of the computed rows
+    over layer 0 of that cache and their fp32 output projection."""
+    seq_len, hidden = hidden_states.shape
+    num_layers = donor_kv.shape[0]
+    feats = num_heads * head_dim
+    dt = hidden_states.dtype
+    if scale is None:
+        scale = 1.0 / math.sqrt(head_dim)
+    mask = compute_mask.to(device=dev)
+    mask = (mask if mask.dtype == torch.bool else mask != 0).contiguous()
+    num_pairs = len(donor_positions)
+    dpos = tpos = None
+    if num_pairs:
+        dpos = _lib.as_index(donor_positions, dev)
+        tpos = _lib.as_index(target_positions, dev)
+    fused = (dt != torch.float32 and hidden % 64 == 0
+             and (qkv_bias is None or qkv_bias.dtype == dt)
+             and _mfma_rows_ok(hidden_states, qkv_weight))
+    code = _lib.dtype_code(hidden_states)
+    ws_bytes = _lib.size_query("sb_partial_prefill_attention_workspace_size", num_heads,
+                               seq_len, head_dim, _lib.SB_DTYPE[torch.float32])
+    part_at = ((seq_len + 1) * 4 + 255) // 256 * 256
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)  # positions, count, partials
+    index = torch.empty(seq_len, dtype=torch.int32, device=dev)
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(5)]
+    es = hidden_states.element_size()
+    with _lib.on_device(dev):
+        stream = torch.cuda.current_stream(dev)
+        st = stream.cuda_stream
+        pos = ws.data_ptr()
+        ev[0].record(stream)
+        _lib.call("sb_prefill_index", mask.data_ptr(), _lib.ptr(dpos), _lib.ptr(tpos),
+                  num_pairs, seq_len, donor_kv.shape[3], index.data_ptr(), pos, st)
+        ev[1].record(stream)
+        if fused:
+            qkv = torch.empty((seq_len, 3 * feats), dtype=dt, device=dev)
+            bias = None if qkv_bias is None else qkv_bias.contiguous()
+            _lib.call("sb_qkv_projection_rows", qkv.data_ptr(), hidden_states.data_ptr(),
+                      qkv_weight.data_ptr(), _lib.ptr(bias), pos, seq_len, hidden, 3 * feats,
+                      hidden_states.stride(0), qkv_weight.stride(0), 3 * feats, code, st)
+        else:
+            # (reuse rows are projected as well; none of them is read)
+            qkv = torch.nn.functional.linear(
+                hidden_states.float(), qkv_weight.float(),
+                None if qkv_bias is None else qkv_bias.float()).to(dt)
+        ev[2].record(stream)
+        # (the first launches are under way while the rest is allocated)
+        cache = torch.empty((num_layers, 2, num_heads, seq_len, head_dim), dtype=dt, device=dev)
+        _lib.call("sb_prefill_assemble", cache.data_ptr(), donor_kv.data_ptr(), qkv.data_ptr(),
+                  index.data_ptr(), num_layers, num_heads, seq_len, head_dim,
+                  _lib.strides(donor_kv), 3 * feats, code, st)
+        ev[3].record(stream)
+        attn = torch.empty((seq_len, feats), dtype=torch.float32, device=dev)
+        out = torch.empty((seq_len, output_projection.shape[0]), dtype=dt, device=dev)
+        bias32 = None if output_bias is None else output_bias.float().contiguous()
+        count = torch.empty(4, dtype=torch.uint8, pin_memory=True)
+        heads_major = _lib.i64_array((seq_len * head_dim, head_dim, 1))
+        _lib.call("sb_partial_attention_rows_f32", attn.data_ptr(), qkv.data_ptr(),
+                  cache.data_ptr(), cache.data_ptr() + feats * seq_len * es, pos,
+                  pos + part_at, ws_bytes - part_at, num_heads, seq_len, head_dim,
+                  float(scale), _lib.i64_array((head_dim, 3 * feats, 1)), heads_major,
+                  heads_major, _lib.i64_array((head_dim, feats, 1)), code, st)
+        _lib.call("sb_prefill_output_projection", out.data_ptr(), attn.data_ptr(),
+                  output_projection.data_ptr(), _lib.ptr(bias32), mask.data_ptr(), pos,
+                  seq_len, feats, output_projection.shape[0], feats,
+                  output_projection.stride(0), out.stride(0), code, st)
+        count.copy_(ws[4 * seq_len:4 * seq_len + 4], non_blocking=True)
+        ev[4].record(stream)
+        ev[4].synchronize()
+    num_computed = int(count.view(torch.int32)[0])
+    index_ms = ev[0].elapsed_time(ev[1])
+    assemble_ms = ev[2].elapsed_time(ev[3])
+    return PartialPrefillResult(
+        output=out,
+        kv_cache=cache,
+        positions_computed=num_computed,
+        positions_reused=seq_len - num_computed,
+        computation_ratio=num_computed / seq_len,
+        scatter_time_ms=index_ms + assemble_ms,
+        projection_time_ms=ev[1].elapsed_time(ev[2]),
+        attention_time_ms=ev[3].elapsed_time(ev[4]),
+        total_time_ms=ev[0].elapsed_time(ev[4]),
+    )
+
+
+def _prefill_composed(dev, hidden_states, donor_kv, qkv_weight, output_projection,
+                      donor_positions, target_positions, compute_mask, num_heads, head_dim,
+                      qkv_bias, output_bias, scale) -> PartialPrefillResult:
+    """:func:`partial_prefill` composed from this module's functions and torch operations."""
     seq_len = hidden_states.shape[0]
     num_layers = donor_kv.shape[0]
     if scale is None:

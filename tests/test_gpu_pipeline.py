@@ -207,6 +207,51 @@ def test_partial_prefill_matches_oracle(dev, case, dtype):
             f"output outside the bar: max excess {float((diff - tol).max())}"
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("s,hid,h,d,layers,feats,share", [
+    (1, 64, 1, 64, 1, 4, 1.0),          # one position, one feature quad
+    (33, 48, 3, 64, 2, 36, 0.5),        # hidden no multiple of 64; a second row tile of one row
+    (257, 128, 5, 128, 3, 100, 0.0),    # nothing computed: donor rows and zeros only
+    (1025, 192, 2, 128, 1, 68, 0.4),    # one position past an index workgroup
+    (700, 256, 4, 64, 1, 16384, 0.3)])  # wide output tiles
+def test_partial_prefill_stages_match_composed(dev, dtype, s, hid, h, d, layers, feats, share):
+    """The stage kernels against the composition of the module's functions, over tile edges,
+    strided donors, repeated and out-of-range pairs and biases."""
+    g = gen(900 + s)
+    f = h * d
+    wide = torch.randn((layers, 2, h, s + 9, 2 * d), generator=g).to(dtype).to(dev)
+    donor = wide[..., d:]                                       # strided rows
+    x = torch.randn((s, hid), generator=g).to(dtype).to(dev)
+    wq = (torch.randn((3 * f, hid), generator=g) * hid ** -0.5).to(dtype).to(dev)
+    bq = (torch.randn(3 * f, generator=g) * 0.1).to(dtype).to(dev)
+    wo = (torch.randn((feats, f), generator=g) * f ** -0.5).to(dtype).to(dev)
+    bo = torch.randn(feats, generator=g).to(dtype).to(dev)
+    cm = torch.rand(s, generator=g) < share
+    tp = torch.cat([torch.arange(0, s, 2), torch.tensor([-1, s, s + 5])])
+    dp = torch.cat([torch.randperm(s + 9, generator=g)[:tp.numel() - 3], torch.tensor([0, 1, 2])])
+    if s > 8:
+        dp[:4] = torch.tensor([-3, s + 9, 1 << 30, 0])          # out of range: not moved
+        tp[3], dp[5] = tp[2], 7                                 # a target named twice
+    args = (x, donor, wq, wo, dp.to(torch.int32).to(dev), tp.to(torch.int32).to(dev),
+            cm.to(dev), h, d, bq, bo, None)
+    assert tk._prefill_stages_ok(*args)
+    got = tk.partial_prefill(*args)
+    want = tk._prefill_composed(x.device, *args)
+    assert (got.positions_computed, got.positions_reused) == (int(cm.sum()), int((~cm).sum()))
+    assert not bool(got.output.cpu()[~cm].any())
+    # donor rows and zeros are the same bits; new K/V come from one projection kernel on the
+    # same rows (fp32: the library's GEMM, which may sum in another order for another shape)
+    assert_bit_exact(got.kv_cache[:, :, :, ~cm.to(dev)].cpu(),
+                     want.kv_cache[:, :, :, ~cm.to(dev)].cpu())
+    if not cm.any():
+        return
+    eps = {torch.float32: 2.0 ** -20, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+    for a, b in ((got.kv_cache, want.kv_cache), (got.output, want.output)):
+        a, b = a.float(), b.float()
+        # one rounding to the dtype on each side, of fp32 results that differ in the last bits
+        assert float((a - b).abs().max()) <= eps * float(b.abs().max())
+
+
 # ---- Llama-3-8B batch at full size --------------------------------------------------------
 
 def test_llama3_8b_batch_full_size(dev):
