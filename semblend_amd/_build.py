@@ -1,8 +1,9 @@
-"""Build recipe for libsemblend_hip.so (gfx950).
+"""Build recipe for libsemblend_hip.so (gfx950) and libsemblend_host.so.
 
 Compiles every ``csrc/*.hip`` translation unit with hipcc for gfx950 only and links them into
 ``semblend_amd/libsemblend_hip.so``, next to the Python package that loads it. Object files
-go to ``_build/`` at the repository root (git-ignored).
+go to ``_build/`` at the repository root (git-ignored). ``csrc/sb_host.cpp`` (Python index lists to
+host arrays, against the interpreter's own headers) becomes ``libsemblend_host.so`` beside it.
 
 Usage: ``python -m semblend_amd._build`` or ``semblend_amd._build.build()``.
 """
@@ -14,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -22,6 +24,8 @@ REPO = PKG_DIR.parent
 BUILD_DIR = REPO / "_build"
 LIB_NAME = "libsemblend_hip.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+HOST_LIB_NAME = "libsemblend_host.so"
+HOST_LIB_PATH = PKG_DIR / HOST_LIB_NAME
 ARCH = "gfx950"
 
 # Flags shared by every translation unit. Packed-FP32 instructions are disabled for device
@@ -68,8 +72,20 @@ def _compile(src: Path, hipcc: str, verbose: bool) -> Path:
     return obj
 
 
+def _build_host(hipcc: str, verbose: bool) -> None:
+    tmp = HOST_LIB_PATH.with_suffix(".so.tmp")
+    cmd = [hipcc, "-O3", "-std=c++17", "-fPIC", "-shared", "-x", "c++", str(CSRC / "sb_host.cpp"),
+           f"-I{sysconfig.get_paths()['include']}", "-o", str(tmp)]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"hipcc failed on sb_host.cpp:\n{res.stderr}")
+    os.replace(tmp, HOST_LIB_PATH)
+
+
 def build(verbose: bool = False) -> Path:
-    """Compile all HIP sources and link the shared library. Always rebuilds."""
+    """Compile all sources and link the shared libraries. Always rebuilds."""
     hipcc = _hipcc()
     BUILD_DIR.mkdir(exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
@@ -85,6 +101,7 @@ def build(verbose: bool = False) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    _build_host(hipcc, verbose)
     return LIB_PATH
 
 

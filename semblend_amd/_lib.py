@@ -127,6 +127,9 @@ SIZE_QUERIES: dict[str, list] = {
     "sb_qkv_projection_paged_workspace_size": [_i64, _i64, _i64, _i64, _i64, _i32],
 }
 
+# Python index lists to host arrays (csrc/sb_host.cpp).
+HOST_LIB_PATH = Path(__file__).resolve().parent / "libsemblend_host.so"
+_host: ctypes.PyDLL | None = None
 _lib: ctypes.CDLL | None = None
 _load_error: str | None = None
 
@@ -172,9 +175,27 @@ def lib() -> ctypes.CDLL:
     return _load()
 
 
+def host_lib() -> ctypes.PyDLL:
+    """The loaded list converters; raises RuntimeError if they cannot be loaded."""
+    global _host
+    if _host is None:
+        if not HOST_LIB_PATH.exists():
+            raise RuntimeError(f"{HOST_LIB_PATH} is missing; build it with "
+                               "`python -m semblend_amd._build`")
+        lib = ctypes.PyDLL(str(HOST_LIB_PATH), mode=os.RTLD_NOW | os.RTLD_LOCAL)
+        lib.sb_host_pairs.restype = _i64
+        lib.sb_host_pairs.argtypes = [ctypes.py_object, _i64, _vp, _vp]
+        lib.sb_host_rotation_counts.restype = _i64
+        lib.sb_host_rotation_counts.argtypes = [ctypes.py_object, _i64, _i64, _i64, _vp, _vp,
+                                                _i64p]
+        _host = lib
+    return _host
+
+
 def available() -> bool:
     try:
         _load()
+        host_lib()
         return True
     except RuntimeError:
         return False
@@ -213,6 +234,11 @@ def strides(t: torch.Tensor, dims: tuple[int, ...] | None = None):
 def i32_array(values) -> ctypes.Array:
     """Host int32 array for arguments the library reads on the host."""
     return (ctypes.c_int32 * len(values))(*values)
+
+
+def i32_from(array: ctypes.Array, start: int):
+    """The int32 host array from entry ``start`` on, as a pointer argument."""
+    return array if start == 0 else ctypes.cast(ctypes.byref(array, 4 * start), I32P)
 
 
 def i64_array(values) -> ctypes.Array:

@@ -18,6 +18,8 @@ Triton kernels store fp16 regardless of the cache dtype, :183-190, which is not 
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -459,6 +461,22 @@ def _rotation_counts(positions: list[int], block_size: int,
     return counts, processed
 
 
+def _rotation_arrays(positions, block_size: int, num_blocks_per_seq: int):
+    """``_rotation_counts`` as (int32 host array of the positions, of their counts, entries used
+    in both, positions processed); plain lists of ints are resolved natively."""
+    if type(positions) is list:
+        n = len(positions)
+        keys, reps = (ctypes.c_int32 * n)(), (ctypes.c_int32 * n)()
+        used = ctypes.c_int64(0)
+        done = _lib.host_lib().sb_host_rotation_counts(
+            positions, n, block_size, num_blocks_per_seq, keys, reps, used)
+        if done >= 0:
+            return keys, reps, used.value, done
+    counts, done = _rotation_counts(positions, block_size, num_blocks_per_seq)
+    return (_lib.i32_array(list(counts.keys())), _lib.i32_array(list(counts.values())),
+            len(counts), done)
+
+
 def apply_rope_delta_inplace(
     kv_cache: torch.Tensor,
     block_table: torch.Tensor,
@@ -492,35 +510,34 @@ def apply_rope_delta_inplace(
         kst = (st[0], st[2], st[3], st[4])
     _check_head_dim(head_dim, head_dim, "apply_rope_delta_inplace")
     nbs = block_table.shape[0]
-    counts, modified = _rotation_counts(positions, block_size, nbs)
-    if not counts:
+    keys, reps, n, modified = _rotation_arrays(positions, block_size, nbs)
+    if not n:
         return 0
     bt = _lib.as_index(block_table, dev)
     inv_freq = inv_freq_table(rope_base, head_dim, dev)
-    reps = list(counts.values())
-    repeated = any(c != 1 for c in reps)
-    keys = list(counts.keys())
+    repeated = modified != n
     with _lib.on_device(dev):
         inline = _lib.SB_INLINE_POSITIONS_MAX
-        if len(keys) <= inline or torch.cuda.is_current_stream_capturing():
+        if n <= inline or torch.cuda.is_current_stream_capturing():
             # Short lists (and any list under graph capture, in launches of up to 256
             # positions) travel inside the launch: no index upload.
-            for c0 in range(0, len(keys), inline):
+            for c0 in range(0, n, inline):
                 _lib.call(
                     "sb_apply_rope_delta_inplace_host",
-                    kv_cache.data_ptr(), bt.data_ptr(), _lib.i32_array(keys[c0:c0 + inline]),
-                    _lib.i32_array(reps[c0:c0 + inline]) if repeated else None,
-                    len(keys[c0:c0 + inline]), int(delta), inv_freq.data_ptr(), num_heads,
+                    kv_cache.data_ptr(), bt.data_ptr(), _lib.i32_from(keys, c0),
+                    _lib.i32_from(reps, c0) if repeated else None,
+                    min(inline, n - c0), int(delta), inv_freq.data_ptr(), num_heads,
                     block_size, head_dim, nb_total, nbs, _lib.i64_array(kst),
                     _lib.dtype_code(kv_cache), _lib.stream_handle(dev),
                 )
             return modified
-        pos_t = _lib.upload_index(torch.tensor(keys, dtype=torch.int32), dev)
-        rep_t = _lib.upload_index(torch.tensor(reps, dtype=torch.int32), dev) if repeated else None
+        pos_t = _lib.upload_index(torch.frombuffer(keys, dtype=torch.int32, count=n), dev)
+        rep_t = _lib.upload_index(torch.frombuffer(reps, dtype=torch.int32, count=n),
+                                  dev) if repeated else None
         _lib.call(
             "sb_apply_rope_delta_inplace",
             kv_cache.data_ptr(), bt.data_ptr(), pos_t.data_ptr(),
-            None if rep_t is None else rep_t.data_ptr(), len(counts), int(delta),
+            None if rep_t is None else rep_t.data_ptr(), n, int(delta),
             inv_freq.data_ptr(), num_heads, block_size, head_dim, nb_total, nbs,
             _lib.i64_array(kst), _lib.dtype_code(kv_cache), _lib.stream_handle(dev),
         )
@@ -694,6 +711,13 @@ def paged_layout(kv_cache: torch.Tensor, layout: str | None = None):
 def _pairs_on_device(permutation, dev: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
     """(sources, targets) int32 device tensors from a list of (src, tgt) pairs or a [P, 2]
     tensor, uploaded once from pinned memory without blocking the host."""
+    if type(permutation) is list and not torch.cuda.is_current_stream_capturing():
+        n = len(permutation)
+        both = torch.empty((2, n), dtype=torch.int32, pin_memory=True)
+        at = both.data_ptr()
+        if _lib.host_lib().sb_host_pairs(permutation, n, at, at + 4 * n) == n:
+            both = both.to(dev, non_blocking=True)
+            return both[0], both[1]
     if isinstance(permutation, torch.Tensor):
         pairs = permutation.reshape(-1, 2).to(torch.int32)
     else:

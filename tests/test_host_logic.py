@@ -236,6 +236,37 @@ def test_rotation_counts():
         rc._rotation_counts([-200], 16, 8)
 
 
+@pytest.mark.parametrize("pos", [
+    [0], [5, 5, -1, 3, 79, 80, 1000, -80, 5, 79], [1000, 80], [True, 1], [3.0], [1 << 40, 2],
+    list(range(0, 700, 3)) * 3])
+def test_native_rotation_counts_match_python(pos):
+    """Plain int lists are resolved natively, others in Python: same positions, counts and
+    order either way."""
+    want, done = rc._rotation_counts(pos, 16, 5)
+    keys, reps, n, got = rc._rotation_arrays(pos, 16, 5)
+    assert (n, got) == (len(want), done)
+    assert list(zip(keys[:n], reps[:n])) == list(want.items())
+    with pytest.raises(IndexError):
+        rc._rotation_arrays(pos + [-81], 16, 5)
+
+
+def test_native_pairs_take_exact_ints_only():
+    from semblend_amd import _lib
+
+    out = torch.zeros((2, 3), dtype=torch.int32)
+
+    def native(pairs):
+        return _lib.host_lib().sb_host_pairs(pairs, len(pairs), out.data_ptr(),
+                                             out.data_ptr() + 12)
+
+    assert native([(1, -2), [3, 2 ** 31 - 1], (-2 ** 31, 0)]) == 3
+    assert out.tolist() == [[1, 3, -2 ** 31], [-2, 2 ** 31 - 1, 0]]
+    for bad in ([(1, 2.0)], [(1, True)], [(1, 2 ** 31)], [(1, 2, 3)], [(1,)], [7], [(1, "2")],
+                [torch.tensor([1, 2])]):
+        assert native(bad) == -1
+    assert _lib.host_lib().sb_host_pairs(((1, 2),), 1, out.data_ptr(), out.data_ptr()) == -1
+
+
 def test_rotation_counts_agree_with_oracle_count():
     kv = torch.randn(10, 2, 2, 16, 8)
     bt = torch.tensor([4, 2, 0, 9], dtype=torch.int32)
