@@ -455,19 +455,43 @@ constexpr int kResidentSlots = kRowGroups == 1 ? 256 * SB_ATTN_OCCUPANCY * 4 / k
 #endif
 constexpr int kItemsPerSlot = SB_ATTN_ITEMS_PER_SLOT;
 
+// Shortest key chunk. Work enough for every slot: 512 keys, below which the partials cost more
+// than the shorter items give. A call whose items are too few for the slots splits finer, because
+// there the time is one item's serial chain of tiles (about 1.5 us each with a CU to itself):
+// until about 256 items run (one per CU) or 40000 (row, chunk) partials are written, whichever
+// comes first, and no finer than 128 keys. Contexts of at most 384 keys stay whole (a merge
+// launch costs what the split would save: 300 tokens, 5 rows 9.5 us whole, 11.4 us in 128s).
+// Chunks of 512 against this rule, 28 / 4 heads x 128 and (in parentheses) 32 / 8 x 128, graph
+// replays: 10 rows of 1000 tokens 20.2 -> 13.6 us (19.6 -> 12.8); 40 of 4096 29.2 -> 24.9
+// (24.9 -> 20.7); 8 of 8000 21.6 -> 17.9 (22.1 -> 18.9); past either limit it loses: 200 rows of
+// 1000 tokens in 128s 26.3 us against 21.6 in 192s; 100 of 8000 in 256s (384 items) 35.7
+// against 31.2 in 512s.
+// item_keys: sum over the launch of row tiles x KV heads x keys; row_keys: of rows x KV heads x
+// keys.
+__host__ __device__ inline int64_t min_chunk(int64_t item_keys, int64_t row_keys,
+                                             int64_t kv_len) {
+  if (kv_len <= 384) return 512;
+  const int64_t a = item_keys / 256, b = row_keys / 40000;
+  const int64_t ks = ((a > b ? a : b) + 63) / 64 * 64;
+  return ks < 128 ? 128 : (ks > 512 ? 512 : ks);
+}
 // Key-range split of a call: items no longer than the average work per slot (assuming the
 // rows' key ranges average half the context), so that longest-first scheduling balances the
-// CUs. Host plan and device-derived split use this one rule.
+// CUs. Host plan and device-derived split use this one rule. rows_kv: flattened rows of one KV
+// head.
 struct KeySplit {
   int ksplit;
   int max_chunks;
 };
-__host__ __device__ inline KeySplit key_split(int64_t n_tiles, int64_t num_kv_heads,
-                                              int64_t kv_len, int64_t block_size, bool paged) {
+__host__ __device__ inline KeySplit key_split(int64_t rows_kv, int64_t n_tiles,
+                                              int64_t num_kv_heads, int64_t kv_len,
+                                              int64_t block_size, bool paged) {
   const int64_t kv_pad = (kv_len + kTileKeys - 1) / kTileKeys * kTileKeys;
   int64_t ks = n_tiles * num_kv_heads * (kv_len / 2) / (kResidentSlots * kItemsPerSlot);
   ks = ks / kTileKeys * kTileKeys;
-  if (ks < 512) ks = 512;
+  const int64_t least = min_chunk(n_tiles * num_kv_heads * kv_len,
+                                  rows_kv * num_kv_heads * kv_len, kv_len);
+  if (ks < least) ks = least;
   if (paged) {
     const int64_t cap = chunk_cap(block_size);
     if (ks > cap) ks = cap;
@@ -507,10 +531,11 @@ namespace sb {
 
 // The device-derived split of a dense call (device_split), from its row-tile count.
 template <bool F32>
-__device__ __forceinline__ void apply_device_split(AttnArgs& a, int64_t n_tiles_live) {
+__device__ __forceinline__ void apply_device_split(AttnArgs& a, int64_t rows_kv,
+                                                   int64_t n_tiles_live) {
   if (!a.device_split) return;
   const KeySplit sp = F32 ? key_split_f32(n_tiles_live, a.num_kv_heads, a.kv_len, a.head_dim)
-                          : key_split(n_tiles_live, a.num_kv_heads, a.kv_len, 1, false);
+                          : key_split(rows_kv, n_tiles_live, a.num_kv_heads, a.kv_len, 1, false);
   a.ksplit = sp.ksplit;
   a.ksplit_first = sp.ksplit;
   a.max_chunks = sp.max_chunks;
@@ -562,7 +587,7 @@ attn_mfma_kernel(const AttnBatch batch) {
   const int64_t rows_kv = n_rows * a.group;
   const int64_t n_tiles_live = (rows_kv + TR - 1) / TR;
   if (n_tiles_live <= 0) return;  // no rows (uniform)
-  apply_device_split<false>(a, n_tiles_live);
+  apply_device_split<false>(a, rows_kv, n_tiles_live);
   const Item item = decode_item(a, n_tiles_live, item_b);
   if (item.tile < 0 || item.chunk >= a.max_chunks) return;  // uniform, before any barrier
   const int kvh = item.kvh;
@@ -1202,15 +1227,19 @@ attn_mfma_kernel(const AttnBatch batch) {
 #define SB_MERGE_BATCH_CHUNKS 6
 #endif
 constexpr int kMergeBatch = SB_MERGE_BATCH_CHUNKS;
-// One unit: 32 rows of row tile `tile` of KV head `kvh` (mb = (tile * parts + part) * Hkv +
-// kvh). Returns early when the unit has nothing to merge; its one barrier is reached by every
+// One unit: 32 / CG rows of row tile `tile` of KV head `kvh` (mb = (tile * parts + part) * Hkv +
+// kvh), 8 CG lanes per row: with CG > 1 each group of 8 lanes takes every CG-th chunk and the
+// groups' sums meet in lane exchanges, so that a row of many chunks is not one serial chain of
+// loads. Returns early when the unit has nothing to merge; its one barrier is reached by every
 // thread of the workgroup (the returns before it are uniform).
-template <int DT, int D>
+template <int DT, int D, int CG>
 __device__ __forceinline__ void merge_unit(const AttnArgs& a, int64_t mb, int64_t n_tiles_live,
                                            int64_t rows_kv, int* red) {
+  constexpr int MB = CG > 1 ? 8 : kMergeBatch;  // chunks a lane loads at once
   const int tid = threadIdx.x;
   const int TR = a.tile_rows;  // 64 (fp32), 128 or 256
-  const int parts = TR / 32;
+  constexpr int RPU = 32 / CG;  // rows per unit
+  const int parts = TR / RPU;
   const int kvh = static_cast<int>(mb % a.num_kv_heads);
   const int64_t rest = mb / a.num_kv_heads;
   const int64_t tile = rest / parts;
@@ -1232,7 +1261,8 @@ __device__ __forceinline__ void merge_unit(const AttnArgs& a, int64_t mb, int64_
   const int kend = max(max(red[0], red[1]), max(red[2], red[3])) + 1;
   const int nchunks = chunk_count(a, kend);
   if (nchunks <= 1) return;
-  const int row_in_tile = part * 32 + tid / 8;
+  const int row_in_tile = part * RPU + tid / (8 * CG);
+  const int sub = CG > 1 ? (tid / 8) % CG : 0;  // this lane's chunk group
   const int64_t r = tile * TR + row_in_tile;
   if (r >= rows_kv) return;
   const int64_t pi = r / a.group;
@@ -1248,15 +1278,15 @@ __device__ __forceinline__ void merge_unit(const AttnArgs& a, int64_t mb, int64_
 #pragma unroll
   for (int e = 0; e < DPT; ++e) acc[e] = 0.f;
   float lsum = 0.f, mmax = -INFINITY;
-  // Batches of kMergeBatch chunks: a batch's (m, l) and values are requested at once (one round
+  // Batches of MB chunks: a batch's (m, l) and values are requested at once (one round
   // trip to memory), then added relative to the largest m so far.
-  for (int c0 = 0; c0 < nchunks; c0 += kMergeBatch) {
-    float2 ml[kMergeBatch];
-    float4 v[kMergeBatch][DPT / 4];
+  for (int c0 = sub; c0 < nchunks; c0 += MB * CG) {
+    float2 ml[MB];
+    float4 v[MB][DPT / 4];
 #pragma unroll
-    for (int ch = 0; ch < kMergeBatch; ++ch) {
-      if (c0 + ch < nchunks) {
-        const int64_t slot = (base + c0 + ch) * TR + row_in_tile;
+    for (int ch = 0; ch < MB; ++ch) {
+      if (c0 + ch * CG < nchunks) {
+        const int64_t slot = (base + c0 + ch * CG) * TR + row_in_tile;
         ml[ch] = *reinterpret_cast<const float2*>(a.part_ml + slot * 2);
 #pragma unroll
         for (int q = 0; q < DPT / 4; ++q)
@@ -1265,9 +1295,9 @@ __device__ __forceinline__ void merge_unit(const AttnArgs& a, int64_t mb, int64_
     }
     float mnew = mmax;
 #pragma unroll
-    for (int ch = 0; ch < kMergeBatch; ++ch)
-      if (c0 + ch < nchunks) mnew = fmaxf(mnew, ml[ch].x);
-    if (c0 > 0 && mnew > mmax && mmax != -INFINITY) {
+    for (int ch = 0; ch < MB; ++ch)
+      if (c0 + ch * CG < nchunks) mnew = fmaxf(mnew, ml[ch].x);
+    if (c0 >= CG && mnew > mmax && mmax != -INFINITY) {
       const float alpha = __builtin_amdgcn_exp2f(mmax - mnew);
       lsum *= alpha;
 #pragma unroll
@@ -1275,8 +1305,8 @@ __device__ __forceinline__ void merge_unit(const AttnArgs& a, int64_t mb, int64_
     }
     mmax = mnew;
 #pragma unroll
-    for (int ch = 0; ch < kMergeBatch; ++ch) {
-      if (c0 + ch >= nchunks || ml[ch].x == -INFINITY) continue;
+    for (int ch = 0; ch < MB; ++ch) {
+      if (c0 + ch * CG >= nchunks || ml[ch].x == -INFINITY) continue;
       const float w = __builtin_amdgcn_exp2f(ml[ch].x - mmax);
       lsum += w * ml[ch].y;
 #pragma unroll
@@ -1288,10 +1318,26 @@ __device__ __forceinline__ void merge_unit(const AttnArgs& a, int64_t mb, int64_
       }
     }
   }
+  if constexpr (CG > 1) {
+#pragma unroll
+    for (int o = 8; o < 8 * CG; o <<= 1) {
+      const float mn = fmaxf(mmax, __shfl_xor(mmax, o, 64));
+      const float w = mmax == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mmax - mn);
+      mmax = mn;
+      lsum *= w;
+      lsum += __shfl_xor(lsum, o, 64);
+#pragma unroll
+      for (int e = 0; e < DPT; ++e) {
+        acc[e] *= w;
+        acc[e] += __shfl_xor(acc[e], o, 64);
+      }
+    }
+  }
   const float inv = 1.f / lsum;
   char* op = a.o + qrow * a.o_s_row + qh * a.o_s_head;
 #pragma unroll
   for (int q = 0; q < DPT / 4; ++q) {
+    if (CG > 1 && q % CG != sub) continue;  // the groups share out the stores
     if constexpr (DT == SB_DTYPE_F32) {
       *reinterpret_cast<float4*>(op + (d_begin + 4 * q) * 4) = make_float4(
           acc[4 * q] / lsum, acc[4 * q + 1] / lsum, acc[4 * q + 2] / lsum, acc[4 * q + 3] / lsum);
@@ -1308,22 +1354,24 @@ __device__ __forceinline__ void merge_unit(const AttnArgs& a, int64_t mb, int64_
 // STRIDED (calls whose split follows the device row count): a fixed grid strides over the
 // live units; a grid sized for every possible row tile would spend most of its workgroups on
 // the count load alone. Otherwise one unit per workgroup.
-template <int DT, int D, bool STRIDED>
+template <int DT, int D, bool STRIDED, int CG>
 __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnBatch batch) {
   __shared__ int red[4];
   AttnArgs a = batch.a;
-  const int64_t mb = select_request(batch, a, blockIdx.x, true);
+  // (a batched launch lays out its requests in units of 32 rows: CG workgroups each)
+  int64_t mb = select_request(batch, a, blockIdx.x / CG, true);
+  mb = mb * CG + blockIdx.x % CG;
   const int TR = a.tile_rows;
   const int64_t rows_kv = attn_num_rows(a) * a.group;
   const int64_t n_tiles_live = (rows_kv + TR - 1) / TR;
   if (!STRIDED) {
-    merge_unit<DT, D>(a, mb, n_tiles_live, rows_kv, red);
+    merge_unit<DT, D, CG>(a, mb, n_tiles_live, rows_kv, red);
     return;
   }
-  apply_device_split<DT == SB_DTYPE_F32>(a, n_tiles_live);
-  const int64_t units = n_tiles_live * a.num_kv_heads * (TR / 32);
+  apply_device_split<DT == SB_DTYPE_F32>(a, rows_kv, n_tiles_live);
+  const int64_t units = n_tiles_live * a.num_kv_heads * (TR / 32 * CG);
   for (int64_t u = mb; u < units; u += gridDim.x) {
-    merge_unit<DT, D>(a, u, n_tiles_live, rows_kv, red);
+    merge_unit<DT, D, CG>(a, u, n_tiles_live, rows_kv, red);
     __syncthreads();  // red[] is reused by the next unit
   }
 }
@@ -1441,6 +1489,27 @@ namespace {
     }                                                                                     \
   } while (0)
 
+constexpr int64_t kMergeStrideGrid = 2048;  // merge workgroups of a device-split call
+// Launches the merge of split-key partials over `units` units of 32 rows. Rows of more than
+// kMergeBatch chunks spread them over four groups of lanes where the units are too few to hide a
+// row's chain of loads behind other units (22 chunks of 40 x 4 rows of 8 heads: 5.5 us); with
+// many units the chains overlap, and four groups only add idle loads (28 heads of 614 rows, 7
+// chunks: 22.5 us against 11.5 with one).
+constexpr int64_t kMergeWideUnits = 512;
+#define SB_MERGE_LAUNCH(DT, D, STRIDED, units, max_chunks, st, args)                          \
+  do {                                                                                        \
+    const int64_t sb_cap = (STRIDED) ? kMergeStrideGrid : int64_t{0x7fffffff};                \
+    if ((max_chunks) > kMergeBatch && (units) <= kMergeWideUnits) {                           \
+      const dim3 sb_mg(static_cast<unsigned>(std::min<int64_t>((units) * 4, sb_cap)));        \
+      SB_LAUNCH("attn_merge", (attn_merge_kernel<DT, D, STRIDED, 4>), sb_mg, dim3(256), st,   \
+                args);                                                                        \
+    } else {                                                                                  \
+      const dim3 sb_mg(static_cast<unsigned>(std::min<int64_t>(units, sb_cap)));              \
+      SB_LAUNCH("attn_merge", (attn_merge_kernel<DT, D, STRIDED, 1>), sb_mg, dim3(256), st,   \
+                args);                                                                        \
+    }                                                                                         \
+  } while (0)
+
 bool mfma_path(int32_t dtype, int64_t head_dim) {
   return (dtype == SB_DTYPE_BF16 || dtype == SB_DTYPE_F16) &&
          (head_dim == 64 || head_dim == 128);
@@ -1482,7 +1551,8 @@ Plan make_plan(int64_t rows_upper, int64_t group, int64_t num_kv_heads, int64_t 
     pl.max_chunks = op->max_chunks;
   } else {
     const KeySplit sp = f32 ? key_split_f32(pl.n_tiles, num_kv_heads, kv_len, head_dim)
-                            : key_split(pl.n_tiles, num_kv_heads, kv_len, block_size, paged);
+                            : key_split(rows_upper * group, pl.n_tiles, num_kv_heads, kv_len,
+                                      block_size, paged);
     pl.ksplit = sp.ksplit;
     pl.ksplit_first = sp.ksplit;
     pl.max_chunks = sp.max_chunks;
@@ -1495,20 +1565,22 @@ Plan make_plan(int64_t rows_upper, int64_t group, int64_t num_kv_heads, int64_t 
 
 // Split of a call whose row count is known only on the device (dense drop-in): the kernels
 // derive it from that count with key_split; the launch covers the largest item count and
-// the workspace the largest partials over every possible count of row tiles.
-constexpr int64_t kMergeStrideGrid = 2048;  // merge workgroups of a device-split call
+// the workspace the largest partials over every possible count of row tiles (of a count's
+// splits, the one with the fewest rows is the finest).
 struct DeviceSplitBounds {
   int64_t items;      // workgroups of the attention launch
+  int most_chunks;    // key chunks of the finest split
   int64_t part_rows;  // flattened rows of split-key partials (O rows, then m/l pairs)
 };
 DeviceSplitBounds device_split_bounds(int64_t n_tiles_upper, int64_t num_kv_heads,
                                       int64_t kv_len, int tile_rows, int64_t head_dim,
                                       bool f32) {
-  DeviceSplitBounds b{0, 0};
+  DeviceSplitBounds b{0, 1, 0};
   for (int64_t t = 1; t <= n_tiles_upper; ++t) {
     const KeySplit sp = f32 ? key_split_f32(t, num_kv_heads, kv_len, head_dim)
-                            : key_split(t, num_kv_heads, kv_len, 1, false);
+                            : key_split((t - 1) * tile_rows + 1, t, num_kv_heads, kv_len, 1, false);
     b.items = std::max<int64_t>(b.items, t * num_kv_heads * sp.max_chunks);
+    b.most_chunks = std::max(b.most_chunks, sp.max_chunks);
     if (sp.max_chunks > 1)
       b.part_rows = std::max<int64_t>(b.part_rows, num_kv_heads * t * sp.max_chunks * tile_rows);
   }
@@ -1534,11 +1606,13 @@ int launch_attention_f32(const char* fn, AttnArgs a, int64_t rows_upper, void* w
   int64_t part_rows =
       pl.part_bytes > 0 ? a.num_kv_heads * pl.n_tiles * pl.max_chunks * pl.tile_rows : 0;
   int64_t gx = pl.n_tiles * a.num_kv_heads * pl.max_chunks;
+  int most_chunks = pl.max_chunks;
   if (a.device_split) {
     const DeviceSplitBounds b =
         device_split_bounds(pl.n_tiles, a.num_kv_heads, a.kv_len, pl.tile_rows, a.head_dim, true);
     part_rows = b.part_rows;
     gx = b.items;
+    most_chunks = b.most_chunks;
   }
   if (part_rows > 0 && (!workspace || workspace_bytes < part_rows * (a.head_dim + 2) * 4)) {
     a.device_split = 0;
@@ -1553,21 +1627,17 @@ int launch_attention_f32(const char* fn, AttnArgs a, int64_t rows_upper, void* w
   }
   if (gx > 0x7fffffff) return fail(fn, "grid too large");
   const dim3 grid(static_cast<unsigned>(gx));
-  int64_t mx = pl.n_tiles * a.num_kv_heads * (pl.tile_rows / 32);
-  if (a.device_split) mx = std::min<int64_t>(mx, kMergeStrideGrid);
-  if (mx > 0x7fffffff) return fail(fn, "grid too large");
-  const dim3 mgrid(static_cast<unsigned>(mx));
+  const int64_t mx = pl.n_tiles * a.num_kv_heads * (pl.tile_rows / 32);
+  if (mx * 4 > 0x7fffffff) return fail(fn, "grid too large");
   AttnBatch one{};
   one.a = a;
 #define SB_F32_CASE(IT, D, PAGED)                                                         \
   if (in_dtype == IT && a.head_dim == D && (a.paged != 0) == PAGED) {                     \
     SB_LAUNCH("attn_f32", (attn_f32_kernel<IT, D, PAGED>), grid, dim3(kF32Threads), st, a); \
     if (part_rows > 0 && a.device_split)                                                  \
-      SB_LAUNCH("attn_merge", (attn_merge_kernel<SB_DTYPE_F32, D, true>), mgrid,          \
-                dim3(256), st, one);                                                      \
+      SB_MERGE_LAUNCH(SB_DTYPE_F32, D, true, mx, most_chunks, st, one);                   \
     else if (part_rows > 0)                                                               \
-      SB_LAUNCH("attn_merge", (attn_merge_kernel<SB_DTYPE_F32, D, false>), mgrid,         \
-                dim3(256), st, one);                                                      \
+      SB_MERGE_LAUNCH(SB_DTYPE_F32, D, false, mx, most_chunks, st, one);                  \
     return check_launch(fn);                                                              \
   }
   SB_F32_CASE(SB_DTYPE_F32, 64, true)
@@ -1601,12 +1671,14 @@ int launch_attention(const char* fn, AttnArgs a, int32_t dtype, int64_t rows_upp
                                                 pl.tile_rows
                                           : 0;
     int64_t gx = pl.n_tiles * a.num_kv_heads * pl.max_chunks;
+    int most_chunks = pl.max_chunks;
     if (a.device_split) {
       // The kernels split by the device row count: cover every count that can occur.
       const DeviceSplitBounds b =
           device_split_bounds(pl.n_tiles, a.num_kv_heads, a.kv_len, pl.tile_rows, a.head_dim, false);
       part_rows = b.part_rows;
       gx = b.items;
+      most_chunks = b.most_chunks;
     }
     if (part_rows > 0) {
       const int64_t need = part_rows * (a.head_dim + 2) * 4;
@@ -1617,9 +1689,8 @@ int launch_attention(const char* fn, AttnArgs a, int32_t dtype, int64_t rows_upp
     }
     if (gx > 0x7fffffff) return fail(fn, "grid too large");
     dim3 grid(static_cast<unsigned>(gx));
-    int64_t mx = pl.n_tiles * a.num_kv_heads * (pl.tile_rows / 32);
-    if (a.device_split) mx = std::min<int64_t>(mx, kMergeStrideGrid);  // strided merge
-    dim3 mgrid(static_cast<unsigned>(mx));
+    const int64_t mx = pl.n_tiles * a.num_kv_heads * (pl.tile_rows / 32);
+    if (mx * 4 > 0x7fffffff) return fail(fn, "grid too large");
     AttnBatch one{};
     one.a = a;
     one.num_reqs = 0;
@@ -1627,9 +1698,9 @@ int launch_attention(const char* fn, AttnArgs a, int32_t dtype, int64_t rows_upp
   if (dtype == DT && a.head_dim == D) {                                                 \
     SB_ATT_LAUNCH(DT, D, grid, st, one);                                               \
     if (part_rows > 0 && a.device_split)                                                \
-      SB_LAUNCH("attn_merge", (attn_merge_kernel<DT, D, true>), mgrid, dim3(256), st, one); \
+      SB_MERGE_LAUNCH(DT, D, true, mx, most_chunks, st, one);                           \
     else if (part_rows > 0)                                                             \
-      SB_LAUNCH("attn_merge", (attn_merge_kernel<DT, D, false>), mgrid, dim3(256), st, one); \
+      SB_MERGE_LAUNCH(DT, D, false, mx, most_chunks, st, one);                          \
     return check_launch(fn);                                                            \
   }
     SB_ATT_CASE(SB_DTYPE_BF16, 128)
@@ -1667,7 +1738,7 @@ VarlenPlan make_varlen_plan(int64_t num_reqs, const int64_t* rows, const int64_t
   pl.n_tiles.assign(num_reqs, 0);
   pl.max_chunks.assign(num_reqs, 1);
   pl.row_begin.assign(num_reqs, 0);
-  int64_t work = 0, kv_max = 0, run = 0;
+  int64_t work = 0, kv_max = 0, run = 0, item_keys = 0, row_keys = 0;
   for (int64_t r = 0; r < num_reqs; ++r) {
     pl.row_begin[r] = run;
     run += rows[r];
@@ -1676,6 +1747,8 @@ VarlenPlan make_varlen_plan(int64_t num_reqs, const int64_t* rows, const int64_t
     if (rows[r] > 0 && blocks[r] > 0) {
       pl.order.push_back(static_cast<int>(r));
       work += pl.n_tiles[r] * num_kv_heads * (kv / 2);
+      item_keys += pl.n_tiles[r] * num_kv_heads * kv;
+      row_keys += rows[r] * group * num_kv_heads * kv;
       kv_max = kv > kv_max ? kv : kv_max;
     }
   }
@@ -1684,7 +1757,8 @@ VarlenPlan make_varlen_plan(int64_t num_reqs, const int64_t* rows, const int64_t
   });
   int64_t ks = work / kResidentSlots;
   ks = ks / kTileKeys * kTileKeys;
-  if (ks < 512) ks = 512;
+  const int64_t least = min_chunk(item_keys, row_keys, kv_max);
+  if (ks < least) ks = least;
   const int64_t cap = chunk_cap(block_size);
   if (ks > cap) ks = cap;
   const int64_t kv_pad = (kv_max + kTileKeys - 1) / kTileKeys * kTileKeys;
@@ -1761,19 +1835,19 @@ int launch_attention_varlen(const char* fn, AttnArgs a, int32_t dtype, int64_t n
       sl.part_begin = part_rows;
       items += pl.n_tiles[r] * a.num_kv_heads * pl.max_chunks[r];
       merges += pl.n_tiles[r] * a.num_kv_heads * (tr / 32);
+      b.a.max_chunks = std::max(b.a.max_chunks, sl.max_chunks);
       if (pl.max_chunks[r] > 1) {
         part_rows += a.num_kv_heads * pl.n_tiles[r] * pl.max_chunks[r] * tr;
         split = true;
       }
     }
     if (b.a.part_o) b.a.part_ml = b.a.part_o + part_total * a.head_dim;
-    if (items > 0x7fffffff || merges > 0x7fffffff) return fail(fn, "grid too large");
+    if (items > 0x7fffffff || merges * 4 > 0x7fffffff) return fail(fn, "grid too large");
     const dim3 grid(static_cast<unsigned>(items));
-    const dim3 mgrid(static_cast<unsigned>(merges));
 #define SB_ATT_VCASE(DT, D)                                                             \
   if (dtype == DT && a.head_dim == D) {                                                 \
     SB_ATT_LAUNCH(DT, D, grid, st, b);                                                 \
-    if (split) SB_LAUNCH("attn_merge", (attn_merge_kernel<DT, D, false>), mgrid, dim3(256), st, b); \
+    if (split) SB_MERGE_LAUNCH(DT, D, false, merges, b.a.max_chunks, st, b);             \
     const int rc = check_launch(fn);                                                    \
     if (rc) return rc;                                                                  \
     continue;                                                                           \
@@ -1852,7 +1926,7 @@ HostOrderPlan plan_paged_order(const int32_t* pos, int64_t num_rows, int64_t gro
     }
     kend[static_cast<size_t>(t)] = m + 1;
   }
-  const KeySplit base = key_split(n_tiles, num_kv_heads, kv_len, block_size, true);
+  const KeySplit base = key_split(rows_kv, n_tiles, num_kv_heads, kv_len, block_size, true);
   AttnArgs geo{};
   auto cost_of = [&](int chunk, int64_t t) -> int64_t {  // 64-key tiles of one item
     const int64_t k0 = chunk_begin(geo, chunk);

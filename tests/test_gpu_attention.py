@@ -358,3 +358,42 @@ def test_fp32_rising_scores_and_strided_inputs(dev):
     bq[..., :d] = q.to(dev)
     got = tk.partial_prefill_attention_paged(bq[..., :d], big[..., :d], bt.to(dev), pos.to(dev))
     assert_attn_close(got, ref.partial_attention_paged(q, kv, bt, pos))
+
+
+# ---- small calls: fine key splits and the merge that spreads a row's chunks over lanes ----
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d,ctx,rows,bs", [
+    (4, 2, 64, 384, 3, 16),      # whole: one chunk
+    (4, 2, 128, 400, 3, 16),     # four chunks of 128: the merge of few chunks
+    (4, 2, 128, 900, 2, 24),     # eight chunks: the last holds 4 keys
+    (14, 2, 64, 8000, 1, 16),    # 63 chunks: two batches of the wide merge
+    (32, 8, 128, 3200, 40, 32)])
+def test_small_calls_split_and_merge(dev, dtype, hq, hkv, d, ctx, rows, bs):
+    g = gen(500 + ctx)
+    nb = -(-ctx // bs)
+    kv = randn((nb + 3, 2, hkv, bs, d), dtype, 501)
+    bt = torch.randperm(nb + 3, generator=g)[:nb].to(torch.int32)
+    pos = torch.cat([torch.tensor([0, ctx - 1])[:rows],
+                     torch.randperm(ctx - 2, generator=g)[:max(0, rows - 2)] + 1])
+    pos = pos.sort().values.to(torch.int32)
+    q = randn((pos.numel(), hq, d), dtype, 502)
+    got = tk.partial_prefill_attention_paged(q.to(dev), kv.to(dev), bt.to(dev), pos.to(dev))
+    assert_attn_close(got, ref.partial_attention_paged(q, kv, bt, pos))
+    half = tk.partial_prefill_attention_paged_varlen(
+        torch.cat([q, q]).to(dev), kv.to(dev), torch.stack([bt, bt]).to(dev),
+        torch.cat([pos, pos]).to(dev), [pos.numel()] * 2, [nb] * 2)
+    assert_attn_close(half[pos.numel():], ref.partial_attention_paged(q, kv, bt, pos))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [[2999], [0, 1500, 2999], list(range(0, 3000, 9))])
+def test_dense_few_rows_of_a_long_context(dev, dtype, rows):
+    """The device-derived split of few rows (fine chunks, wide strided merge) and of many."""
+    q, k, v = (randn((2, 3000, 64), dtype, 510 + i) for i in range(3))
+    mask = torch.zeros(3000, dtype=torch.bool)
+    mask[rows] = True
+    got = tk.partial_prefill_attention(q.to(dev), k.to(dev), v.to(dev), mask.to(dev)).cpu()
+    want = ref.partial_prefill_attention(q.float(), k.float(), v.float(), mask)
+    assert_attn_close(got[:, rows], want[:, rows].to(dtype))
+    assert not bool(got[:, ~mask].any())
