@@ -25,7 +25,8 @@
 //   dense mode  all features -> out[positions[row]] (the [S, F] drop-in layout).
 // Bias (input dtype) is added in fp32; with RoPE, Q and K are rotated by the row's position
 // (angle = float(p) * inv_freq[i]) with cos/sin from a per-(row, pair) table that a small
-// kernel fills first (fp64 sincos rounded once to fp32, as in the RoPE kernels).
+// kernel fills first, or workgroups of the split product itself (fp64 sincos rounded once to fp32,
+// as in the RoPE kernels).
 
 #include <algorithm>
 #include <type_traits>
@@ -67,12 +68,11 @@ constexpr int kStages = SB_QKV_STAGES;  // LDS ring depth: loads run kStages - 1
 constexpr int kTileChunks = kTK / 8;  // 16-byte chunks per tile row
 constexpr int kLoadRows = kQThreads / kTileChunks;  // tile rows one load of every thread fills
 static_assert(kTK == 32 || kTK == 64, "tile rows of 64 or 128 bytes");
-static_assert(kStages >= 2 && kStages <= 4, "the step waits cover rings of 2 to 4 stages");
 constexpr int kGroup = SB_QKV_GROUP;  // row tiles per band of the tile order
 constexpr int kXcds = 8;       // MI355X: workgroups go round-robin to 8 XCDs
 
 // QKV_PARTIAL: the split form's product for small row counts, the hidden dimension split over
-// grid.y (each slice's fp32 partial product to a workspace; qkv_epilogue_kernel sums the
+// workgroups (each slice's fp32 partial product to a workspace; qkv_epilogue_kernel sums the
 // slices in order and runs the split form's epilogue).
 enum QkvMode : int { QKV_SPLIT = 0, QKV_DENSE = 1, QKV_PARTIAL = 2 };
 
@@ -101,6 +101,11 @@ struct QkvArgs {
   float* part;                // QKV_PARTIAL: [splits][R][F] fp32 partial products
   int64_t split_steps;        // QKV_PARTIAL: k-steps per slice of the hidden dimension
   int64_t splits;             // epilogue: slices to sum (0 or 1: one product)
+  // QKV_PARTIAL: workgroup b runs tile b % tiles of slice b / tiles; those past the last slice
+  // fill the epilogue's RoPE table (nullptr: no RoPE).
+  int64_t tiles;
+  float4* table;
+  const float* inv_freq;
 };
 
 // 16-byte chunk position of chunk c of tile row r. 256 bytes of banks hold 256 / (2 kTK)
@@ -185,42 +190,38 @@ __device__ __forceinline__ uint32_t qkv_pack2_fast(float lo, float hi) {
 // cos / sin of every (computed row, rotary pair), correctly rounded to fp32 (fp64 sincos):
 // entry e of row n = (cos, sin) of pairs 2e and 2e + 1, angle float(p) * inv_freq[pair];
 // rows without a valid position get the identity. Layouts:
-//   row-major (IL false)  table[n * D/4 + e], num_rows rows;
-//   interleaved (IL true) table[((n / 32) * D/4 + e) * 32 + n % 32], rows padded to a
-//   multiple of 32 (identity): the fused kernel's lanes hold 32 consecutive rows, so one
-//   entry of all of them is 512 contiguous bytes.
-template <bool IL>
-__global__ void qkv_rope_table_kernel(const int32_t* positions, int64_t num_rows,
-                                      int64_t seq_len, const float* inv_freq, int half_d,
-                                      float4* table) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int quads = half_d / 2;
-  const int64_t table_rows = IL ? (num_rows + 31) / 32 * 32 : num_rows;
-  if (idx >= table_rows * quads) return;
-  int64_t n;
-  int k;
-  if (IL) {
-    const int64_t grp = idx / (32 * quads);
-    const int64_t rem = idx - grp * 32 * quads;
-    k = static_cast<int>(rem / 32);
-    n = grp * 32 + (rem & 31);
-  } else {
-    n = idx / quads;
-    k = static_cast<int>(idx - n * quads);
-  }
+//   row-major    table[n * D/4 + e], num_rows rows (the split product's epilogue and the library
+//                form);
+//   interleaved  table[((n / 32) * D/4 + e) * 32 + n % 32], rows padded to a multiple of 32
+//                (identity): the fused kernel's lanes hold 32 consecutive rows, so one entry of
+//                all of them is 512 contiguous bytes.
+__device__ __forceinline__ float4 qkv_rope_entry(const int32_t* positions, int64_t n,
+                                                 int64_t num_rows, int64_t seq_len,
+                                                 const float* inv_freq, int k) {
   const int p = n < num_rows ? positions[n] : -1;
   float4 v = make_float4(1.f, 0.f, 1.f, 0.f);
   if (p >= 0 && p < seq_len) {
     sincos_rn(static_cast<float>(p) * inv_freq[2 * k], &v.y, &v.x);
     sincos_rn(static_cast<float>(p) * inv_freq[2 * k + 1], &v.w, &v.z);
   }
-  table[idx] = v;
+  return v;
+}
+__global__ void qkv_rope_table_kernel(const int32_t* positions, int64_t num_rows,
+                                      int64_t seq_len, const float* inv_freq, int half_d,
+                                      float4* table) {
+  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int quads = half_d / 2;
+  if (idx >= (num_rows + 31) / 32 * 32 * quads) return;
+  const int64_t grp = idx / (32 * quads);
+  const int64_t rem = idx - grp * 32 * quads;
+  table[idx] = qkv_rope_entry(positions, grp * 32 + (rem & 31), num_rows, seq_len, inv_freq,
+                              static_cast<int>(rem / 32));
 }
 
 // The projection. Workgroup tile: TM = 64 BI features x TN = 64 BJ rows, 4 waves as 2 x 2,
 // each wave BI x BJ MFMA blocks of 32 x 32 (BI = 4, BJ = 2..4: up to a 128 x 128 wave tile
 // and 256 accumulators, one workgroup per CU; BI = BJ = 2: 64 x 64, two per CU).
-template <int DT, int MODE, int BI, int BJ>
+template <int DT, int MODE, int BI, int BJ, int ST>
 __global__ __launch_bounds__(kQThreads, BI * BJ > 4 ? 1 : 2) void qkv_mfma_kernel(QkvArgs a) {
   using vec8 = std::conditional_t<DT == SB_DTYPE_BF16, qbf16x8_t, qf16x8_t>;
   constexpr int TM = 64 * BI, TN = 64 * BJ;
@@ -228,32 +229,42 @@ __global__ __launch_bounds__(kQThreads, BI * BJ > 4 ? 1 : 2) void qkv_mfma_kerne
   constexpr int LB = TN * kTileChunks / kQThreads;  // B loads per thread per stage (= BJ)
   constexpr int NKS = kTK / 16;                     // MFMA k-substeps per step
   // The LDS ring (A stages, then B stages); after the k loop it holds the output tile.
-  __shared__ __align__(16) uint16_t smem[kStages * (TM + TN) * kTK];
-  static_assert(TM * TN <= kStages * (TM + TN) * kTK, "output tile fits in the ring");
+  __shared__ __align__(16) uint16_t smem[ST * (TM + TN) * kTK];
+  static_assert(TM * TN <= ST * (TM + TN) * kTK, "output tile fits in the ring");
+  static_assert(ST >= 2 && ST <= 4, "the step waits cover rings of 2 to 4 stages");
   auto As = [&](int stage) { return smem + stage * TM * kTK; };
-  auto Bs = [&](int stage) { return smem + kStages * TM * kTK + stage * TN * kTK; };
+  auto Bs = [&](int stage) { return smem + ST * TM * kTK + stage * TN * kTK; };
   __shared__ int64_t brow[TN];   // byte offset of each tile row's hidden row
   __shared__ int bpos[TN];       // its position (-1: no row)
   __shared__ int64_t kvofs[TN];  // split: byte offset of its paged slot (-1: none)
   __shared__ __align__(16) float bias_s[TM];  // the tile's bias (0 without bias / past F)
 
   const int tid = threadIdx.x;
+  const int64_t slice = MODE == QKV_PARTIAL ? blockIdx.x / a.tiles : 0;
+  if (MODE == QKV_PARTIAL && slice >= a.splits) {  // uniform
+    const int quads = a.head_dim / 4;
+    const int64_t e = (blockIdx.x - a.splits * a.tiles) * kQThreads + tid;
+    if (e < a.num_rows * quads)
+      a.table[e] = qkv_rope_entry(a.positions, e / quads, a.num_rows, a.seq_len, a.inv_freq,
+                                  static_cast<int>(e % quads));
+    return;
+  }
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar
   const int lane = tid & 63, lq = lane & 31, lg = lane >> 5;
   const int wm = wave & 1, wn = wave >> 1;
   const int64_t n_ft = (a.num_features + TM - 1) / TM;
   const int64_t n_rt = (a.num_rows + TN - 1) / TN;
   int64_t ft, rt;
-  qkv_tile(blockIdx.x, n_ft, n_rt, &ft, &rt);
+  qkv_tile(blockIdx.x - slice * a.tiles, n_ft, n_rt, &ft, &rt);
   const int64_t m0 = ft * TM;
   const int64_t n0 = rt * TN;
   int64_t rows = a.num_rows;
   if (a.count) rows = min(rows, static_cast<int64_t>(*a.count));
   if (n0 >= rows) return;  // uniform
-  // This workgroup's k-steps: all of them, or (QKV_PARTIAL) slice blockIdx.y.
+  // This workgroup's k-steps: all of them, or (QKV_PARTIAL) those of its slice.
   int64_t kbeg = 0, nsteps = a.k_steps;
   if (MODE == QKV_PARTIAL) {
-    kbeg = static_cast<int64_t>(blockIdx.y) * a.split_steps;
+    kbeg = slice * a.split_steps;
     nsteps = min(a.split_steps, a.k_steps - kbeg);
     if (nsteps <= 0) return;  // uniform
   }
@@ -320,27 +331,27 @@ __global__ __launch_bounds__(kQThreads, BI * BJ > 4 ? 1 : 2) void qkv_mfma_kerne
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  // Ring of kStages: step kt lives in stage kt % kStages; loads run kStages - 1 steps ahead.
+  // Ring of ST: step kt lives in stage kt % ST; loads run ST - 1 steps ahead.
   // One barrier per step both publishes step kt and retires step kt - 1, whose stage the
   // loads issued right after it refill.
 #pragma unroll
-  for (int s0 = 0; s0 < kStages - 1; ++s0)
+  for (int s0 = 0; s0 < ST - 1; ++s0)
     if (s0 < nsteps) issue(s0, s0);
-  // Step kt; REFILL: whether it issues the loads of step kt + kStages - 1 (every step but
-  // the last kStages - 1), a compile-time choice so that the loads need no branch.
+  // Step kt; REFILL: whether it issues the loads of step kt + ST - 1 (every step but
+  // the last ST - 1), a compile-time choice so that the loads need no branch.
   auto step = [&](int64_t kt, auto refill_c) {
     constexpr bool REFILL = decltype(refill_c)::value;
-    const int st = static_cast<int>(kt % kStages);
-    // Steps issued after this one: at most kStages - 2, fewer near the end; they may stay
+    const int st = static_cast<int>(kt % ST);
+    // Steps issued after this one: at most ST - 2, fewer near the end; they may stay
     // in flight while step kt must have landed.
     const int64_t ahead = nsteps - 1 - kt;
-    if (kStages >= 4 && ahead >= 2) qkv_wait_vm<2 * (LA + LB)>();
-    else if (kStages >= 3 && ahead >= 1) qkv_wait_vm<LA + LB>();
+    if (ST >= 4 && ahead >= 2) qkv_wait_vm<2 * (LA + LB)>();
+    else if (ST >= 3 && ahead >= 1) qkv_wait_vm<LA + LB>();
     else qkv_wait_vm<0>();
     __syncthreads();
-    const int rst = static_cast<int>((kt + kStages - 1) % kStages);
+    const int rst = static_cast<int>((kt + ST - 1) % ST);
 #if !SB_QKV_FRAG_PIPE
-    if (REFILL) issue(rst, kt + kStages - 1);
+    if (REFILL) issue(rst, kt + ST - 1);
 #endif
     // Per k-substep: the wave's BI A and BJ B fragments, then BI x BJ MFMAs. The fragments
     // are double-buffered: those of substep ks + 1 are read while the MFMAs of substep ks
@@ -379,12 +390,13 @@ __global__ __launch_bounds__(kQThreads, BI * BJ > 4 ? 1 : 2) void qkv_mfma_kerne
           else
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_f[i], b_f[j], acc[i][j], 0, 0, 0);
 #if SB_QKV_FRAG_PIPE
-          constexpr int kSpread = SB_QKV_DMA_SPREAD < NKS ? SB_QKV_DMA_SPREAD : NKS;
+          constexpr int kWant = BI * BJ < 4 ? NKS : SB_QKV_DMA_SPREAD;
+          constexpr int kSpread = kWant < NKS ? kWant : NKS;
           constexpr int kPer = (LA + LB + kSpread - 1) / kSpread;  // loads per substep
           static_assert(kPer <= BI * BJ, "every load follows an MFMA of its substep");
           const int q = ks * kPer + i * BJ + j;
           if (REFILL && i * BJ + j < kPer && q < LA + LB) {
-            issue_one(rst, kt + kStages - 1, q);
+            issue_one(rst, kt + ST - 1, q);
             __builtin_amdgcn_sched_barrier(0);
           }
 #endif
@@ -398,14 +410,14 @@ __global__ __launch_bounds__(kQThreads, BI * BJ > 4 ? 1 : 2) void qkv_mfma_kerne
   };
   {
     int64_t kt = 0;
-    for (; kt + kStages - 1 < nsteps; ++kt) step(kt, std::true_type{});
+    for (; kt + ST - 1 < nsteps; ++kt) step(kt, std::true_type{});
     for (; kt < nsteps; ++kt) step(kt, std::false_type{});
   }
 
   if constexpr (MODE == QKV_PARTIAL) {
     // The slice's fp32 product: lane (lq, lg) of block (i, j) holds row wn*32*BJ + 32j + lq,
     // features wm*32*BI + 32i + 8g + 4lg .. +3 in register group g.
-    float* pp = a.part + static_cast<int64_t>(blockIdx.y) * a.num_rows * a.num_features;
+    float* pp = a.part + slice * a.num_rows * a.num_features;
 #pragma unroll
     for (int j = 0; j < BJ; ++j) {
       const int64_t n = n0 + wn * (32 * BJ) + j * 32 + lq;
@@ -600,13 +612,7 @@ __global__ __launch_bounds__(256) void qkv_gather_kernel(char* xg, const char* h
   if (t >= num_rows * quads) return;
   const int64_t n = t / quads;
   const int k = static_cast<int>(t - n * quads);
-  const int p = positions[n];
-  float4 v = make_float4(1.f, 0.f, 1.f, 0.f);
-  if (p >= 0 && p < seq_len) {
-    sincos_rn(static_cast<float>(p) * inv_freq[2 * k], &v.y, &v.x);
-    sincos_rn(static_cast<float>(p) * inv_freq[2 * k + 1], &v.w, &v.z);
-  }
-  table[t] = v;
+  table[t] = qkv_rope_entry(positions, n, num_rows, seq_len, inv_freq, k);
 }
 
 // Epilogue of a projection computed elsewhere (a library GEMM with fp32 output): for row n
@@ -737,8 +743,20 @@ constexpr int64_t kCus = 256;
 #define SB_QKV_MIN_SPLIT_STEPS 12
 #endif
 constexpr int64_t kMinSplitSteps = SB_QKV_MIN_SPLIT_STEPS;
+// Finer slices, down to kFinestSteps, while the partial products stay below kFewPartialBytes: a
+// step's loads take about one memory latency however few products it has, so a slice's time is
+// its number of steps until the partials cost more. Qwen2.5-0.5B shape (896 -> 1152) 65 rows 14.0
+// -> 9.8 us, 300 rows 14.3 -> 11.9; the 7B shape at 200 rows in slices of 7 steps (26 MB) 27.6 us
+// against 24.0 in slices of 14.
+// Up to 64 rows take 128 x 64 tiles with three steps of loads in flight, one workgroup per CU
+// (16 CUs left to the RoPE table). Graph replays before and after: 7B shape 1 / 16 / 64 rows
+// 17.7 / 18.8 / 20.8 -> 11.9 / 12.6 / 15.2 us, 0.5B 12.9 / 12.7 / 13.2 -> 7.7 / 8.4 / 9.5 us,
+// Llama-3-8B (4096 -> 6144) 19.3 / 20.6 / 23.3 -> 15.0 / 15.6 / 17.4 us.
+constexpr int64_t kFinestSteps = 4;
+constexpr int64_t kFewPartialBytes = 10 << 20;
+constexpr int kNarrowStages = 4;
 struct QkvPlan {
-  int bj = 0;               // 3 or 2: 256 x 64 bj tiles; 0: 128 x 128 tiles
+  int bj = 0;               // 3 or 2: 256 x 64 bj tiles; 0: 128 x 128; 1: 128 x 64 (split only)
   int64_t tiles = 0;
   int64_t splits = 1;       // slices of the hidden dimension (> 1: QKV_PARTIAL)
   int64_t split_steps = 0;  // k-steps per slice
@@ -761,10 +779,20 @@ QkvPlan qkv_plan(int64_t rows, int64_t features, int64_t k_steps, bool allow_spl
     pl.bj = 0;  // small tiles
     pl.tiles = small;
     if (allow_split && pl.tiles > 0 && pl.tiles < kCus) {
-      const int64_t s = std::min<int64_t>((2 * kCus) / pl.tiles, k_steps / kMinSplitSteps);
+      const int64_t fit = (2 * kCus) / pl.tiles;
+      int64_t s = std::max<int64_t>(
+          std::min<int64_t>(fit, k_steps / kMinSplitSteps),
+          std::min<int64_t>({fit, k_steps / kFinestSteps, kFewPartialBytes / (rows * features * 4)}));
+      if (rows <= 64) {
+        pl.bj = 1;
+        s = std::min<int64_t>(std::max<int64_t>(kCus - 16, pl.tiles) / pl.tiles,
+                              k_steps / kFinestSteps);
+      }
       if (s > 1) {
         pl.split_steps = (k_steps + s - 1) / s;
         pl.splits = (k_steps + pl.split_steps - 1) / pl.split_steps;
+      } else {
+        pl.bj = 0;
       }
     }
   }
@@ -774,17 +802,23 @@ QkvPlan qkv_plan(int64_t rows, int64_t features, int64_t k_steps, bool allow_spl
 template <int MODE>
 int launch_qkv(const char* fn, const QkvArgs& a, int32_t dtype, hipStream_t st,
                const QkvPlan& pl) {
-  if (pl.tiles > 0x7fffffff || pl.splits > 65535) return fail(fn, "grid too large");
-  const dim3 grid(static_cast<unsigned>(pl.tiles),
-                  static_cast<unsigned>(MODE == QKV_PARTIAL ? pl.splits : 1));
-  const int bj = pl.bj;
-#define SB_QKV_CASE(DT, BI, BJ)                                                              \
-  SB_LAUNCH("qkv_mfma", (qkv_mfma_kernel<DT, MODE, BI, BJ>), grid, dim3(kQThreads), st, a)
-#define SB_QKV_DT(DT)                   \
-  switch (bj) {                         \
-    case 3: SB_QKV_CASE(DT, 4, 3); break; \
-    case 2: SB_QKV_CASE(DT, 4, 2); break; \
-    default: SB_QKV_CASE(DT, 2, 2); break; \
+  const int64_t extra = MODE == QKV_PARTIAL && a.table
+                            ? (a.num_rows * (a.head_dim / 4) + kQThreads - 1) / kQThreads : 0;
+  const int64_t blocks = MODE == QKV_PARTIAL ? pl.tiles * pl.splits + extra : pl.tiles;
+  if (blocks > 0x7fffffff) return fail(fn, "grid too large");
+  const dim3 grid(static_cast<unsigned>(blocks));
+#define SB_QKV_CASE(DT, BI, BJ, ST)                                                           \
+  SB_LAUNCH("qkv_mfma", (qkv_mfma_kernel<DT, MODE, BI, BJ, ST>), grid, dim3(kQThreads), st, a)
+#define SB_QKV_DT(DT)                                                 \
+  if constexpr (MODE == QKV_PARTIAL) {                                \
+    if (pl.bj == 1) SB_QKV_CASE(DT, 2, 1, kNarrowStages);             \
+    else SB_QKV_CASE(DT, 2, 2, kStages);                              \
+  } else {                                                            \
+    switch (pl.bj) {                                                  \
+      case 3: SB_QKV_CASE(DT, 4, 3, kStages); break;                  \
+      case 2: SB_QKV_CASE(DT, 4, 2, kStages); break;                  \
+      default: SB_QKV_CASE(DT, 2, 2, kStages); break;                 \
+    }                                                                 \
   }
   if (dtype == SB_DTYPE_BF16) {
     SB_QKV_DT(SB_DTYPE_BF16)
@@ -893,17 +927,18 @@ extern "C" int sb_qkv_projection_paged(
     if (workspace_bytes < ws_need) return fail(fn, "workspace too small");
   }
   if (inv_freq) {
-    // The fused kernel reads the interleaved layout, the split product's epilogue kernel the
-    // row-major one.
+    // The fused kernel reads the interleaved layout; the split product's epilogue reads the
+    // row-major one, which workgroups beside the product's tiles fill.
     float4* table = static_cast<float4*>(workspace);
-    const int64_t n = (num_rows + 31) / 32 * 32 * (head_dim / 4);
-    const dim3 grid(static_cast<unsigned>((n + 255) / 256));
-    if (pl.splits > 1)
-      SB_LAUNCH("qkv_rope_table", qkv_rope_table_kernel<false>, grid, dim3(256), st, positions,
-                num_rows, seq_len, inv_freq, static_cast<int>(head_dim / 2), table);
-    else
-      SB_LAUNCH("qkv_rope_table", qkv_rope_table_kernel<true>, grid, dim3(256), st, positions,
-                num_rows, seq_len, inv_freq, static_cast<int>(head_dim / 2), table);
+    if (pl.splits > 1) {
+      a.table = table;
+      a.inv_freq = inv_freq;
+    } else {
+      const int64_t n = (num_rows + 31) / 32 * 32 * (head_dim / 4);
+      SB_LAUNCH("qkv_rope_table", qkv_rope_table_kernel,
+                dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), st, positions, num_rows,
+                seq_len, inv_freq, static_cast<int>(head_dim / 2), table);
+    }
     rc = check_launch(fn);
     if (rc) return rc;
     a.rope_cs = table;
@@ -923,9 +958,10 @@ extern "C" int sb_qkv_projection_paged(
     a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) +
                                       qkv_table_bytes(num_rows, head_dim, inv_freq != nullptr));
     a.split_steps = pl.split_steps;
+    a.tiles = pl.tiles;
+    a.splits = pl.splits;
     rc = launch_qkv<QKV_PARTIAL>(fn, a, dtype, st, pl);
     if (rc) return rc;
-    a.splits = pl.splits;
     return launch_qkv_epilogue(fn, a, a.part, a.num_features, dtype, st);
   }
   return launch_qkv<QKV_SPLIT>(fn, a, dtype, st, pl);

@@ -278,3 +278,15 @@ def test_projection_zero_rows(dev):
     q = tk.qkv_projection_paged(x, w, torch.zeros(0, dtype=torch.int32, device=dev), cache, bt,
                                 4, 2, 32, rope_base=1e4)
     assert q.shape == (0, 4, 32) and torch.all(cache == 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n_rows,hidden,hq,hkv,d,rope", [
+    (1, 512, 2, 1, 64, 1e6),      # two slices of four steps, one row
+    (63, 576, 3, 1, 40, None),    # nine steps: uneven slices; 200 features, no table
+    (64, 3584, 14, 2, 64, 1e6),   # a full 64-row tile, many slices
+    (65, 960, 14, 2, 64, 1e6),    # one row past it: 128-row tiles in fine slices
+    (300, 896, 14, 2, 64, 1e6)])
+def test_projection_split_over_few_rows(dev, dtype, n_rows, hidden, hq, hkv, d, rope):
+    x, w, b, pos, bt, cache = _case(400, hidden, hq, hkv, d, n_rows, dtype, 700 + n_rows)
+    _check_paged(dev, x, w, b, pos, bt, cache, hq, hkv, d, rope, backend="fused")
