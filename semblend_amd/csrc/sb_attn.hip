@@ -466,28 +466,57 @@ constexpr int kItemsPerSlot = SB_ATTN_ITEMS_PER_SLOT;
 // (24.9 -> 20.7); 8 of 8000 21.6 -> 17.9 (22.1 -> 18.9); past either limit it loses: 200 rows of
 // 1000 tokens in 128s 26.3 us against 21.6 in 192s; 100 of 8000 in 256s (384 items) 35.7
 // against 31.2 in 512s.
-// item_keys: sum over the launch of row tiles x KV heads x keys; row_keys: of rows x KV heads x
+// tile_keys: sum over the launch of row tiles x KV heads x keys; row_keys: of rows x KV heads x
 // keys.
-__host__ __device__ inline int64_t min_chunk(int64_t item_keys, int64_t row_keys,
+__host__ __device__ inline int64_t min_chunk(int64_t tile_keys, int64_t row_keys,
                                              int64_t kv_len) {
   if (kv_len <= 384) return 512;
-  const int64_t a = item_keys / 256, b = row_keys / 40000;
+  const int64_t a = tile_keys / 256, b = row_keys / 40000;
   const int64_t ks = ((a > b ? a : b) + 63) / 64 * 64;
   return ks < 128 ? 128 : (ks > 512 ? 512 : ks);
 }
-// Key-range split of a call: items no longer than the average work per slot (assuming the
-// rows' key ranges average half the context), so that longest-first scheduling balances the
-// CUs. Host plan and device-derived split use this one rule. rows_kv: flattened rows of one KV
-// head.
+// Keys per item for row tiles whose key ranges rise evenly to kv_len, W = the average work of a
+// resident workgroup slot:
+//   W below 2304 keys: the shortest items of which no more than one per slot run. Items of W keys
+//   are a third more than the slots (each tile's last chunk is short), and the second round of a
+//   few costs as much as the first. The count is estimated as n (n + 1) / 2 whole ranges plus half
+//   an item per tile, against 240 slots (ranges are not even). Where that asks for more than 2 W
+//   (as many tiles as slots), W itself.
+//   W up to 5500 keys: 0.72 W, about two rounds, in which early items make up for late ones.
+//   Larger W: W (0.72 W is slower there: 2458 rows of 16000 tokens 281 -> 316 us, 1000 of 32000
+//   186 -> 259).
+// Graph replays, items of W keys against these: dense 28 heads x 128, 4096 tokens, 614 rows
+// 76 -> 66.5 us; 28 / 4 heads, 1200 rows of 4096 92 -> 68 us, 400 of 4096 the same, 1200 of 16000
+// 200 -> 174; 32 / 8 heads, 600 of 4096 56 -> 43, 1500 of 8000 147 -> 134; 14 / 2 x 64, 3000 of
+// 16000 169 -> 144, 800 of 16000 68 -> 71.
+// t: row tiles x KV heads; whole_keys: sum over (request, KV head) of (tiles + 1) / 2 key ranges;
+// work_keys: of tiles / 2 ranges.
+__host__ __device__ inline int64_t item_keys(int64_t t, int64_t whole_keys, int64_t work_keys) {
+  const int64_t w = work_keys / (kResidentSlots * kItemsPerSlot);
+  if (w >= 5500) return w;
+  if (w >= 2304) return w * 23 / 32;
+  const int64_t slots = kResidentSlots - 16 - t / 2;
+  if (slots <= 0 || whole_keys > 0xffffffffll) return w;  // (32-bit quotient)
+  const int64_t fit = (static_cast<uint32_t>(whole_keys) / static_cast<uint32_t>(slots) +
+                       kTileKeys - 1) / kTileKeys * kTileKeys;
+  return fit > 2 * w ? w : (fit > w ? fit : w);
+}
+// Key-range split of a call. The dense drop-in derives it on the device with this same rule;
+// host plans (`planned`), which order the items of known positions longest first, start from
+// items of W keys. rows_kv: flattened rows of one KV head.
 struct KeySplit {
   int ksplit;
   int max_chunks;
 };
 __host__ __device__ inline KeySplit key_split(int64_t rows_kv, int64_t n_tiles,
                                               int64_t num_kv_heads, int64_t kv_len,
-                                              int64_t block_size, bool paged) {
+                                              int64_t block_size, bool paged,
+                                              bool planned = false) {
   const int64_t kv_pad = (kv_len + kTileKeys - 1) / kTileKeys * kTileKeys;
-  int64_t ks = n_tiles * num_kv_heads * (kv_len / 2) / (kResidentSlots * kItemsPerSlot);
+  const int64_t t = n_tiles * num_kv_heads;
+  int64_t ks = planned || n_tiles < 2
+                   ? t * (kv_len / 2) / (kResidentSlots * kItemsPerSlot)
+                   : item_keys(t, (t + num_kv_heads) * (kv_len / 2), t * (kv_len / 2));
   ks = ks / kTileKeys * kTileKeys;
   const int64_t least = min_chunk(n_tiles * num_kv_heads * kv_len,
                                   rows_kv * num_kv_heads * kv_len, kv_len);
@@ -1738,7 +1767,8 @@ VarlenPlan make_varlen_plan(int64_t num_reqs, const int64_t* rows, const int64_t
   pl.n_tiles.assign(num_reqs, 0);
   pl.max_chunks.assign(num_reqs, 1);
   pl.row_begin.assign(num_reqs, 0);
-  int64_t work = 0, kv_max = 0, run = 0, item_keys = 0, row_keys = 0;
+  int64_t work = 0, kv_max = 0, run = 0, tiles = 0, whole = 0, tile_keys = 0,
+          row_keys = 0;
   for (int64_t r = 0; r < num_reqs; ++r) {
     pl.row_begin[r] = run;
     run += rows[r];
@@ -1747,7 +1777,9 @@ VarlenPlan make_varlen_plan(int64_t num_reqs, const int64_t* rows, const int64_t
     if (rows[r] > 0 && blocks[r] > 0) {
       pl.order.push_back(static_cast<int>(r));
       work += pl.n_tiles[r] * num_kv_heads * (kv / 2);
-      item_keys += pl.n_tiles[r] * num_kv_heads * kv;
+      tiles += pl.n_tiles[r] * num_kv_heads;
+      whole += (pl.n_tiles[r] + 1) * num_kv_heads * (kv / 2);
+      tile_keys += pl.n_tiles[r] * num_kv_heads * kv;
       row_keys += rows[r] * group * num_kv_heads * kv;
       kv_max = kv > kv_max ? kv : kv_max;
     }
@@ -1755,9 +1787,9 @@ VarlenPlan make_varlen_plan(int64_t num_reqs, const int64_t* rows, const int64_t
   std::stable_sort(pl.order.begin(), pl.order.end(), [&](int x, int y) {
     return blocks[x] * block_size > blocks[y] * block_size;
   });
-  int64_t ks = work / kResidentSlots;
+  int64_t ks = item_keys(tiles, whole, work);
   ks = ks / kTileKeys * kTileKeys;
-  const int64_t least = min_chunk(item_keys, row_keys, kv_max);
+  const int64_t least = min_chunk(tile_keys, row_keys, kv_max);
   if (ks < least) ks = least;
   const int64_t cap = chunk_cap(block_size);
   if (ks > cap) ks = cap;
@@ -1926,7 +1958,8 @@ HostOrderPlan plan_paged_order(const int32_t* pos, int64_t num_rows, int64_t gro
     }
     kend[static_cast<size_t>(t)] = m + 1;
   }
-  const KeySplit base = key_split(rows_kv, n_tiles, num_kv_heads, kv_len, block_size, true);
+  const KeySplit base =
+      key_split(rows_kv, n_tiles, num_kv_heads, kv_len, block_size, true, true);
   AttnArgs geo{};
   auto cost_of = [&](int chunk, int64_t t) -> int64_t {  // 64-key tiles of one item
     const int64_t k0 = chunk_begin(geo, chunk);

@@ -397,3 +397,36 @@ def test_dense_few_rows_of_a_long_context(dev, dtype, rows):
     want = ref.partial_prefill_attention(q.float(), k.float(), v.float(), mask)
     assert_attn_close(got[:, rows], want[:, rows].to(dtype))
     assert not bool(got[:, ~mask].any())
+
+
+@pytest.mark.parametrize("hq,hkv,d,ctx,rows", [
+    (32, 8, 128, 4000, 600),    # ten row tiles: one item per slot at most
+    (28, 4, 128, 9000, 1500),   # an average slot of 2300-5500 keys: about two rounds
+    (28, 4, 64, 20000, 2200),   # more than that
+    (28, 28, 64, 1500, 2000)])  # more row tiles than slots
+def test_key_split_rules_cover_every_key(dev, hq, hkv, d, ctx, rows):
+    """Sampled rows of each split rule against the oracle, the same rows through the batched
+    entry (its own split) beside a short request, and all rows against a planned launch."""
+    g = gen(600 + ctx)
+    rows = min(rows, ctx)
+    nb = -(-ctx // 16)
+    kv = randn((nb + 40, 2, hkv, 16, d), torch.bfloat16, 601)
+    bt = torch.randperm(nb + 40, generator=g)[:nb].to(torch.int32)
+    pos = torch.randperm(ctx, generator=g)[:rows].sort().values.to(torch.int32)
+    q = randn((rows, hq, d), torch.bfloat16, 602)
+    qd, kvd, btd, posd = q.to(dev), kv.to(dev), bt.to(dev), pos.to(dev)
+    got = tk.partial_prefill_attention_paged(qd, kvd, btd, posd)
+    sel = torch.randperm(rows, generator=g)[:12].sort().values
+    sel[0], sel[-1] = 0, rows - 1
+    want = ref.partial_attention_paged(q[sel], kv, bt, pos[sel])
+    assert_attn_close(got.cpu()[sel], want)
+    plan = tk.plan_partial_attention_paged(pos, hq, hkv, d, 16, nb, torch.bfloat16, dev)
+    planned = tk.partial_prefill_attention_paged(qd, kvd, btd, posd, plan=plan)
+    assert_attn_close(got, planned.float().cpu())
+    short = min(rows, 40)
+    tables = torch.stack([btd, btd])
+    both = tk.partial_prefill_attention_paged_varlen(
+        torch.cat([qd, qd[:short]]), kvd, tables, torch.cat([posd, posd[:short]]),
+        [rows, short], [nb, nb])
+    assert_attn_close(both[:rows].cpu()[sel], want)
+    assert_attn_close(both[rows:], got[:short].float().cpu())
