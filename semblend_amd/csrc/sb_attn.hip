@@ -2056,23 +2056,13 @@ extern "C" int sb_partial_prefill_attention(void* out, const void* q, const void
   int32_t* pos = static_cast<int32_t*>(workspace);
   const int64_t idx_bytes = ((seq_len + 1) * 4 + 255) / 256 * 256;
 
-  // Zero the rows that are not computed (output semantics of torch.zeros_like + row writes).
-  {
-    const int vb = vec_bytes({reinterpret_cast<int64_t>(out), os[0] * es, os[1] * es,
-                              head_dim * es});
-    const int vpr = static_cast<int>(head_dim * es / vb);
-    const int64_t total = num_heads * seq_len * vpr;
-    const dim3 grid(static_cast<unsigned>((total + 255) / 256));
-    char* o = static_cast<char*>(out);
-    const int64_t sh = os[0] * es, ss = os[1] * es;
-    if (vb >= 16) SB_LAUNCH("zero_rows", zero_rows_kernel<16>, grid, dim3(256), st, o, compute_mask, num_heads, seq_len, sh, ss, vpr);
-    else if (vb == 8) SB_LAUNCH("zero_rows", zero_rows_kernel<8>, grid, dim3(256), st, o, compute_mask, num_heads, seq_len, sh, ss, vpr);
-    else if (vb == 4) SB_LAUNCH("zero_rows", zero_rows_kernel<4>, grid, dim3(256), st, o, compute_mask, num_heads, seq_len, sh, ss, vpr);
-    else SB_LAUNCH("zero_rows", zero_rows_kernel<2>, grid, dim3(256), st, o, compute_mask, num_heads, seq_len, sh, ss, vpr);
-  }
-  SB_LAUNCH("mask_compact", mask_compact_kernel<0>, dim3(1), dim3(1024), st, compute_mask, seq_len,
-            pos, pos + seq_len);
-  int rc = check_launch(fn);
+  // Zero the rows that are not computed (output semantics of torch.zeros_like + row writes) and
+  // compact the mask.
+  const int rc = launch_zero_compact(
+      fn, static_cast<char*>(out), compute_mask, num_heads, seq_len, os[0] * es, os[1] * es,
+      head_dim * es,
+      vec_bytes({reinterpret_cast<int64_t>(out), os[0] * es, os[1] * es, head_dim * es}), pos,
+      pos + seq_len, st);
   if (rc) return rc;
 
   AttnArgs a{};

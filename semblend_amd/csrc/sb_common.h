@@ -189,7 +189,7 @@ __device__ __forceinline__ void sincos_rn(float x, float* s, float* c) {
 // into ascending positions (+ count) in one workgroup, and write zeros into the output rows
 // whose mask entry is 0 (rows of [heads, seq, ...] under byte strides).
 // ---------------------------------------------------------------------------------------
-// One workgroup of 1024 threads (mask_compact_kernel, or a workgroup of a larger launch).
+// One workgroup of 1024 threads.
 __device__ __forceinline__ void mask_compact_unit(const uint8_t* mask, int64_t n,
                                                   int32_t* pos_out, int32_t* count_out) {
   // Each thread takes 16 consecutive mask bytes per round (one 16-byte load when the mask is
@@ -244,29 +244,55 @@ __device__ __forceinline__ void mask_compact_unit(const uint8_t* mask, int64_t n
   if (tid == 0) *count_out = base;
 }
 
-template <int kUnused = 0>
-__global__ __launch_bounds__(1024) void mask_compact_kernel(const uint8_t* mask, int64_t n,
-                                                            int32_t* pos_out,
-                                                            int32_t* count_out) {
-  mask_compact_unit(mask, n, pos_out, count_out);
+// Both in one launch: workgroup (0, 0) compacts while the others write the zeros, so the
+// compaction (one workgroup's chain of rounds) costs no launch of its own. A thread takes one
+// vector of a position and every gridDim.y-th head of it. 28 heads x 4096 positions x 256 bytes,
+// 85% of them zeroed: 7.1 + 4.7 us in two launches, 6.9 us in this one.
+constexpr int kMaskThreads = 1024;
+template <int VB>
+__global__ __launch_bounds__(kMaskThreads) void zero_compact_kernel(
+    char* out, const uint8_t* mask, int64_t num_heads, int64_t seq_len, int64_t s_head,
+    int64_t s_seq, int vpr, int32_t* pos_out, int32_t* count_out) {
+  if (blockIdx.x == 0) {
+    if (blockIdx.y == 0) mask_compact_unit(mask, seq_len, pos_out, count_out);
+    return;
+  }
+  const int64_t idx = static_cast<int64_t>(blockIdx.x - 1) * kMaskThreads + threadIdx.x;
+  // (32-bit quotient where it fits: 64-bit division is a long instruction sequence)
+  const int64_t s = idx <= 0xffffffffll
+                        ? static_cast<int64_t>(static_cast<uint32_t>(idx) / static_cast<uint32_t>(vpr))
+                        : idx / vpr;
+  if (s >= seq_len || mask[s]) return;
+  char* p = out + s * s_seq + (idx - s * vpr) * VB;
+  for (int64_t h = blockIdx.y; h < num_heads; h += gridDim.y) {
+    char* q = p + h * s_head;
+    if (VB == 16) *reinterpret_cast<uint4*>(q) = make_uint4(0, 0, 0, 0);
+    else if (VB == 8) *reinterpret_cast<uint2*>(q) = make_uint2(0, 0);
+    else if (VB == 4) *reinterpret_cast<uint32_t*>(q) = 0u;
+    else *reinterpret_cast<uint16_t*>(q) = 0;
+  }
 }
 
-template <int VB>
-__global__ void zero_rows_kernel(char* out, const uint8_t* mask, int64_t num_heads,
-                                 int64_t seq_len, int64_t s_head, int64_t s_seq, int vpr) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t total = num_heads * seq_len * vpr;
-  if (idx >= total) return;
-  const int64_t j = idx % vpr;
-  const int64_t row = idx / vpr;
-  const int64_t s = row % seq_len;
-  const int64_t h = row / seq_len;
-  if (mask[s]) return;
-  char* p = out + h * s_head + s * s_seq + j * VB;
-  if (VB == 16) *reinterpret_cast<uint4*>(p) = make_uint4(0, 0, 0, 0);
-  else if (VB == 8) *reinterpret_cast<uint2*>(p) = make_uint2(0, 0);
-  else if (VB == 4) *reinterpret_cast<uint32_t*>(p) = 0u;
-  else *reinterpret_cast<uint16_t*>(p) = 0;
+// Launches it for rows of `row_bytes` bytes (`vb`: the largest vector width that the rows of
+// `out` allow).
+inline int launch_zero_compact(const char* fn, char* out, const uint8_t* mask, int64_t num_heads,
+                               int64_t seq_len, int64_t s_head, int64_t s_seq, int64_t row_bytes,
+                               int vb, int32_t* pos_out, int32_t* count_out, hipStream_t st) {
+  vb = vb >= 16 ? 16 : vb >= 8 ? 8 : vb >= 4 ? 4 : 2;
+  const int vpr = static_cast<int>(row_bytes / vb);
+  const int64_t gx = 1 + (seq_len * vpr + kMaskThreads - 1) / kMaskThreads;
+  if (gx > 0x7fffffff) return fail(fn, "grid too large");
+  const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(num_heads < 16 ? num_heads : 16));
+#define SB_ZERO_CASE(VB)                                                                        \
+  if (vb == VB)                                                                                 \
+    SB_LAUNCH("zero_compact", zero_compact_kernel<VB>, grid, dim3(kMaskThreads), st, out, mask, \
+              num_heads, seq_len, s_head, s_seq, vpr, pos_out, count_out);
+  SB_ZERO_CASE(16)
+  SB_ZERO_CASE(8)
+  SB_ZERO_CASE(4)
+  SB_ZERO_CASE(2)
+#undef SB_ZERO_CASE
+  return check_launch(fn);
 }
 
 }  // namespace sb

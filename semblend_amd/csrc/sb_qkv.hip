@@ -1074,14 +1074,8 @@ extern "C" int sb_masked_qkv_projection(void* out, const void* hidden, const voi
   int32_t* pos = static_cast<int32_t*>(workspace);
   // Reuse rows are zero (the reference multiplies them by the mask); computed rows are
   // written by the projection.
-  const int vpr = static_cast<int>(out_features * 2 / 8);
-  const int64_t total = seq_len * vpr;
-  SB_LAUNCH("zero_rows", zero_rows_kernel<8>, dim3(static_cast<unsigned>((total + 255) / 256)),
-            dim3(256), st, static_cast<char*>(out), compute_mask, int64_t{1}, seq_len,
-            int64_t{0}, out_stride * 2, vpr);
-  SB_LAUNCH("mask_compact", mask_compact_kernel<0>, dim3(1), dim3(1024), st, compute_mask,
-            seq_len, pos, pos + seq_len);
-  rc = check_launch(fn);
+  rc = launch_zero_compact(fn, static_cast<char*>(out), compute_mask, 1, seq_len, 0,
+                           out_stride * 2, out_features * 2, 16, pos, pos + seq_len, st);
   if (rc) return rc;
   return launch_qkv_dense(fn, a, pos, out, out_stride, dtype, st);
 }
