@@ -499,23 +499,33 @@ __global__ void rope_index_kernel(const int32_t* dpos, int64_t num_pairs, int64_
   atomicMax(&ws[seq_len + d], static_cast<int32_t>(num_pairs - i));
 }
 
-// Both steps in one single-workgroup launch (zero the table, barrier, count), for tables and
-// pair lists small enough that one workgroup builds them in about the time of a launch.
+// Both steps in one launch: a workgroup resolves kIndexThreads positions in LDS, scanning the
+// whole pair list (up to kIndexScanPairs: 32 rounds of loads), instead of one workgroup that
+// zeroes and counts the table in memory (8192 positions and pairs: 6.5 us, here 3.3 us).
 constexpr int kIndexThreads = 1024;
-constexpr int64_t kIndexFusedMax = 1 << 20;  // seq_len * 2 + num_pairs
-__global__ __launch_bounds__(kIndexThreads) void rope_index_fused_kernel(const int32_t* dpos,
-                                                                         int64_t num_pairs,
-                                                                         int64_t seq_len,
-                                                                         int32_t* ws) {
+constexpr int64_t kIndexScanPairs = 32 * kIndexThreads;
+__global__ __launch_bounds__(kIndexThreads) void rope_index_scan_kernel(const int32_t* dpos,
+                                                                        int64_t num_pairs,
+                                                                        int64_t seq_len,
+                                                                        int32_t* ws) {
+  __shared__ int count[kIndexThreads], last[kIndexThreads];
   const int tid = threadIdx.x;
-  for (int64_t i = tid; i < 2 * seq_len; i += kIndexThreads) ws[i] = 0;
+  const int64_t s0 = static_cast<int64_t>(blockIdx.x) * kIndexThreads;
+  count[tid] = 0;
+  last[tid] = 0;
   __syncthreads();
+#pragma unroll 4
   for (int64_t i = tid; i < num_pairs; i += kIndexThreads) {
-    const int64_t d = dpos[i];
-    if (d < 0 || d >= seq_len) continue;
-    atomicAdd(&ws[d], 1);
-    atomicMax(&ws[seq_len + d], static_cast<int32_t>(num_pairs - i));
+    const int64_t d = dpos[i] - s0;
+    if (d >= 0 && d < kIndexThreads) {
+      atomicAdd(&count[d], 1);
+      atomicMax(&last[d], static_cast<int32_t>(num_pairs - i));
+    }
   }
+  __syncthreads();
+  if (s0 + tid >= seq_len) return;
+  ws[s0 + tid] = count[tid];
+  ws[seq_len + s0 + tid] = last[tid];
 }
 
 struct RopeRowsArgs {
@@ -1188,9 +1198,10 @@ int rope_k_impl(const char* fn, void* out, const void* k, const int32_t* donor_p
   const int64_t n = 2 * seq_len;
   if (distinct) {
     // no index
-  } else if (n + num_pairs <= kIndexFusedMax) {
-    SB_LAUNCH("rope_index", rope_index_fused_kernel, dim3(1), dim3(kIndexThreads), st,
-              donor_pos, num_pairs, seq_len, ws);
+  } else if (num_pairs <= kIndexScanPairs && seq_len <= int64_t{0x7fffffff} * kIndexThreads) {
+    SB_LAUNCH("rope_index", rope_index_scan_kernel,
+              dim3(static_cast<unsigned>((seq_len + kIndexThreads - 1) / kIndexThreads)),
+              dim3(kIndexThreads), st, donor_pos, num_pairs, seq_len, ws);
   } else {
     SB_LAUNCH("fill_i32", fill_i32_kernel, dim3(static_cast<unsigned>((n + 255) / 256)),
               dim3(256), st, ws, n, 0);

@@ -362,3 +362,20 @@ def test_nope_permute_paged_kv(dev, dtype):
     rc.nope_permute_paged_kv(kd, bt.to(dev), perm)
     assert_bit_exact(kd[:, 1], want[:, 1])
     assert_rope_close(kd, want)
+
+
+@pytest.mark.parametrize("seq,pairs", [(1, 3), (1023, 1023), (1025, 2000), (3000, 32768),
+                                       (3000, 32769)])
+def test_rope_k_index_edges(dev, seq, pairs):
+    """The per-position pair index at the edges of its workgroups and of the list length that one
+    launch scans: repeated donor positions rotate in pair order, out-of-range ones not at all."""
+    g = gen(60 + seq)
+    k = randn((1, 1, seq, 64), torch.float32, 61)
+    dp = torch.randint(-2, seq + 2, (pairs,), generator=g).to(torch.int32)
+    if pairs > 3000:  # mostly out of range: at most a few rotations per row
+        dp[torch.rand(pairs, generator=g) < 0.97] = -1
+    tp = (dp + torch.randint(-50, 50, (pairs,), generator=g)).to(torch.int32)
+    got = rc.rope_correct_k(k.to(dev), dp.to(dev), tp.to(dev), head_dim=64)
+    ok = (dp >= 0) & (dp < seq)
+    want = ref.rope_correct_k(k.clone(), dp[ok], tp[ok], head_dim=64)
+    assert_rope_close(got, want, composed=True)
