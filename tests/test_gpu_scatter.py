@@ -272,3 +272,29 @@ def test_device_copy_rejects_unaligned(dev):
         _lib.device_copy(a[:40], a[16:56])
     with pytest.raises(RuntimeError, match="aligned"):
         _lib.device_copy(a[1:17], a[32:48])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,pairs", [(1, 5), (3, 40), (5, 300), (9, 2000), (32, 700)])
+def test_single_layer_scatter_spreads_heads(dev, dtype, heads, pairs):
+    """One-layer paged scatters whose heads are spread over workgroups (no multiple of a slice,
+    fewer heads than one), with and without RoPE."""
+    from semblend_amd import rope_correction as rc
+    from tests.helpers import assert_rope_close, gen, randn
+
+    g = gen(40 + heads)
+    s, bs, d = 2100, 16, 64
+    nb = -(-s // bs)
+    bt = torch.randperm(nb + 2, generator=g)[:nb].to(torch.int32)
+    dp = torch.randperm(s, generator=g)[:pairs].to(torch.int32)
+    tp = torch.randperm(s, generator=g)[:pairs].to(torch.int32)
+    cache = randn((nb + 2, 2, heads, bs, d), dtype, 41)
+    donor = randn((2, heads, s, d), dtype, 42)
+    got = tk.scatter_donor_kv_paged(cache.to(dev), donor.to(dev), bt.to(dev), dp.to(dev),
+                                    tp.to(dev))
+    assert_bit_exact(got, ref.scatter_donor_kv_paged(cache.clone(), donor, bt, dp, tp))
+    got = rc.rope_correct_scatter_paged(cache.to(dev), donor.to(dev), bt.to(dev), dp.to(dev),
+                                        tp.to(dev)).cpu()
+    want = ref.rope_correct_scatter_paged(cache.clone(), donor, bt, dp, tp)
+    assert_bit_exact(got[:, 1], want[:, 1])
+    assert_rope_close(got[:, 0], want[:, 0])
