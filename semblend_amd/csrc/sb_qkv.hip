@@ -747,13 +747,13 @@ constexpr int64_t kMinSplitSteps = SB_QKV_MIN_SPLIT_STEPS;
 // step's loads take about one memory latency however few products it has, so a slice's time is
 // its number of steps until the partials cost more. Qwen2.5-0.5B shape (896 -> 1152) 65 rows 14.0
 // -> 9.8 us, 300 rows 14.3 -> 11.9; the 7B shape at 200 rows in slices of 7 steps (26 MB) 27.6 us
-// against 24.0 in slices of 14.
+// against 24.0 in slices of 14, at 64 rows 6 slices (7 MB) 15.2 us against 14.5 with 4.
 // Up to 64 rows take 128 x 64 tiles with three steps of loads in flight, one workgroup per CU
 // (16 CUs left to the RoPE table). Graph replays before and after: 7B shape 1 / 16 / 64 rows
-// 17.7 / 18.8 / 20.8 -> 11.9 / 12.6 / 15.2 us, 0.5B 12.9 / 12.7 / 13.2 -> 7.7 / 8.4 / 9.5 us,
+// 17.7 / 18.8 / 20.8 -> 11.9 / 12.6 / 14.5 us, 0.5B 12.9 / 12.7 / 13.2 -> 7.7 / 8.4 / 9.5 us,
 // Llama-3-8B (4096 -> 6144) 19.3 / 20.6 / 23.3 -> 15.0 / 15.6 / 17.4 us.
 constexpr int64_t kFinestSteps = 4;
-constexpr int64_t kFewPartialBytes = 10 << 20;
+constexpr int64_t kFewPartialBytes = 5 << 20;
 constexpr int kNarrowStages = 4;
 struct QkvPlan {
   int bj = 0;               // 3 or 2: 256 x 64 bj tiles; 0: 128 x 128; 1: 128 x 64 (split only)
@@ -779,15 +779,12 @@ QkvPlan qkv_plan(int64_t rows, int64_t features, int64_t k_steps, bool allow_spl
     pl.bj = 0;  // small tiles
     pl.tiles = small;
     if (allow_split && pl.tiles > 0 && pl.tiles < kCus) {
-      const int64_t fit = (2 * kCus) / pl.tiles;
-      int64_t s = std::max<int64_t>(
+      pl.bj = rows <= 64 ? 1 : 0;
+      const int64_t fit = pl.bj == 1 ? std::max<int64_t>(kCus - 16, pl.tiles) / pl.tiles
+                                     : (2 * kCus) / pl.tiles;
+      const int64_t s = std::max<int64_t>(
           std::min<int64_t>(fit, k_steps / kMinSplitSteps),
           std::min<int64_t>({fit, k_steps / kFinestSteps, kFewPartialBytes / (rows * features * 4)}));
-      if (rows <= 64) {
-        pl.bj = 1;
-        s = std::min<int64_t>(std::max<int64_t>(kCus - 16, pl.tiles) / pl.tiles,
-                              k_steps / kFinestSteps);
-      }
       if (s > 1) {
         pl.split_steps = (k_steps + s - 1) / s;
         pl.splits = (k_steps + pl.split_steps - 1) / pl.split_steps;

@@ -296,7 +296,7 @@ def qkv_projection_paged(
     kernel of its own (bias, RoPE, one rounding, Q and the paged K/V write); "auto" takes the
     library form from 513 to 1024 rows and the fused form otherwise (which splits the hidden
     dimension when its row tiles are too few for the CUs). Qwen2.5-7B shape, graph replays on
-    one MI355X, fused / library: 15 / 21 us at 64 rows, 21 / 25.5 at 128, 26 / 39 at 256,
+    one MI355X, fused / library: 14.5 / 21 us at 64 rows, 21 / 25.5 at 128, 26 / 39 at 256,
     33.5 / 36.5 at 512, 42 / 42 at 768, 49 / 50.5 at 1024, 76 / 80 at 2048, 89 / 98 at 2458,
     158 / 165 at 4096. The fused form needs no fp32 intermediate of rows x features. Both accumulate in
     fp32 and round once.
