@@ -507,7 +507,7 @@ __global__ void rope_index_kernel(const int32_t* dpos, int64_t num_pairs, int64_
 
 // Both steps in one launch: a workgroup resolves kIndexThreads positions in LDS, scanning the
 // whole pair list (up to kIndexScanPairs: 32 rounds of loads), instead of one workgroup that
-// zeroes and counts the table in memory (8192 positions and pairs: 6.5 us, here 3.3 us).
+// zeroes and counts the table in memory (8192 positions and pairs: 6.1-6.5 us, here 4.2-4.8 us).
 constexpr int kIndexThreads = 1024;
 constexpr int64_t kIndexScanPairs = 32 * kIndexThreads;
 __global__ __launch_bounds__(kIndexThreads) void rope_index_scan_kernel(const int32_t* dpos,

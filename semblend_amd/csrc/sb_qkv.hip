@@ -754,9 +754,15 @@ constexpr int64_t kMinSplitSteps = SB_QKV_MIN_SPLIT_STEPS;
 // Llama-3-8B (4096 -> 6144) 19.3 / 20.6 / 23.3 -> 15.0 / 15.6 / 17.4 us.
 constexpr int64_t kFinestSteps = 4;
 constexpr int64_t kFewPartialBytes = 5 << 20;
+// The dense form (no split: its row count is known on the device only) takes the same 128 x 64
+// tiles where they fit one round or the k loop is long enough for the loads in flight to pay for
+// one workgroup per CU instead of two. Masked projection, graph replays: 3584 -> 4608, 30% of 700
+// rows 42.6 -> 26.5 us; 1792 -> 5376, 30% of 500 22 -> 16.7; 896 -> 2688, 30% of 300 13.4 -> 12.0,
+// but of 1024 rows (14 steps, 336 tiles) 14.0 us against 19.0 with them.
+constexpr int64_t kDeepSteps = 24;
 constexpr int kNarrowStages = 4;
 struct QkvPlan {
-  int bj = 0;               // 3 or 2: 256 x 64 bj tiles; 0: 128 x 128; 1: 128 x 64 (split only)
+  int bj = 0;               // 3 or 2: 256 x 64 bj tiles; 0: 128 x 128; 1: 128 x 64
   int64_t tiles = 0;
   int64_t splits = 1;       // slices of the hidden dimension (> 1: QKV_PARTIAL)
   int64_t split_steps = 0;  // k-steps per slice
@@ -778,6 +784,11 @@ QkvPlan qkv_plan(int64_t rows, int64_t features, int64_t k_steps, bool allow_spl
   if (pl.tiles * 2 < kCus || (pl.tiles < kCus && small <= 2 * kCus)) {
     pl.bj = 0;  // small tiles
     pl.tiles = small;
+    const int64_t narrow = ((features + 127) / 128) * ((rows + 63) / 64);
+    if (!allow_split && pl.tiles < kCus && (narrow <= kCus || k_steps >= kDeepSteps)) {
+      pl.bj = 1;
+      pl.tiles = narrow;
+    }
     if (allow_split && pl.tiles > 0 && pl.tiles < kCus) {
       pl.bj = rows <= 64 ? 1 : 0;
       const int64_t fit = pl.bj == 1 ? std::max<int64_t>(kCus - 16, pl.tiles) / pl.tiles
@@ -814,6 +825,7 @@ int launch_qkv(const char* fn, const QkvArgs& a, int32_t dtype, hipStream_t st,
     switch (pl.bj) {                                                  \
       case 3: SB_QKV_CASE(DT, 4, 3, kStages); break;                  \
       case 2: SB_QKV_CASE(DT, 4, 2, kStages); break;                  \
+      case 1: SB_QKV_CASE(DT, 2, 1, kNarrowStages); break;            \
       default: SB_QKV_CASE(DT, 2, 2, kStages); break;                 \
     }                                                                 \
   }

@@ -290,3 +290,17 @@ def test_projection_zero_rows(dev):
 def test_projection_split_over_few_rows(dev, dtype, n_rows, hidden, hq, hkv, d, rope):
     x, w, b, pos, bt, cache = _case(400, hidden, hq, hkv, d, n_rows, dtype, 700 + n_rows)
     _check_paged(dev, x, w, b, pos, bt, cache, hq, hkv, d, rope, backend="fused")
+
+
+@pytest.mark.parametrize("seq,hidden,feats", [(65, 128, 200),    # narrow tiles, two k-steps
+                                              (300, 1600, 1000),  # a long k loop
+                                              (1100, 192, 3000)])  # short loop, many tiles
+def test_masked_projection_tile_choice(dev, seq, hidden, feats):
+    g = gen(750 + seq)
+    x, w = randn((seq, hidden), torch.bfloat16, 751), randn((feats, hidden), torch.bfloat16, 752)
+    w = (w.float() * hidden ** -0.5).to(torch.bfloat16)
+    for mask in (torch.rand(seq, generator=g) < 0.4, torch.ones(seq, dtype=torch.bool)):
+        got = tk.masked_qkv_projection(x.to(dev), w.to(dev), mask.to(dev))
+        want = ref.masked_qkv_projection(x, w, mask)
+        _assert_proj_close(got, want, _absdot(x, w))
+        assert not bool(got.cpu()[~mask].any())
