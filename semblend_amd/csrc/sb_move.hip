@@ -155,8 +155,6 @@ struct MoveArgs {
   // v_layers_per_group (0: one interleaved decode with layers_per_group for both planes).
   int k_slices;
   int v_layers_per_group;
-  // Single-layer launches: (head) rows per grid.z slice (0: all of them in one thread's walk).
-  int rows_per_slice;
   int src_index_check;     // ROW_INDEX source: also require src_pos to be a valid paged slot
   int cached_loads;        // source rows may repeat across pairs: cached, not nontemporal, loads
   int vpr;                 // vectors per row
@@ -423,11 +421,7 @@ void move_rows_kernel(MoveArgs a, InlineArg<INLINE> ix) {
     ang_b = static_cast<float>(dst_pos[i]);
   }
 
-  int r_begin = 0, nrows = (l1 - l0) * a.num_heads;  // rows [r_begin, nrows) of the group
-  if (a.rows_per_slice > 0) {
-    r_begin = static_cast<int>(blockIdx.z) * a.rows_per_slice;
-    nrows = min(nrows, r_begin + a.rows_per_slice);
-  }
+  const int nrows = (l1 - l0) * a.num_heads;
   auto row_of = [&](const RowSide& side, int r) {
     const int l = l0 + r / a.num_heads;
     const int h = r - (r / a.num_heads) * a.num_heads;
@@ -447,7 +441,7 @@ void move_rows_kernel(MoveArgs a, InlineArg<INLINE> ix) {
       }
     }
     const int64_t vofs = static_cast<int64_t>(j) * VB;
-    for (int r0 = r_begin; r0 < nrows; r0 += kBatch) {
+    for (int r0 = 0; r0 < nrows; r0 += kBatch) {
       uint32_t w[kBatch][W];
       if (a.cached_loads) {
 #pragma unroll
@@ -700,12 +694,13 @@ bool make_geometry(int64_t head_dim, int64_t esize, std::initializer_list<int64_
 }
 
 // Workgroups that fill the chip (256 CUs x 8 waves per SIMD). A single-layer launch with fewer
-// spreads its heads over grid.z, one batch of kBatch rows per thread, or half a batch where even
-// that leaves most CUs without a workgroup: a thread's batches are serial round trips to memory
+// gives each thread one batch of kBatch rows at most, or half a batch where even that leaves most
+// CUs without a workgroup (the largest divisor of the head count: the head groups take the place
+// of the layers, so the kernel is the same): a thread's batches are serial round trips to memory
 // that too few waves hide. (A rotating slice evaluates its own cos/sin; smaller slices lose to
 // that.) Graph replays of the fused RoPE scatter: 8 heads x 128, 3482 pairs fp16 9.8 -> 8.2 us
-// (2 rows 9.4, 1 row 11.9), 400 pairs 7.0 -> 4.7 (4 rows 5.4), 32 heads x 128, 3482 pairs
-// 40.8 -> 25.2 (2 rows 28.5), 850 pairs 20.4 -> 9.4.
+// (2 rows 9.4, 1 row 11.9), 400 pairs 7.0 -> 4.5 (4 rows 5.4), 32 heads x 128, 3482 pairs
+// 40.8 -> 24.6 (2 rows 28.5), 850 pairs 20.4 -> 8.3.
 constexpr int64_t kFillBlocks = 2048;
 constexpr int64_t kFewBlocks = 256;
 template <int ROT, int SRCM, int DSTM>
@@ -716,16 +711,22 @@ int launch_move(const char* fn, const MoveArgs& a0, int32_t dtype, const Geometr
   a.tpr_log2 = g.tpr_log2;
   const int64_t rows_per_block = kThreads >> g.tpr_log2;
   const int64_t gx = (a.num_pairs + rows_per_block - 1) / rows_per_block;
-  if (gx > 0x7fffffff || grid_y > 65535) return fail(fn, "grid too large");
-  dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(grid_y));
-  if (a.num_layers == 1 && gx * grid_y < kFillBlocks && a.num_heads <= 65535) {
+  if (a.num_layers == 1 && !a.src.layers && !a.dst.layers && gx * grid_y < kFillBlocks) {
     const int64_t batches = (a.num_heads + kBatch - 1) / kBatch;
-    const int rows = gx * grid_y * batches < kFewBlocks ? kBatch / 2 : kBatch;
-    if (a.num_heads > rows) {
-      a.rows_per_slice = rows;
-      grid.z = static_cast<unsigned>((a.num_heads + rows - 1) / rows);
+    int rows = gx * grid_y * batches < kFewBlocks ? kBatch / 2 : kBatch;
+    while (a.num_heads % rows != 0) --rows;
+    const int64_t parts = a.num_heads / rows;
+    if (parts > 1 && rows > 1 && grid_y * parts <= 65535) {
+      a.src.s_layer = rows * a.src.s_head;
+      a.dst.s_layer = rows * a.dst.s_head;
+      a.num_heads = rows;
+      a.num_layers = static_cast<int>(parts);
+      if (a.k_slices > 0) a.k_slices = static_cast<int>(parts);
+      grid_y *= static_cast<int>(parts);
     }
   }
+  if (gx > 0x7fffffff || grid_y > 65535) return fail(fn, "grid too large");
+  dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(grid_y));
 #define SB_MOVE_CASE(DT, VB)                                                              \
   if (dtype == DT && g.vb == VB) {                                                        \
     SB_LAUNCH("move_rows", (move_rows_kernel<DT, VB, ROT, SRCM, DSTM, false>), grid,     \
