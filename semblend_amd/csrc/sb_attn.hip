@@ -1523,12 +1523,14 @@ constexpr int64_t kMergeStrideGrid = 2048;  // merge workgroups of a device-spli
 // kMergeBatch chunks spread them over four groups of lanes where the units are too few to hide a
 // row's chain of loads behind other units (22 chunks of 40 x 4 rows of 8 heads: 5.5 us); with
 // many units the chains overlap, and four groups only add idle loads (28 heads of 614 rows, 7
-// chunks: 22.5 us against 11.5 with one).
+// chunks: 22.5 us against 11.5 with one). A strided merge counts the units of every row that could
+// be computed, and half as many of them are the line (307 of 1024 rows of 14 heads: 6.5 us with
+// four groups, 5.2 with one).
 constexpr int64_t kMergeWideUnits = 512;
 #define SB_MERGE_LAUNCH(DT, D, STRIDED, units, max_chunks, st, args)                          \
   do {                                                                                        \
     const int64_t sb_cap = (STRIDED) ? kMergeStrideGrid : int64_t{0x7fffffff};                \
-    if ((max_chunks) > kMergeBatch && (units) <= kMergeWideUnits) {                           \
+    if ((max_chunks) > kMergeBatch && (units) * ((STRIDED) ? 2 : 1) <= kMergeWideUnits) {     \
       const dim3 sb_mg(static_cast<unsigned>(std::min<int64_t>((units) * 4, sb_cap)));        \
       SB_LAUNCH("attn_merge", (attn_merge_kernel<DT, D, STRIDED, 4>), sb_mg, dim3(256), st,   \
                 args);                                                                        \
