@@ -182,7 +182,10 @@ def host_lib() -> ctypes.PyDLL:
         if not HOST_LIB_PATH.exists():
             raise RuntimeError(f"{HOST_LIB_PATH} is missing; build it with "
                                "`python -m semblend_amd._build`")
-        lib = ctypes.PyDLL(str(HOST_LIB_PATH), mode=os.RTLD_NOW | os.RTLD_LOCAL)
+        try:
+            lib = ctypes.PyDLL(str(HOST_LIB_PATH), mode=os.RTLD_NOW | os.RTLD_LOCAL)
+        except OSError as exc:  # pragma: no cover - depends on the runtime image
+            raise RuntimeError(f"failed to load {HOST_LIB_PATH}: {exc}") from exc
         lib.sb_host_pairs.restype = _i64
         lib.sb_host_pairs.argtypes = [ctypes.py_object, _i64, _vp, _vp]
         lib.sb_host_rotation_counts.restype = _i64
