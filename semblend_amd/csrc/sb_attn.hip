@@ -483,8 +483,9 @@ __host__ __device__ inline int64_t min_chunk(int64_t tile_keys, int64_t row_keys
 //   an item per tile, against 240 slots (ranges are not even). Where that asks for more than 2 W
 //   (as many tiles as slots), W itself.
 //   W up to 5500 keys: 0.72 W, about two rounds, in which early items make up for late ones.
-//   Larger W: W (0.72 W is slower there: 2458 rows of 16000 tokens 281 -> 316 us, 1000 of 32000
-//   186 -> 259).
+//   Larger W, or as many row tiles as slots (which balance by themselves; a finer split would only
+//   add partials, past the no-allocation entry's array in places): W. (0.72 W is slower at large
+//   W: 2458 rows of 16000 tokens 281 -> 316 us, 1000 of 32000 186 -> 259.)
 // Graph replays, items of W keys against these: dense 28 heads x 128, 4096 tokens, 614 rows
 // 76 -> 66.5 us; 28 / 4 heads, 1200 rows of 4096 92 -> 68 us, 400 of 4096 the same, 1200 of 16000
 // 200 -> 174; 32 / 8 heads, 600 of 4096 56 -> 43, 1500 of 8000 147 -> 134; 14 / 2 x 64, 3000 of
@@ -493,7 +494,7 @@ __host__ __device__ inline int64_t min_chunk(int64_t tile_keys, int64_t row_keys
 // work_keys: of tiles / 2 ranges.
 __host__ __device__ inline int64_t item_keys(int64_t t, int64_t whole_keys, int64_t work_keys) {
   const int64_t w = work_keys / (kResidentSlots * kItemsPerSlot);
-  if (w >= 5500) return w;
+  if (w >= 5500 || t >= kResidentSlots) return w;
   if (w >= 2304) return w * 23 / 32;
   const int64_t slots = kResidentSlots - 16 - t / 2;
   if (slots <= 0 || whole_keys > 0xffffffffll) return w;  // (32-bit quotient)

@@ -329,3 +329,14 @@ def test_projection_workspace_covers_the_split_product():
     assert size(2458, 28, 4, 128, 3584, 1) == 2464 * 128 * 4
     assert size(2458, 28, 4, 128, 3584, 0) == 0
     assert size(0, 28, 4, 128, 3584, 1) == 0
+
+
+@pytest.mark.parametrize("hq,hkv,ctx,rows", [(32, 32, 4096, 4000), (64, 8, 4096, 2458),
+                                             (28, 4, 16384, 2458), (28, 4, 9000, 1500),
+                                             (32, 8, 8000, 1300), (32, 8, 4096, 600)])
+def test_split_partials_stay_within_the_no_allocation_array(hq, hkv, ctx, rows):
+    """Key splits finer than one chunk per slot must not push a call that the no-allocation entry
+    serves past its array."""
+    need = _lib.size_query("sb_partial_attention_paged_workspace_size", rows, hq, hkv, 128, 16,
+                           -(-ctx // 16), 2)
+    assert need <= _lib.size_query("sb_partial_attention_paged_noalloc_max_scratch")
