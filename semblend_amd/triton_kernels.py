@@ -229,7 +229,7 @@ def masked_qkv_projection(
     other cases run torch's GEMM in fp32 on the device, as the reference's fallback does.
     Reference: :451-522.
     """
-    dev = _lib.require_device(hidden_states, qkv_weight)
+    dev = _lib.require_device(hidden_states, qkv_weight, qkv_bias)
     seq_len, hidden = hidden_states.shape
     out_features = qkv_weight.shape[0]
     dt = hidden_states.dtype
@@ -307,7 +307,7 @@ def qkv_projection_paged(
 
     if backend not in ("auto", "fused", "library"):
         raise ValueError("backend must be 'auto', 'fused' or 'library'")
-    dev = _lib.require_device(hidden_states, qkv_weight, kv_cache)
+    dev = _lib.require_device(hidden_states, qkv_weight, kv_cache, qkv_bias)
     dt = hidden_states.dtype
     if dt not in (torch.bfloat16, torch.float16):
         raise TypeError("qkv_projection_paged runs bf16 / fp16 (the MFMA path)")
@@ -330,8 +330,10 @@ def qkv_projection_paged(
     n = pos.shape[0]
     if out is None:
         out = torch.empty((n, num_heads, head_dim), dtype=dt, device=dev)
-    elif out.shape != (n, num_heads, head_dim) or out.dtype != dt or not out.is_contiguous():
-        raise ValueError("out must be a contiguous [R, Hq, D] tensor of the input dtype")
+    elif (out.shape != (n, num_heads, head_dim) or out.dtype != dt or not out.is_contiguous()
+          or out.device != dev):
+        raise ValueError("out must be a contiguous [R, Hq, D] tensor of the inputs' dtype and "
+                         "device")
     if n == 0:
         return out
     bias = None if qkv_bias is None else qkv_bias.contiguous()
@@ -750,7 +752,8 @@ def partial_prefill(
     (``_prefill_stages``); other calls, and calls that record gradients, compose the stages
     from this module's functions and torch (``_prefill_composed``), with the same results.
     """
-    dev = _lib.require_device(hidden_states, donor_kv, qkv_weight, output_projection)
+    dev = _lib.require_device(hidden_states, donor_kv, qkv_weight, output_projection, qkv_bias,
+                              output_bias)
     args = (hidden_states, donor_kv, qkv_weight, output_projection, donor_positions,
             target_positions, compute_mask, num_heads, head_dim, qkv_bias, output_bias, scale)
     if _prefill_stages_ok(*args):
@@ -785,7 +788,7 @@ def _prefill_stages_ok(hidden_states, donor_kv, qkv_weight, output_projection, d
             or output_projection.stride(0) * es % 16):
         return False
     for b, n in ((qkv_bias, 3 * feats), (output_bias, output_projection.shape[0])):
-        if b is not None and (tuple(b.shape) != (n,) or not b.is_cuda):
+        if b is not None and (tuple(b.shape) != (n,) or b.device != hidden_states.device):
             return False
     if not isinstance(compute_mask, torch.Tensor) or tuple(compute_mask.shape) != (seq_len,):
         return False

@@ -304,3 +304,27 @@ def test_masked_projection_tile_choice(dev, seq, hidden, feats):
         want = ref.masked_qkv_projection(x, w, mask)
         _assert_proj_close(got, want, _absdot(x, w))
         assert not bool(got.cpu()[~mask].any())
+
+
+def test_bias_or_output_of_another_device_is_refused(dev):
+    """The projections hand the bias and ``out`` to their kernels as raw pointers: one that is
+    not on the inputs' device is refused before a launch."""
+    x, w, b, pos, bt, cache = _case(40, 128, 2, 1, 64, 8, torch.bfloat16, 790)
+    xd, wd = x.to(dev), w.to(dev)
+    mask = torch.ones(40, dtype=torch.bool, device=dev)
+    with pytest.raises(RuntimeError, match="device"):
+        tk.masked_qkv_projection(xd, wd, mask, b)
+    for backend in ("fused", "library"):
+        with pytest.raises(RuntimeError, match="device"):
+            tk.qkv_projection_paged(xd, wd, pos.to(dev), cache.to(dev), bt.to(dev), 2, 1, 64,
+                                    qkv_bias=b, backend=backend)
+        with pytest.raises(ValueError, match="device"):
+            tk.qkv_projection_paged(xd, wd, pos.to(dev), cache.to(dev), bt.to(dev), 2, 1, 64,
+                                    out=torch.empty((8, 2, 64), dtype=x.dtype), backend=backend)
+    donor = torch.zeros((1, 2, 2, 40, 64), dtype=torch.bfloat16, device=dev)
+    w3 = torch.zeros((3 * 128, 128), dtype=torch.bfloat16, device=dev)
+    wo = torch.zeros((64, 128), dtype=torch.bfloat16, device=dev)
+    for biases in ((torch.zeros(384, dtype=torch.bfloat16), None),
+                   (None, torch.zeros(64, dtype=torch.bfloat16))):
+        with pytest.raises(RuntimeError, match="device"):
+            tk.partial_prefill(xd, donor, w3, wo, pos, pos, mask, 2, 64, *biases)

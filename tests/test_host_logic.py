@@ -445,3 +445,28 @@ def test_group_pairs_by_donor():
             start = e
     assert len(seen) == int(((didx >= 0) & (didx < nd)).sum())
     assert group_pairs_by_donor([5], [1], [2], 3) == []
+
+
+# ---- which calls of partial_prefill take its stage kernels ----
+
+def _prefill_args(dtype=torch.bfloat16, s=24, h=2, d=64, hid=64, feats=36, donor_len=30):
+    """Arguments that fit the stage kernels (the route test reads shapes, types and addresses
+    only, so CPU tensors do)."""
+    f = h * d
+    return {"hidden_states": torch.zeros((s, hid), dtype=dtype),
+            "donor_kv": torch.zeros((2, 2, h, donor_len, d), dtype=dtype),
+            "qkv_weight": torch.zeros((3 * f, hid), dtype=dtype),
+            "output_projection": torch.zeros((feats, f), dtype=dtype),
+            "donor_positions": torch.arange(4, dtype=torch.int32),
+            "target_positions": torch.arange(4, dtype=torch.int32),
+            "compute_mask": torch.ones(s, dtype=torch.bool), "num_heads": h, "head_dim": d,
+            "qkv_bias": torch.zeros(3 * f, dtype=dtype),
+            "output_bias": torch.zeros(feats, dtype=dtype), "scale": None}
+
+
+@pytest.mark.parametrize("bias", ["qkv_bias", "output_bias"])
+def test_prefill_route_takes_biases_of_the_inputs_device_only(bias):
+    args = _prefill_args()
+    assert tk._prefill_stages_ok(**args)
+    assert tk._prefill_stages_ok(**dict(args, **{bias: None}))
+    assert not tk._prefill_stages_ok(**dict(args, **{bias: args[bias].to("meta")}))
