@@ -26,6 +26,7 @@ import math
 from dataclasses import dataclass
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -749,8 +750,9 @@ def partial_prefill(
     Attention uses layer 0 only, as in the reference.
 
     head_dim 64 or 128 with one dtype throughout runs as six launches that touch the cache once
-    (``_prefill_stages``); other calls, and calls that record gradients, compose the stages
-    from this module's functions and torch (``_prefill_composed``), with the same results.
+    (``_prefill_stages``); other calls, and calls that torch differentiates (in either mode),
+    transforms or traces, compose the stages from this module's functions and torch
+    (``_prefill_composed``), with the same results.
     """
     dev = _lib.require_device(hidden_states, donor_kv, qkv_weight, output_projection, qkv_bias,
                               output_bias)
@@ -761,11 +763,33 @@ def partial_prefill(
     return _prefill_composed(dev, *args)
 
 
+def _torch_only_sees_values(tensors) -> bool:
+    """Whether a call on these tensors may go to kernels that read their memory, past torch's
+    operators: no tensor subclass, functorch wrapper (vmap, jvp, grad), forward-mode tangent or
+    lazily negated view among them, and no tracer or dispatch mode that follows the operators.
+    (Reverse mode is looked up by the caller.)"""
+    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
+        return False
+    wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+    dual = forward_ad._current_level >= 0
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and not wrapped(t)
+               and not t.is_neg()
+               and not (dual and forward_ad.unpack_dual(t).tangent is not None)
+               for t in tensors if t is not None)
+
+
 def _prefill_stages_ok(hidden_states, donor_kv, qkv_weight, output_projection, donor_positions,
                        target_positions, compute_mask, num_heads, head_dim, qkv_bias,
                        output_bias, scale) -> bool:
     """Whether a call fits the kernels of :func:`_prefill_stages` (shapes, dtypes, alignment)
-    and records no gradient. A call that does not is composed, or rejected there."""
+    and torch neither records nor transforms it. A call that does not is composed, or rejected
+    there."""
+    inputs = (hidden_states, donor_kv, qkv_weight, output_projection, qkv_bias, output_bias)
+    if not isinstance(compute_mask, torch.Tensor) or not _torch_only_sees_values(
+            (*inputs, compute_mask)):
+        return False
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in inputs):
+        return False
     dt = hidden_states.dtype
     if head_dim not in (64, 128) or dt not in _lib.SB_DTYPE or num_heads < 1:
         return False
@@ -790,15 +814,9 @@ def _prefill_stages_ok(hidden_states, donor_kv, qkv_weight, output_projection, d
     for b, n in ((qkv_bias, 3 * feats), (output_bias, output_projection.shape[0])):
         if b is not None and (tuple(b.shape) != (n,) or b.device != hidden_states.device):
             return False
-    if not isinstance(compute_mask, torch.Tensor) or tuple(compute_mask.shape) != (seq_len,):
+    if tuple(compute_mask.shape) != (seq_len,) or len(donor_positions) != len(target_positions):
         return False
-    if len(donor_positions) != len(target_positions):
-        return False
-    if scale is not None and not float(scale) * 1.4426950408889634 > 1e-37:
-        return False
-    return not (torch.is_grad_enabled() and any(
-        t is not None and t.requires_grad
-        for t in (hidden_states, donor_kv, qkv_weight, output_projection, qkv_bias, output_bias)))
+    return scale is None or float(scale) * 1.4426950408889634 > 1e-37
 
 
 def _prefill_stages(dev, hidden_states, donor_kv, qkv_weight, output_projection,

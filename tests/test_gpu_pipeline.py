@@ -252,6 +252,44 @@ def test_partial_prefill_stages_match_composed(dev, dtype, s, hid, h, d, layers,
         assert float((a - b).abs().max()) <= eps * float(b.abs().max())
 
 
+def _stage_args(dev, dtype=torch.float32, s=70, hid=64, h=2, d=64, layers=1, feats=40, seed=950):
+    """Arguments of a call that takes the stage kernels: pairs, 40% computed, both biases."""
+    g = gen(seed)
+    f = h * d
+    rand = lambda *shape, scale=1.0: (torch.randn(shape, generator=g) * scale).to(dtype).to(dev)
+    pos = torch.arange(0, s, 2, dtype=torch.int32).to(dev)
+    return [rand(s, hid), rand(layers, 2, h, s, d), rand(3 * f, hid, scale=hid ** -0.5),
+            rand(feats, f, scale=f ** -0.5), pos, pos.flip(0), (torch.rand(s, generator=g) < 0.4).to(dev),
+            h, d, rand(3 * f, scale=0.1), rand(feats), None]
+
+
+@pytest.mark.parametrize("at", [3, 10])  # output_projection, output_bias
+def test_partial_prefill_forward_derivatives_and_vmap(dev, at):
+    """The output is linear in the output projection and its bias: the forward-mode tangent is
+    the output of a call with the tangent in that input's place, and vmap over that input the
+    calls one by one."""
+    from torch.autograd import forward_ad
+
+    args = _stage_args(dev)
+    assert tk._prefill_stages_ok(*args)
+    zero = list(args)
+    zero[3], zero[10] = torch.zeros_like(args[3]), torch.zeros_like(args[10])
+    zero[at] = torch.randn(args[at].shape, generator=gen(951)).to(dev)
+    want = tk.partial_prefill(*zero).output
+    with forward_ad.dual_level():
+        dual = list(args)
+        dual[at] = forward_ad.make_dual(args[at], zero[at])
+        out = forward_ad.unpack_dual(tk.partial_prefill(*dual).output)
+        assert out.tangent is not None
+    tol = 2.0 ** -18 * float(want.abs().max())  # fp32 sums of 128 products in another order
+    assert float((out.tangent - want).abs().max()) <= tol
+    both = torch.stack([args[at], zero[at]])
+    got = torch.vmap(lambda x: tk.partial_prefill(*args[:at], x, *args[at + 1:]).output)(both)
+    for x, y in zip(both, got):
+        one = tk.partial_prefill(*args[:at], x, *args[at + 1:]).output
+        assert float((y - one).abs().max()) <= 2.0 ** -18 * float(one.abs().max())
+
+
 # ---- Llama-3-8B batch at full size --------------------------------------------------------
 
 def test_llama3_8b_batch_full_size(dev):

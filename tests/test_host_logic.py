@@ -470,3 +470,45 @@ def test_prefill_route_takes_biases_of_the_inputs_device_only(bias):
     assert tk._prefill_stages_ok(**args)
     assert tk._prefill_stages_ok(**dict(args, **{bias: None}))
     assert not tk._prefill_stages_ok(**dict(args, **{bias: args[bias].to("meta")}))
+
+
+@pytest.mark.filterwarnings("ignore::DeprecationWarning")  # of torch.jit's tracer itself
+@pytest.mark.parametrize("name", ["hidden_states", "output_projection", "output_bias"])
+def test_prefill_route_leaves_transformed_calls_to_torch(name):
+    """A tensor with a forward-mode tangent, under vmap, of a subclass or negated lazily, and
+    calls under a tracer or a dispatch mode, are composed from torch's operators."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    args = _prefill_args(torch.float32)
+    t = args[name]
+
+    def route(x):
+        return tk._prefill_stages_ok(**dict(args, **{name: x}))
+
+    assert route(t) and route(torch.nn.Parameter(t, requires_grad=False))
+    assert not route(torch.nn.Parameter(t))
+    with torch.no_grad():
+        assert route(torch.nn.Parameter(t))
+    with forward_ad.dual_level():
+        assert route(t)
+        assert not route(forward_ad.make_dual(t, torch.ones_like(t)))
+    seen = []
+    torch.vmap(lambda x: (seen.append(route(x)), x)[1])(t[None])
+    torch.func.jvp(lambda x: (seen.append(route(x)), x)[1], (t,), (t,))
+    torch.jit.trace(lambda x: (seen.append(route(x)), x + 1)[1], (t,), check_trace=False)
+    assert seen == [False] * 3
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert not route(t.as_subclass(Sub))
+    assert not route(torch._neg_view(t))
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert not route(t)
+    assert route(t)
