@@ -804,6 +804,7 @@ def _prefill_stages_ok(hidden_states, donor_kv, qkv_weight, output_projection, d
     if (seq_len < 1 or not 1 <= layers <= 32767 or seq_len > 1 << 20
             or tuple(qkv_weight.shape) != (3 * feats, hidden)
             or tuple(donor_kv.shape[1:3]) != (2, num_heads) or donor_kv.shape[4] != head_dim
+            or donor_kv.shape[3] < 1  # no donor rows, no address: composed
             or donor_kv.stride(4) != 1 or donor_kv.data_ptr() % 16
             or any(s * es % 16 for s in donor_kv.stride()[:4])):
         return False

@@ -290,6 +290,26 @@ def test_partial_prefill_forward_derivatives_and_vmap(dev, at):
         assert float((y - one).abs().max()) <= 2.0 ** -18 * float(one.abs().max())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_partial_prefill_without_a_donor(dev, dtype):
+    """No donor found: a donor of zero positions and no pairs is the composed form's result, and
+    that of a donor from which nothing is taken."""
+    args = _stage_args(dev, dtype)
+    args[4] = args[5] = torch.zeros(0, dtype=torch.int32, device=dev)
+    full = tk.partial_prefill(*args)
+    args[1] = args[1][:, :, :, :0]
+    for empty in (args[1], args[1].contiguous()):
+        args[1] = empty
+        got = tk.partial_prefill(*args)
+        want = tk._prefill_composed(dev, *args)
+        assert got.positions_computed == full.positions_computed
+        assert_bit_exact(got.kv_cache.cpu(), want.kv_cache.cpu())
+        assert_bit_exact(got.output.cpu(), want.output.cpu())
+        eps = 2.0 ** -18 if dtype == torch.float32 else 2.0 ** -7
+        for a, b in ((got.kv_cache, full.kv_cache), (got.output, full.output)):
+            assert float((a.float() - b.float()).abs().max()) <= eps * float(b.float().abs().max())
+
+
 # ---- Llama-3-8B batch at full size --------------------------------------------------------
 
 def test_llama3_8b_batch_full_size(dev):

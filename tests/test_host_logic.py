@@ -512,3 +512,12 @@ def test_prefill_route_leaves_transformed_calls_to_torch(name):
     with Mode():
         assert not route(t)
     assert route(t)
+
+
+def test_prefill_route_composes_a_call_without_donor_rows():
+    """An empty donor has no address for the stage kernels; a donor of one row has."""
+    none = torch.zeros(0, dtype=torch.int32)
+    assert not tk._prefill_stages_ok(**dict(_prefill_args(donor_len=0), donor_positions=none,
+                                            target_positions=none))
+    assert tk._prefill_stages_ok(**dict(_prefill_args(donor_len=1), donor_positions=none,
+                                        target_positions=none))
