@@ -879,6 +879,8 @@ def _prefill_stages(dev, hidden_states, donor_kv, qkv_weight, output_projection,
         attn = torch.empty((seq_len, feats), dtype=torch.float32, device=dev)
         out = torch.empty((seq_len, output_projection.shape[0]), dtype=dt, device=dev)
         bias32 = None if output_bias is None else output_bias.float().contiguous()
+        if bias32 is not None and bias32.data_ptr() % 16:  # a view into a larger fp32 tensor
+            bias32 = bias32.clone()
         count = torch.empty(4, dtype=torch.uint8, pin_memory=True)
         heads_major = _lib.i64_array((seq_len * head_dim, head_dim, 1))
         _lib.call("sb_partial_attention_rows_f32", attn.data_ptr(), qkv.data_ptr(),

@@ -310,6 +310,18 @@ def test_partial_prefill_without_a_donor(dev, dtype):
             assert float((a.float() - b.float()).abs().max()) <= eps * float(b.float().abs().max())
 
 
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_partial_prefill_output_bias_at_any_offset(dev, offset):
+    """An fp32 output bias that is a view at an address of no multiple of 16 bytes."""
+    args = _stage_args(dev)
+    want = tk.partial_prefill(*args).output
+    flat = torch.zeros(44, device=dev)
+    flat[offset:offset + 40] = args[10]
+    args[10] = flat[offset:offset + 40]
+    assert args[10].data_ptr() % 16 and tk._prefill_stages_ok(*args)
+    assert_bit_exact(tk.partial_prefill(*args).output.cpu(), want.cpu())
+
+
 # ---- Llama-3-8B batch at full size --------------------------------------------------------
 
 def test_llama3_8b_batch_full_size(dev):
