@@ -709,8 +709,9 @@ class PartialPrefillResult:
     kv_cache: [num_layers, 2, num_heads, seq_len, head_dim] assembled target cache;
     positions_computed / positions_reused: compute-mask counts;
     computation_ratio: positions_computed / seq_len;
-    *_time_ms: HIP-event timings of the scatter, projection and attention stages and of the
-    whole call.
+    *_time_ms: HIP-event timings of the scatter (the donor rows' index and the assembly of the
+    cache), projection and attention stages (the attention without its output projection) and
+    of the whole call.
     """
 
     output: torch.Tensor
@@ -848,7 +849,7 @@ def _prefill_stages(dev, hidden_states, donor_kv, qkv_weight, output_projection,
     part_at = ((seq_len + 1) * 4 + 255) // 256 * 256
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)  # positions, count, partials
     index = torch.empty(seq_len, dtype=torch.int32, device=dev)
-    ev = [torch.cuda.Event(enable_timing=True) for _ in range(5)]
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(6)]
     es = hidden_states.element_size()
     with _lib.on_device(dev):
         stream = torch.cuda.current_stream(dev)
@@ -888,13 +889,14 @@ def _prefill_stages(dev, hidden_states, donor_kv, qkv_weight, output_projection,
                   pos + part_at, ws_bytes - part_at, num_heads, seq_len, head_dim,
                   float(scale), _lib.i64_array((head_dim, 3 * feats, 1)), heads_major,
                   heads_major, _lib.i64_array((head_dim, feats, 1)), code, st)
+        ev[4].record(stream)
         _lib.call("sb_prefill_output_projection", out.data_ptr(), attn.data_ptr(),
                   output_projection.data_ptr(), _lib.ptr(bias32), mask.data_ptr(), pos,
                   seq_len, feats, output_projection.shape[0], feats,
                   output_projection.stride(0), out.stride(0), code, st)
         count.copy_(ws[4 * seq_len:4 * seq_len + 4], non_blocking=True)
-        ev[4].record(stream)
-        ev[4].synchronize()
+        ev[5].record(stream)
+        ev[5].synchronize()
     num_computed = int(count.view(torch.int32)[0])
     index_ms = ev[0].elapsed_time(ev[1])
     assemble_ms = ev[2].elapsed_time(ev[3])
@@ -907,7 +909,7 @@ def _prefill_stages(dev, hidden_states, donor_kv, qkv_weight, output_projection,
         scatter_time_ms=index_ms + assemble_ms,
         projection_time_ms=ev[1].elapsed_time(ev[2]),
         attention_time_ms=ev[3].elapsed_time(ev[4]),
-        total_time_ms=ev[0].elapsed_time(ev[4]),
+        total_time_ms=ev[0].elapsed_time(ev[5]),
     )
 
 

@@ -322,6 +322,36 @@ def test_partial_prefill_output_bias_at_any_offset(dev, offset):
     assert_bit_exact(tk.partial_prefill(*args).output.cpu(), want.cpu())
 
 
+@pytest.mark.parametrize("form", ["stages", "composed"])
+def test_partial_prefill_times_the_attention_alone(dev, form, monkeypatch):
+    """attention_time_ms spans the attention launches and not the output projection, the total
+    everything, in both forms."""
+    log = []
+
+    class Event(torch.cuda.Event):
+        def record(self, *args):
+            log.append(self)
+            super().record(*args)
+
+        def elapsed_time(self, end):
+            return float(log.index(end) * 1000 + log.index(self))
+
+    call, linear = tk._lib.call, torch.nn.functional.linear
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(tk._lib, "call", lambda name, *a: (log.append(name), call(name, *a))[1])
+    monkeypatch.setattr(torch.nn.functional, "linear",
+                        lambda *a: (log.append("linear"), linear(*a))[1])
+    args = _stage_args(dev, torch.bfloat16)
+    res = tk.partial_prefill(*args) if form == "stages" else tk._prefill_composed(dev, *args)
+    end, start = divmod(int(res.attention_time_ms), 1000)
+    within = [x for x in log[start:end] if isinstance(x, str)]
+    assert within == ["sb_partial_attention_rows_f32" if form == "stages"
+                      else "sb_partial_prefill_attention"]
+    end, start = divmod(int(res.total_time_ms), 1000)
+    assert (start, end) == (0, len(log) - 1)
+    assert log.count("linear") == (0 if form == "stages" else 1)
+
+
 # ---- Llama-3-8B batch at full size --------------------------------------------------------
 
 def test_llama3_8b_batch_full_size(dev):
