@@ -766,17 +766,20 @@ def partial_prefill(
 
 def _torch_only_sees_values(tensors) -> bool:
     """Whether a call on these tensors may go to kernels that read their memory, past torch's
-    operators: no tensor subclass, functorch wrapper (vmap, jvp, grad), forward-mode tangent or
-    lazily negated view among them, and no tracer or dispatch mode that follows the operators.
-    (Reverse mode is looked up by the caller.)"""
-    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
+    operators: no tensor subclass, no forward-mode tangent among them, no functorch transform
+    (vmap, jvp, grad) around a wrapped one, and no tracer or dispatch mode that follows the
+    operators. (Reverse mode is looked up by the caller.)"""
+    if torch._C._is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
         return False
-    wrapped = torch._C._functorch.is_functorch_wrapped_tensor
-    dual = forward_ad._current_level >= 0
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and not wrapped(t)
-               and not t.is_neg()
-               and not (dual and forward_ad.unpack_dual(t).tangent is not None)
-               for t in tensors if t is not None)
+    if any(type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter
+           for t in tensors if t is not None):
+        return False
+    if forward_ad._current_level >= 0 and any(
+            forward_ad.unpack_dual(t).tangent is not None for t in tensors if t is not None):
+        return False
+    functorch = torch._C._functorch
+    return functorch.peek_interpreter_stack() is None or not any(
+        functorch.is_functorch_wrapped_tensor(t) for t in tensors if t is not None)
 
 
 def _prefill_stages_ok(hidden_states, donor_kv, qkv_weight, output_projection, donor_positions,
@@ -800,23 +803,27 @@ def _prefill_stages_ok(hidden_states, donor_kv, qkv_weight, output_projection, d
         return False
     seq_len, hidden = hidden_states.shape
     feats = num_heads * head_dim
-    layers = donor_kv.shape[0]
+    layers, planes, heads, donor_len, dim = donor_kv.shape
+    st = donor_kv.stride()
     es = hidden_states.element_size()
     if (seq_len < 1 or not 1 <= layers <= 32767 or seq_len > 1 << 20
-            or tuple(qkv_weight.shape) != (3 * feats, hidden)
-            or tuple(donor_kv.shape[1:3]) != (2, num_heads) or donor_kv.shape[4] != head_dim
-            or donor_kv.shape[3] < 1  # no donor rows, no address: composed
-            or donor_kv.stride(4) != 1 or donor_kv.data_ptr() % 16
-            or any(s * es % 16 for s in donor_kv.stride()[:4])):
+            or qkv_weight.shape != (3 * feats, hidden)
+            or planes != 2 or heads != num_heads or dim != head_dim
+            or donor_len < 1  # no donor rows, no address: composed
+            or st[4] != 1 or donor_kv.data_ptr() % 16
+            or (st[0] | st[1] | st[2] | st[3]) * es % 16):
         return False
-    if (output_projection.shape[1] != feats or output_projection.shape[0] % 4
-            or output_projection.stride(1) != 1 or output_projection.data_ptr() % 16
-            or output_projection.stride(0) * es % 16):
+    out_features, in_features = output_projection.shape
+    st = output_projection.stride()
+    if (in_features != feats or out_features % 4 or st[1] != 1
+            or output_projection.data_ptr() % 16 or st[0] * es % 16):
         return False
-    for b, n in ((qkv_bias, 3 * feats), (output_bias, output_projection.shape[0])):
-        if b is not None and (tuple(b.shape) != (n,) or b.device != hidden_states.device):
+    for b, n in ((qkv_bias, 3 * feats), (output_bias, out_features)):
+        # (a lazily negated bias: the matrices above would not have unit strides)
+        if b is not None and (b.shape != (n,) or b.device != hidden_states.device
+                              or b.is_neg()):
             return False
-    if tuple(compute_mask.shape) != (seq_len,) or len(donor_positions) != len(target_positions):
+    if compute_mask.shape != (seq_len,) or len(donor_positions) != len(target_positions):
         return False
     return scale is None or float(scale) * 1.4426950408889634 > 1e-37
 
