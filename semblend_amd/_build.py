@@ -16,6 +16,7 @@ import shutil
 import subprocess
 import sys
 import sysconfig
+import warnings
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -73,9 +74,17 @@ def _compile(src: Path, hipcc: str, verbose: bool) -> Path:
 
 
 def _build_host(hipcc: str, verbose: bool) -> None:
+    """The list converters, for this interpreter. They are optional (the package converts lists in
+    Python without them): where the interpreter's headers are not installed there is no library."""
+    include = Path(sysconfig.get_paths()["include"])
+    if not (include / "Python.h").exists():
+        HOST_LIB_PATH.unlink(missing_ok=True)
+        warnings.warn(f"{HOST_LIB_NAME} is not built: no Python.h in {include}", RuntimeWarning)
+        return
     tmp = HOST_LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc, "-O3", "-std=c++17", "-fPIC", "-shared", "-x", "c++", str(CSRC / "sb_host.cpp"),
-           f"-I{sysconfig.get_paths()['include']}", "-o", str(tmp)]
+           f"-I{include}", f'-DSB_HOST_SOABI="{sysconfig.get_config_var("SOABI")}"',
+           "-o", str(tmp)]
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)

@@ -11,6 +11,8 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import os
+import sysconfig
+import warnings
 from pathlib import Path
 
 import torch
@@ -127,9 +129,10 @@ SIZE_QUERIES: dict[str, list] = {
     "sb_qkv_projection_paged_workspace_size": [_i64, _i64, _i64, _i64, _i64, _i32],
 }
 
-# Python index lists to host arrays (csrc/sb_host.cpp).
+# Python index lists to host arrays (csrc/sb_host.cpp): None until first wanted, False where it
+# does not load into this interpreter (lists are then converted in Python).
 HOST_LIB_PATH = Path(__file__).resolve().parent / "libsemblend_host.so"
-_host: ctypes.PyDLL | None = None
+_host: ctypes.PyDLL | bool | None = None
 _lib: ctypes.CDLL | None = None
 _load_error: str | None = None
 
@@ -175,30 +178,45 @@ def lib() -> ctypes.CDLL:
     return _load()
 
 
-def host_lib() -> ctypes.PyDLL:
-    """The loaded list converters; raises RuntimeError if they cannot be loaded."""
-    global _host
-    if _host is None:
-        if not HOST_LIB_PATH.exists():
-            raise RuntimeError(f"{HOST_LIB_PATH} is missing; build it with "
-                               "`python -m semblend_amd._build`")
-        try:
-            lib = ctypes.PyDLL(str(HOST_LIB_PATH), mode=os.RTLD_NOW | os.RTLD_LOCAL)
-        except OSError as exc:  # pragma: no cover - depends on the runtime image
-            raise RuntimeError(f"failed to load {HOST_LIB_PATH}: {exc}") from exc
+def _load_host() -> ctypes.PyDLL:
+    if not HOST_LIB_PATH.exists():
+        raise OSError(f"{HOST_LIB_PATH} is missing; build it with "
+                      "`python -m semblend_amd._build`")
+    lib = ctypes.PyDLL(str(HOST_LIB_PATH), mode=os.RTLD_NOW | os.RTLD_LOCAL)
+    try:
+        lib.sb_host_soabi.restype = ctypes.c_char_p
+        lib.sb_host_soabi.argtypes = []
+        built, here = lib.sb_host_soabi().decode(), sysconfig.get_config_var("SOABI")
+        if built != here:  # object layouts are the interpreter's own
+            raise OSError(f"{HOST_LIB_PATH} was built for {built}, this interpreter is {here}")
         lib.sb_host_pairs.restype = _i64
         lib.sb_host_pairs.argtypes = [ctypes.py_object, _i64, _vp, _vp]
         lib.sb_host_rotation_counts.restype = _i64
         lib.sb_host_rotation_counts.argtypes = [ctypes.py_object, _i64, _i64, _i64, _vp, _vp,
                                                 _i64p]
-        _host = lib
-    return _host
+    except AttributeError as exc:
+        raise OSError(f"{HOST_LIB_PATH} does not export the expected functions ({exc})") from exc
+    return lib
+
+
+def host_lib() -> ctypes.PyDLL | None:
+    """The list converters, or None where they cannot be loaded into this interpreter: callers
+    then convert in Python, slower and with the same results (said once, as a warning)."""
+    global _host
+    if _host is None:
+        try:
+            _host = _load_host()
+        except OSError as exc:
+            _host = False
+            warnings.warn(f"index lists are converted in Python: {exc}", RuntimeWarning,
+                          stacklevel=3)
+    return _host or None
 
 
 def available() -> bool:
+    """Whether the kernel library loads (the list converters are optional)."""
     try:
         _load()
-        host_lib()
         return True
     except RuntimeError:
         return False

@@ -31,6 +31,13 @@ constexpr int64_t kI32Max = std::numeric_limits<int32_t>::max();
 
 }  // namespace
 
+// The interpreter ABI (sysconfig's SOABI) this library was built for. It reads list, tuple and int
+// objects through that interpreter's macros, so the loader compares it before any other call.
+#ifndef SB_HOST_SOABI
+#error "SB_HOST_SOABI must name the interpreter ABI"
+#endif
+extern "C" const char* sb_host_soabi() { return SB_HOST_SOABI; }
+
 // first[i], second[i] of the n pairs of `pairs`. Returns n, or -1.
 extern "C" int64_t sb_host_pairs(PyObject* pairs, int64_t n, int32_t* first, int32_t* second) {
   if (!PyList_CheckExact(pairs) || PyList_GET_SIZE(pairs) != n) return -1;

@@ -464,11 +464,12 @@ def _rotation_counts(positions: list[int], block_size: int,
 def _rotation_arrays(positions, block_size: int, num_blocks_per_seq: int):
     """``_rotation_counts`` as (int32 host array of the positions, of their counts, entries used
     in both, positions processed); plain lists of ints are resolved natively."""
-    if type(positions) is list:
+    host = _lib.host_lib() if type(positions) is list else None
+    if host is not None:
         n = len(positions)
         keys, reps = (ctypes.c_int32 * n)(), (ctypes.c_int32 * n)()
         used = ctypes.c_int64(0)
-        done = _lib.host_lib().sb_host_rotation_counts(
+        done = host.sb_host_rotation_counts(
             positions, n, block_size, num_blocks_per_seq, keys, reps, used)
         if done >= 0:
             return keys, reps, used.value, done
@@ -711,11 +712,12 @@ def paged_layout(kv_cache: torch.Tensor, layout: str | None = None):
 def _pairs_on_device(permutation, dev: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
     """(sources, targets) int32 device tensors from a list of (src, tgt) pairs or a [P, 2]
     tensor, uploaded once from pinned memory without blocking the host."""
-    if type(permutation) is list and not torch.cuda.is_current_stream_capturing():
+    host = _lib.host_lib() if type(permutation) is list else None
+    if host is not None and not torch.cuda.is_current_stream_capturing():
         n = len(permutation)
         both = torch.empty((2, n), dtype=torch.int32, pin_memory=True)
         at = both.data_ptr()
-        if _lib.host_lib().sb_host_pairs(permutation, n, at, at + 4 * n) == n:
+        if host.sb_host_pairs(permutation, n, at, at + 4 * n) == n:
             both = both.to(dev, non_blocking=True)
             return both[0], both[1]
     if isinstance(permutation, torch.Tensor):

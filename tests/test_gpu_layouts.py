@@ -320,3 +320,16 @@ def test_rope_deltas_layers_7b_shape(dev):
         wv = rc.standard_view(want, "vllm")
         assert_bit_exact(gv[:, 1], wv[:, 1])
         assert_rope_close(gv, wv)
+
+
+def test_pair_lists_without_the_native_converter(dev, monkeypatch):
+    """The pairs of a list are the same device arrays with and without the converters' library."""
+    perm = [(3, 70), (70, 3), (-1, 5), (2 ** 31 - 1, 0)]
+    for pairs in (perm, [list(p) for p in perm], perm[:1]):
+        with monkeypatch.context() as m:
+            native = rc._pairs_on_device(pairs, dev)
+            m.setattr(rc._lib, "_host", False)
+            plain = rc._pairs_on_device(pairs, dev)
+        for a, b in zip(native, plain):
+            assert a.dtype == b.dtype == torch.int32 and a.tolist() == b.tolist()
+        assert [tuple(p) for p in zip(*(x.tolist() for x in native))] == [tuple(p) for p in pairs]

@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import random
 import sys
+import warnings
 
 import numpy as np
 import pytest
@@ -265,6 +266,40 @@ def test_native_pairs_take_exact_ints_only():
                 [torch.tensor([1, 2])]):
         assert native(bad) == -1
     assert _lib.host_lib().sb_host_pairs(((1, 2),), 1, out.data_ptr(), out.data_ptr()) == -1
+
+
+@pytest.mark.parametrize("why", ["missing", "another interpreter"])
+def test_list_converters_are_optional(why, monkeypatch, tmp_path):
+    """Without the converters' library, or with one built for another interpreter, the package
+    is available and lists are resolved in Python, which is said once."""
+    from semblend_amd import _lib
+
+    want = rc._rotation_arrays([5, 5, -1, 3], 16, 5)
+    monkeypatch.setattr(_lib, "_host", None)
+    if why == "missing":
+        monkeypatch.setattr(_lib, "HOST_LIB_PATH", tmp_path / "none.so")
+    else:
+        monkeypatch.setattr(_lib.sysconfig, "get_config_var", lambda name: "cpython-299-none")
+    with pytest.warns(RuntimeWarning, match="missing" if why == "missing" else "cpython-299"):
+        keys, reps, n, done = rc._rotation_arrays([5, 5, -1, 3], 16, 5)
+    assert (list(keys), list(reps), n, done) == (
+        list(want[0][:n]), list(want[1][:n]), want[2], want[3])
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.host_lib() is None and _lib.available()
+
+
+def test_build_without_interpreter_headers(monkeypatch, tmp_path):
+    """Without Python.h the build leaves no (stale) converter library and does not fail."""
+    from semblend_amd import _build
+
+    stale = tmp_path / "host.so"
+    stale.write_bytes(b"stale")
+    monkeypatch.setattr(_build, "HOST_LIB_PATH", stale)
+    monkeypatch.setattr(_build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    with pytest.warns(RuntimeWarning, match="Python.h"):
+        _build._build_host("no-such-compiler", False)
+    assert not stale.exists()
 
 
 def test_rotation_counts_agree_with_oracle_count():
