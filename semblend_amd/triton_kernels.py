@@ -238,6 +238,9 @@ def masked_qkv_projection(
     if (dt in (torch.bfloat16, torch.float16) and qkv_weight.dtype == dt
             and (qkv_bias is None or qkv_bias.dtype == dt) and hidden % 64 == 0
             and out_features % 8 == 0 and seq_len > 0
+            # the kernel reads these whole: shorter ones are torch's to broadcast or refuse
+            and mask.numel() >= seq_len and qkv_weight.shape[1] >= hidden
+            and (qkv_bias is None or qkv_bias.numel() >= out_features)
             and _mfma_rows_ok(hidden_states, qkv_weight)):
         out = torch.empty((seq_len, out_features), dtype=dt, device=dev)
         mask_u8 = (mask if mask.dtype == torch.bool else mask != 0).contiguous().view(torch.uint8)
@@ -414,6 +417,8 @@ def partial_prefill_attention(
     k = key if key.stride(-1) == 1 else key.contiguous()
     v = value if value.stride(-1) == 1 else value.contiguous()
     mask = compute_mask.to(device=dev)
+    if mask.numel() < seq_len:
+        raise ValueError("compute_mask must have one entry per position")
     if mask.dtype != torch.bool:
         mask = mask != 0
     mask = mask.contiguous().view(torch.uint8)

@@ -328,3 +328,19 @@ def test_bias_or_output_of_another_device_is_refused(dev):
                    (None, torch.zeros(64, dtype=torch.bfloat16))):
         with pytest.raises(RuntimeError, match="device"):
             tk.partial_prefill(xd, donor, w3, wo, pos, pos, mask, 2, 64, *biases)
+
+
+def test_masked_projection_refuses_short_operands(dev):
+    """A bias, mask or weight shorter than the kernels read is refused on the host; a mask of one
+    entry is broadcast, as torch's form of the projection does."""
+    x, w = randn((40, 128), torch.bfloat16, 795).to(dev), randn((64, 128), torch.bfloat16, 796).to(dev)
+    mask = torch.ones(40, dtype=torch.bool, device=dev)
+    for args in ((x, w, mask, torch.zeros(63, dtype=x.dtype, device=dev)), (x, w, mask[:39]),
+                 (x, w[:, :64].contiguous(), mask)):
+        with pytest.raises(RuntimeError):
+            tk.masked_qkv_projection(*args)
+    want = tk.masked_qkv_projection(x, w, mask)
+    _assert_proj_close(tk.masked_qkv_projection(x, w, mask[:1]), want, _absdot(x, w).cpu())
+    q = torch.zeros((2, 40, 64), dtype=x.dtype, device=dev)
+    with pytest.raises(ValueError, match="compute_mask"):
+        tk.partial_prefill_attention(q, q, q, mask[:39])
