@@ -2476,8 +2476,7 @@ extern "C" int sb_partial_attention_paged_noalloc(
   if (num_blocks_per_seq <= 0) return fail(fn, "empty block table or pool");
   const int64_t need = sb_partial_attention_paged_workspace_size(
       num_rows, num_q_heads, num_kv_heads, head_dim, block_size, num_blocks_per_seq, dtype);
-  // (fp32 partials past the array's size: the call runs unsplit)
-  if (need > kNoAllocScratchBytes && dtype != SB_DTYPE_F32)
+  if (need > kNoAllocScratchBytes)  // (16-bit calls only: fp32 partials are at most 102 MB)
     return fail(fn, "this call needs " + std::to_string(need) +
                         " bytes of split-key partials; the no-allocation entry holds at most " +
                         std::to_string(kNoAllocScratchBytes) +
@@ -2496,7 +2495,6 @@ extern "C" int sb_partial_attention_paged_noalloc(
   a.num_rows = num_rows;
   a.nb_per_seq = num_blocks_per_seq;
   a.kv_len = num_blocks_per_seq * block_size;
-  return launch_attention(fn, a, dtype, num_rows, aligned16, ws,
-                          std::min(need, kNoAllocScratchBytes),
+  return launch_attention(fn, a, dtype, num_rows, aligned16, ws, need,
                           static_cast<hipStream_t>(stream));
 }

@@ -39,6 +39,8 @@ constexpr int kF32Threads = 64 * kF32Waves;
 // work unsplit; below that the key range splits so that about 1024 chunks run, none shorter
 // than two tiles of 4096 / D keys: 1000 tokens, 400 rows, 14 / 2 heads x 64 take 24 us against
 // 29.5 us with one tile and 32 us with four (merge and set-up against idle CUs).
+// With t < 1024 row tiles x KV heads a split has at most 2048 / t + 1 chunks each: partials of
+// 3071 x 64 rows of D + 2 floats, 102 MB, whatever the call.
 constexpr int64_t kF32Slots = 1024;
 #ifndef SB_F32_MIN_TILES
 #define SB_F32_MIN_TILES 2

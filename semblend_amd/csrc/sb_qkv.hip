@@ -817,18 +817,16 @@ int launch_qkv(const char* fn, const QkvArgs& a, int32_t dtype, hipStream_t st,
   const dim3 grid(static_cast<unsigned>(blocks));
 #define SB_QKV_CASE(DT, BI, BJ, ST)                                                           \
   SB_LAUNCH("qkv_mfma", (qkv_mfma_kernel<DT, MODE, BI, BJ, ST>), grid, dim3(kQThreads), st, a)
+  // (128 x 64 tiles: split products and the dense form only, see qkv_plan)
 #define SB_QKV_DT(DT)                                                 \
-  if constexpr (MODE == QKV_PARTIAL) {                                \
+  if constexpr (MODE != QKV_SPLIT) {                                  \
     if (pl.bj == 1) SB_QKV_CASE(DT, 2, 1, kNarrowStages);             \
-    else SB_QKV_CASE(DT, 2, 2, kStages);                              \
-  } else {                                                            \
-    switch (pl.bj) {                                                  \
-      case 3: SB_QKV_CASE(DT, 4, 3, kStages); break;                  \
-      case 2: SB_QKV_CASE(DT, 4, 2, kStages); break;                  \
-      case 1: SB_QKV_CASE(DT, 2, 1, kNarrowStages); break;            \
-      default: SB_QKV_CASE(DT, 2, 2, kStages); break;                 \
-    }                                                                 \
-  }
+  }                                                                   \
+  if constexpr (MODE != QKV_PARTIAL) {                                \
+    if (pl.bj == 3) SB_QKV_CASE(DT, 4, 3, kStages);                   \
+    if (pl.bj == 2) SB_QKV_CASE(DT, 4, 2, kStages);                   \
+  }                                                                   \
+  if (pl.bj == 0) SB_QKV_CASE(DT, 2, 2, kStages);
   if (dtype == SB_DTYPE_BF16) {
     SB_QKV_DT(SB_DTYPE_BF16)
   } else {

@@ -340,3 +340,14 @@ def test_split_partials_stay_within_the_no_allocation_array(hq, hkv, ctx, rows):
     need = _lib.size_query("sb_partial_attention_paged_workspace_size", rows, hq, hkv, 128, 16,
                            -(-ctx // 16), 2)
     assert need <= _lib.size_query("sb_partial_attention_paged_noalloc_max_scratch")
+
+
+@pytest.mark.parametrize("hq,hkv,rows,ctx", [(12, 3, 5449, 335556), (32, 32, 2000, 4096),
+                                             (128, 1, 500, 1 << 20), (1023, 1023, 1, 4096)])
+def test_fp32_partials_stay_within_the_no_allocation_array(hq, hkv, rows, ctx):
+    """At most 2048 / t + 1 chunks of each of t < 1024 (row tile, KV head) pairs: 3071 tiles of 64
+    rows of head_dim + 2 floats."""
+    need = _lib.size_query("sb_partial_attention_paged_workspace_size", rows, hq, hkv, 128, 16,
+                           -(-ctx // 16), 0)
+    assert need <= 3071 * 64 * 130 * 4
+    assert need <= _lib.size_query("sb_partial_attention_paged_noalloc_max_scratch")
