@@ -693,15 +693,22 @@ bool make_geometry(int64_t head_dim, int64_t esize, std::initializer_list<int64_
   return true;
 }
 
-// Workgroups that fill the chip (256 CUs x 8 waves per SIMD). A single-layer launch with fewer
+// A single-layer launch of too few workgroups to hide a thread's serial round trips to memory
 // gives each thread one batch of kBatch rows at most, or half a batch where even that leaves most
 // CUs without a workgroup (the largest divisor of the head count: the head groups take the place
-// of the layers, so the kernel is the same): a thread's batches are serial round trips to memory
-// that too few waves hide. (A rotating slice evaluates its own cos/sin; smaller slices lose to
-// that.) Graph replays of the fused RoPE scatter: 8 heads x 128, 3482 pairs fp16 9.8 -> 8.2 us
-// (2 rows 9.4, 1 row 11.9), 400 pairs 7.0 -> 4.5 (4 rows 5.4), 32 heads x 128, 3482 pairs
-// 40.8 -> 24.6 (2 rows 28.5), 850 pairs 20.4 -> 8.3.
-constexpr int64_t kFillBlocks = 2048;
+// of the layers, so the kernel is the same). A rotating slice evaluates its own cos/sin; smaller
+// slices lose to that. Graph replays of the fused RoPE scatter: 8 heads x 128, 3482 pairs fp16
+// 9.8 -> 8.2 us (2 rows 9.4, 1 row 11.9), 400 pairs 7.0 -> 4.5 (4 rows 5.4), 32 heads x 128, 3482
+// pairs 40.8 -> 24.6 (2 rows 28.5), 850 pairs 20.4 -> 8.3.
+// Where the line lies, in workgroups of the undivided launch (time undivided / divided, plain and
+// rotating scatter, bf16 and fp32 rows of 128, the same within 2% for bf16 x 64):
+//   8-28 heads:  1100 1.03-1.15, 1300 1.00-1.09, 1500 0.94-1.03, 1700 0.94-1.01, 2040 0.94-1.01
+//   32-64 heads: 1300 1.02-1.13, 1900 0.99-1.09, 2040 0.98-1.04 (eight batches and more to hide)
+//   no multiple of 4 (slices of 2 or 3 rows): 1100 1.01-1.17, 1300 0.90-1.13, 1700 0.83-1.00
+constexpr int64_t kFillBlocks = 5 * 256;
+constexpr int64_t kFillBlocksDeep = 7 * 256 + 128;
+constexpr int64_t kFillBlocksPartial = 4 * 256 + 128;
+constexpr int64_t kDeepBatches = 8;
 constexpr int64_t kFewBlocks = 256;
 template <int ROT, int SRCM, int DSTM>
 int launch_move(const char* fn, const MoveArgs& a0, int32_t dtype, const Geometry& g,
@@ -711,8 +718,11 @@ int launch_move(const char* fn, const MoveArgs& a0, int32_t dtype, const Geometr
   a.tpr_log2 = g.tpr_log2;
   const int64_t rows_per_block = kThreads >> g.tpr_log2;
   const int64_t gx = (a.num_pairs + rows_per_block - 1) / rows_per_block;
-  if (a.num_layers == 1 && !a.src.layers && !a.dst.layers && gx * grid_y < kFillBlocks) {
-    const int64_t batches = (a.num_heads + kBatch - 1) / kBatch;
+  const int64_t batches = (a.num_heads + kBatch - 1) / kBatch;
+  const int64_t fill = a.num_heads % kBatch != 0   ? kFillBlocksPartial
+                       : batches >= kDeepBatches ? kFillBlocksDeep
+                                                 : kFillBlocks;
+  if (a.num_layers == 1 && !a.src.layers && !a.dst.layers && gx * grid_y < fill) {
     int rows = gx * grid_y * batches < kFewBlocks ? kBatch / 2 : kBatch;
     while (a.num_heads % rows != 0) --rows;
     const int64_t parts = a.num_heads / rows;

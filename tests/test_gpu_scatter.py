@@ -298,3 +298,30 @@ def test_single_layer_scatter_spreads_heads(dev, dtype, heads, pairs):
     want = ref.rope_correct_scatter_paged(cache.clone(), donor, bt, dp, tp)
     assert_bit_exact(got[:, 1], want[:, 1])
     assert_rope_close(got[:, 0], want[:, 0])
+
+
+@pytest.mark.parametrize("heads,pairs", [
+    (8, 20448), (8, 20449),    # 1278 and 1280 workgroups: head groups below 1280
+    (6, 18400), (6, 18401),    # heads of no whole batch: below 1152
+    (32, 30688), (32, 30689)])  # eight batches: below 1920
+def test_single_layer_scatter_at_the_head_group_line(dev, heads, pairs):
+    """The same rows on both sides of the line between head groups and whole rows of heads."""
+    from semblend_amd import rope_correction as rc
+    from tests.helpers import assert_rope_close, gen, randn
+
+    g = gen(50 + heads)
+    s, bs, d, dtype = 31000, 16, 64, torch.bfloat16
+    nb = -(-s // bs)
+    bt = torch.randperm(nb + 2, generator=g)[:nb].to(torch.int32)
+    dp = torch.randperm(s, generator=g)[:pairs].to(torch.int32)
+    tp = torch.randperm(s, generator=g)[:pairs].to(torch.int32)
+    donor = randn((2, heads, s, d), dtype, 52)
+    cache = torch.zeros((nb + 2, 2, heads, bs, d), dtype=dtype)
+    got = tk.scatter_donor_kv_paged(cache.to(dev), donor.to(dev), bt.to(dev), dp.to(dev),
+                                    tp.to(dev))
+    assert_bit_exact(got, ref.scatter_donor_kv_paged(cache.clone(), donor, bt, dp, tp))
+    got = rc.rope_correct_scatter_paged(cache.to(dev), donor.to(dev), bt.to(dev), dp.to(dev),
+                                        tp.to(dev)).cpu()
+    want = ref.rope_correct_scatter_paged(cache.clone(), donor, bt, dp, tp)
+    assert_bit_exact(got[:, 1], want[:, 1])
+    assert_rope_close(got[:, 0], want[:, 0])
