@@ -500,10 +500,17 @@ __global__ void rope_index_kernel(const int32_t* dpos, int64_t num_pairs, int64_
 }
 
 // Both steps in one launch: a workgroup resolves kIndexThreads positions in LDS, scanning the
-// whole pair list (up to kIndexScanPairs: 32 rounds of loads), instead of one workgroup that
-// zeroes and counts the table in memory (8192 positions and pairs: 6.1-6.5 us, here 4.2-4.8 us).
+// whole pair list, instead of one workgroup that zeroes and counts the table in memory (8192
+// positions and pairs: 6.1-6.5 us, here 3.7-4.9 us). Where the list is long, or the workgroups that
+// each scan it are many, a parallel fill and global atomics in two launches are faster. The whole
+// call on one head of 64, two launches / this one, us: 500-8000 positions with any list of that
+// length 7.8-8.7 / 6.0-8.3; 32768 positions with 16000 pairs 10.7 / 10.0, with 32768 11.8 / 12.4;
+// 524288 with 16000 47.8 / 47.2, with 32768 53.1 / 53.5; 1048576 with 8000 77.7 / 77.1, with 16000
+// 81.7 / 83.3, with 32768 88.9 / 93.7.
 constexpr int kIndexThreads = 1024;
-constexpr int64_t kIndexScanPairs = 32 * kIndexThreads;
+constexpr int64_t kIndexScanPairs = 24 * 1024;
+constexpr int64_t kIndexLongSeq = 1 << 19;
+constexpr int64_t kIndexScanPairsLong = 8 * 1024;  // past kIndexLongSeq positions
 __global__ __launch_bounds__(kIndexThreads) void rope_index_scan_kernel(const int32_t* dpos,
                                                                         int64_t num_pairs,
                                                                         int64_t seq_len,
@@ -1232,7 +1239,8 @@ int rope_k_impl(const char* fn, void* out, const void* k, const int32_t* donor_p
   const int64_t n = 2 * seq_len;
   if (distinct) {
     // no index
-  } else if (num_pairs <= kIndexScanPairs && seq_len <= int64_t{0x7fffffff} * kIndexThreads) {
+  } else if (num_pairs <= (seq_len <= kIndexLongSeq ? kIndexScanPairs : kIndexScanPairsLong) &&
+             seq_len <= int64_t{0x7fffffff} * kIndexThreads) {
     SB_LAUNCH("rope_index", rope_index_scan_kernel,
               dim3(static_cast<unsigned>((seq_len + kIndexThreads - 1) / kIndexThreads)),
               dim3(kIndexThreads), st, donor_pos, num_pairs, seq_len, ws);

@@ -379,3 +379,35 @@ def test_rope_k_index_edges(dev, seq, pairs):
     ok = (dp >= 0) & (dp < seq)
     want = ref.rope_correct_k(k.clone(), dp[ok], tp[ok], head_dim=64)
     assert_rope_close(got, want, composed=True)
+
+
+@pytest.mark.parametrize("seq,pairs,launches", [
+    (2000, 24576, 1), (2000, 24577, 2), (524288, 8193, 1), (524289, 8192, 1), (524289, 8193, 2)])
+def test_rope_k_index_launches(dev, seq, pairs, launches):
+    """Short lists are indexed in one launch; long ones, and those of many positions, by a fill
+    and atomics. The rotated rows are the same either way."""
+    from semblend_amd import _lib
+
+    g = gen(70 + pairs)
+    k = randn((1, 1, seq, 64), torch.bfloat16, 71)
+    dp = torch.full((pairs,), -1, dtype=torch.int32)
+    dp[::100] = torch.randint(0, seq, (dp[::100].numel(),), generator=g).to(torch.int32)
+    dp[-1] = seq - 1
+    tp = dp + 5
+    kd, dd, td = k.to(dev), dp.to(dev), tp.to(dev)
+    _lib.kernel_timing(True)
+    try:
+        got = rc.rope_correct_k(kd, dd, td, head_dim=64)
+        torch.cuda.synchronize()
+        seen = sum(_lib.kernel_time(name)[1] for name in ("fill_i32", "rope_index"))
+    finally:
+        _lib.kernel_timing(False)
+    assert seen == launches
+    rows = dp[dp >= 0].long().unique()
+    sub = {int(r): i for i, r in enumerate(rows)}
+    small = torch.tensor([sub[int(x)] for x in dp[dp >= 0]], dtype=torch.int32)
+    want = ref.rope_correct_k(k[:, :, rows].clone(), small, small + 5, head_dim=64)
+    assert_rope_close(got[:, :, rows.to(dev)], want, composed=True)
+    rest = torch.ones(seq, dtype=torch.bool)
+    rest[rows] = False
+    assert torch.equal(got.cpu()[:, :, rest], k[:, :, rest])
