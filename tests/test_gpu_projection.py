@@ -344,3 +344,17 @@ def test_masked_projection_refuses_short_operands(dev):
     q = torch.zeros((2, 40, 64), dtype=x.dtype, device=dev)
     with pytest.raises(ValueError, match="compute_mask"):
         tk.partial_prefill_attention(q, q, q, mask[:39])
+
+
+@pytest.mark.parametrize("live", [0, 1, 64, 65, 280, 699, 700])
+def test_masked_projection_numbers_the_live_tiles(dev, live):
+    """264 possible tiles of 128 x 64 (more than one per CU), of which those of the computed rows
+    run: none, one row, edges of row tiles, and all but one."""
+    seq, hidden, feats = 700, 1600, 3072
+    x, w = randn((seq, hidden), torch.bfloat16, 761), randn((feats, hidden), torch.float32, 762)
+    w = (w * hidden ** -0.5).to(torch.bfloat16)
+    mask = torch.zeros(seq, dtype=torch.bool)
+    mask[torch.randperm(seq, generator=gen(763))[:live]] = True
+    got = tk.masked_qkv_projection(x.to(dev), w.to(dev), mask.to(dev))
+    _assert_proj_close(got, ref.masked_qkv_projection(x, w, mask), _absdot(x, w))
+    assert not bool(got.cpu()[~mask].any())
