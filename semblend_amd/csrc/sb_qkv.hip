@@ -758,6 +758,14 @@ constexpr int64_t kMinSplitSteps = SB_QKV_MIN_SPLIT_STEPS;
 // (16 CUs left to the RoPE table). Graph replays before and after: 7B shape 1 / 16 / 64 rows
 // 17.7 / 18.8 / 20.8 -> 11.9 / 12.6 / 14.5 us, 0.5B 12.9 / 12.7 / 13.2 -> 7.7 / 8.4 / 9.5 us,
 // Llama-3-8B (4096 -> 6144) 19.3 / 20.6 / 23.3 -> 15.0 / 15.6 / 17.4 us.
+// Without RoPE a product of fewer than 2 kMinSplitSteps steps is one launch when it is not split
+// (with RoPE the table is a second one), so there the steps saved have to cover the epilogue
+// launch, about 4 steps, and the partials, about a quarter of a step for each 128 KB. No RoPE,
+// unsplit / split: 896 -> 1152 (9 steps saved) 1 row 9.9 / 8.0 us, 129 rows (1.8 MB) 11.2 / 10.9,
+// 200 rows (2.8 MB) 11.2 / 11.5; 768 -> 2304 (8 saved) 65 rows (1.8 MB) 10.0 / 9.6, 129 rows (3.6
+// MB) 10.5 / 11.4; 512 -> 768 (4 saved) 1 row 7.8 / 7.3, 64 rows 8.4 / 8.8, 700 rows 9.2 / 11.6.
+constexpr int64_t kEpilogueSteps = 4;
+constexpr int64_t kPartialBytesPerQuarterStep = 128 << 10;
 constexpr int64_t kFinestSteps = 4;
 constexpr int64_t kFewPartialBytes = 5 << 20;
 // The dense form (no split: its row count is known on the device only) takes the same 128 x 64
@@ -773,7 +781,7 @@ struct QkvPlan {
   int64_t splits = 1;       // slices of the hidden dimension (> 1: QKV_PARTIAL)
   int64_t split_steps = 0;  // k-steps per slice
 };
-QkvPlan qkv_plan(int64_t rows, int64_t features, int64_t k_steps, bool allow_split) {
+QkvPlan qkv_plan(int64_t rows, int64_t features, int64_t k_steps, bool allow_split, bool rope) {
   QkvPlan pl;
   const int64_t nft = (features + 255) / 256;
   int64_t best = 0;
@@ -799,9 +807,14 @@ QkvPlan qkv_plan(int64_t rows, int64_t features, int64_t k_steps, bool allow_spl
       pl.bj = rows <= 64 ? 1 : 0;
       const int64_t fit = pl.bj == 1 ? std::max<int64_t>(kCus - 16, pl.tiles) / pl.tiles
                                      : (2 * kCus) / pl.tiles;
-      const int64_t s = std::max<int64_t>(
-          std::min<int64_t>(fit, k_steps / kMinSplitSteps),
+      const int64_t coarse = std::min<int64_t>(fit, k_steps / kMinSplitSteps);
+      int64_t s = std::max<int64_t>(
+          coarse,
           std::min<int64_t>({fit, k_steps / kFinestSteps, kFewPartialBytes / (rows * features * 4)}));
+      if (coarse <= 1 && s > 1 && !rope &&
+          4 * (k_steps - (k_steps + s - 1) / s) <
+              4 * kEpilogueSteps + s * rows * features * 4 / kPartialBytesPerQuarterStep)
+        s = 1;
       if (s > 1) {
         pl.split_steps = (k_steps + s - 1) / s;
         pl.splits = (k_steps + pl.split_steps - 1) / pl.split_steps;
@@ -871,7 +884,7 @@ int launch_qkv_dense(const char* fn, QkvArgs a, const int32_t* positions, void* 
   a.out = static_cast<char*>(out);
   a.o_s_row = out_stride * 2;
   return launch_qkv<QKV_DENSE>(fn, a, dtype, st,
-                               qkv_plan(a.num_rows, a.num_features, a.k_steps, false));
+                               qkv_plan(a.num_rows, a.num_features, a.k_steps, false, false));
 }
 
 // Workspace of the split form: the RoPE table first, then (split product) the slices.
@@ -894,7 +907,7 @@ extern "C" int64_t sb_qkv_projection_paged_workspace_size(int64_t num_rows, int6
   if (num_rows <= 0 || num_q_heads <= 0 || num_kv_heads < 0 || head_dim <= 0 || hidden_dim <= 0)
     return 0;
   const int64_t features = (num_q_heads + 2 * num_kv_heads) * head_dim;
-  const QkvPlan pl = qkv_plan(num_rows, features, hidden_dim / kTK, true);
+  const QkvPlan pl = qkv_plan(num_rows, features, hidden_dim / kTK, true, rope != 0);
   const int64_t part = pl.splits > 1 ? pl.splits * num_rows * features * 4 : 0;
   return qkv_table_bytes(num_rows, head_dim, rope != 0) + part;
 }
@@ -931,7 +944,7 @@ extern "C" int sb_qkv_projection_paged(
   a.kv_features = kvf;
   a.head_dim = static_cast<int>(head_dim);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const QkvPlan pl = qkv_plan(num_rows, a.num_features, a.k_steps, true);
+  const QkvPlan pl = qkv_plan(num_rows, a.num_features, a.k_steps, true, inv_freq != nullptr);
   const int64_t ws_need = sb_qkv_projection_paged_workspace_size(
       num_rows, num_q_heads, num_kv_heads, head_dim, hidden_dim, inv_freq ? 1 : 0);
   if (ws_need > 0) {

@@ -358,3 +358,20 @@ def test_masked_projection_numbers_the_live_tiles(dev, live):
     got = tk.masked_qkv_projection(x.to(dev), w.to(dev), mask.to(dev))
     _assert_proj_close(got, ref.masked_qkv_projection(x, w, mask), _absdot(x, w))
     assert not bool(got.cpu()[~mask].any())
+
+
+@pytest.mark.parametrize("n_rows,hidden,hq,hkv,d", [
+    (42, 512, 4, 1, 64), (43, 512, 4, 1, 64),       # two slices of four steps: 128 KB from 43 rows
+    (597, 896, 4, 1, 64), (598, 896, 4, 1, 64),     # three of five: 21 times 128 KB from 598 rows
+    (600, 1536, 2, 1, 64)])                         # 24 steps: split at any row count
+def test_projection_without_rope_splits_where_it_pays(dev, n_rows, hidden, hq, hkv, d):
+    from semblend_amd import _lib
+
+    features = (hq + 2 * hkv) * d
+    steps = hidden // 64
+    size = _lib.size_query("sb_qkv_projection_paged_workspace_size", n_rows, hq, hkv, d, hidden, 0)
+    slices = size // (n_rows * features * 4)
+    saved = steps - -(-steps // max(slices, 1))
+    assert (slices > 1) == (n_rows not in (43, 598)) and (slices < 2 or saved >= 4)
+    x, w, b, pos, bt, cache = _case(700, hidden, hq, hkv, d, n_rows, torch.bfloat16, 770 + n_rows)
+    _check_paged(dev, x, w, b, pos, bt, cache, hq, hkv, d, None, backend="fused")
