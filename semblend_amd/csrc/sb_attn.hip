@@ -188,6 +188,9 @@ struct AttnArgs {
   int ksplit_first;           // keys of a row tile's first chunk (multiple of kTileKeys)
   int max_chunks;             // chunks of the longest key range (chunk_count(kv_len))
   int device_split;           // 1: ksplit, max_chunks and n_tiles follow the device row count
+  int late_from;              // > 0: a middle row's position from here on takes late_ksplit and
+  int late_ksplit;            // late_chunks instead
+  int late_chunks;
   int64_t n_tiles;            // row tiles per kv head used for the partial layout
   int tile_rows;              // flattened query rows per workgroup tile
   float* part_o;              // [Hkv][n_tiles][max_chunks][128][D] fp32, or nullptr
@@ -459,8 +462,11 @@ constexpr int kItemsPerSlot = SB_ATTN_ITEMS_PER_SLOT;
 // than the shorter items give. A call whose items are too few for the slots splits finer, because
 // there the time is one item's serial chain of tiles (about 1.5 us each with a CU to itself):
 // until about 256 items run (one per CU) or 40000 (row, chunk) partials are written, whichever
-// comes first, and no finer than 128 keys. Contexts of at most 384 keys stay whole (a merge
-// launch costs what the split would save: 300 tokens, 5 rows 9.5 us whole, 11.4 us in 128s).
+// comes first, and no finer than 128 keys. Contexts of at most 384 keys, or 512 with many row
+// tiles, stay whole (a merge launch costs what the split would save: 300 tokens, 5 rows 9.5 us
+// whole, 11.4 us in 128s; 426 tokens, all rows of 64 / 8 heads 20.8 and 24.1 in 320s; dense, 28
+// heads, all of 400 rows 24.5 and 28.3 in 128s; but 467 tokens, 51 rows of 32 / 8 heads 21.4 and
+// 17.2 in 128s).
 // Chunks of 512 against this rule, 28 / 4 heads x 128 and (in parentheses) 32 / 8 x 128, graph
 // replays: 10 rows of 1000 tokens 20.2 -> 13.6 us (19.6 -> 12.8); 40 of 4096 29.2 -> 24.9
 // (24.9 -> 20.7); 8 of 8000 21.6 -> 17.9 (22.1 -> 18.9); past either limit it loses: 200 rows of
@@ -468,9 +474,10 @@ constexpr int kItemsPerSlot = SB_ATTN_ITEMS_PER_SLOT;
 // against 31.2 in 512s.
 // tile_keys: sum over the launch of row tiles x KV heads x keys; row_keys: of rows x KV heads x
 // keys.
-__host__ __device__ inline int64_t min_chunk(int64_t tile_keys, int64_t row_keys,
+// t: row tiles x KV heads.
+__host__ __device__ inline int64_t min_chunk(int64_t t, int64_t tile_keys, int64_t row_keys,
                                              int64_t kv_len) {
-  if (kv_len <= 384) return 512;
+  if (kv_len <= 384 || (kv_len <= 512 && t > 32)) return 512;
   const int64_t a = tile_keys / 256, b = row_keys / 40000;
   const int64_t ks = ((a > b ? a : b) + 63) / 64 * 64;
   return ks < 128 ? 128 : (ks > 512 ? 512 : ks);
@@ -502,34 +509,79 @@ __host__ __device__ inline int64_t item_keys(int64_t t, int64_t whole_keys, int6
                        kTileKeys - 1) / kTileKeys * kTileKeys;
   return fit > 2 * w ? w : (fit > w ? fit : w);
 }
-// Key-range split of a call. The dense drop-in derives it on the device with this same rule;
-// host plans (`planned`), which order the items of known positions longest first, start from
-// items of W keys. rows_kv: flattened rows of one KV head.
+// Two splits of one call: for rows that lie early in the context (their key ranges rise to kv_len,
+// item_keys) and for late ones, of which no item ends early. The middle row's position says which:
+// positions[rows / 2] >= late_from on the device takes the late one (any order of the positions is
+// correct). W, the average work of a slot, counts on ranges that average half the context.
+//   * Up to kEvenTiles row tiles x KV heads, W of 512 keys and more: late rows, which here are also
+//     uniform ones, take even chunks, as many as fit one round with every range whole, so that
+//     neither the items that end early nor a last tile of few rows decide between one round and
+//     two. Up to 16 all rows take them. Speed against items of W keys, geometric means over 33-64
+//     tiles with W below / above 1000: uniform rows 1.23 and 1.07 (item_keys 0.98 and 1.00), the
+//     last half of the context 1.22 and 1.09 (0.88, 0.87), the last rows 1.46 and 1.25 (1.06,
+//     1.04); a quarter of the rows at the start and the rest uniform 1.22 and 1.05, where item_keys
+//     has 1.25 and 1.19.
+//   * Up to 2 kEvenTiles, W of 512 to 2303 keys: even chunks for the last half.
+//   * Where even chunks would leave more than an eighth of the slots idle, and for W of 2304 to
+//     5499 keys above kEvenTiles, the last half takes W itself (uniform rows of 20613 tokens in 52
+//     tiles: W 135 us, 4 even chunks 145; the last half in more tiles: item_keys 0.88 of W's speed).
+// Planned launches, whose items are ordered by known positions, start from W. The dense drop-in,
+// whose workgroups derive the split by themselves, takes item_keys for all rows: choosing by the
+// position cost each of them the quotients and a load (28 heads x 128, 614 rows of 4096: 55.8 ->
+// 58.9 us).
 struct KeySplit {
   int ksplit;
   int max_chunks;
 };
-__host__ __device__ inline KeySplit key_split(int64_t rows_kv, int64_t n_tiles,
-                                              int64_t num_kv_heads, int64_t kv_len,
-                                              int64_t block_size, bool paged,
-                                              bool planned = false) {
+struct KeySplits {
+  KeySplit early, late;
+  int64_t late_from;  // the middle row's position from which `late` is taken (where they differ)
+};
+constexpr int64_t kEvenTiles = 64;
+constexpr int64_t kEvenAlways = 16;
+__host__ __device__ inline KeySplit clamp_split(int64_t ks, int64_t least, int64_t cap,
+                                                int64_t kv_len) {
   const int64_t kv_pad = (kv_len + kTileKeys - 1) / kTileKeys * kTileKeys;
-  const int64_t t = n_tiles * num_kv_heads;
-  int64_t ks = planned || n_tiles < 2
-                   ? t * (kv_len / 2) / (kResidentSlots * kItemsPerSlot)
-                   : item_keys(t, (t + num_kv_heads) * (kv_len / 2), t * (kv_len / 2));
   ks = ks / kTileKeys * kTileKeys;
-  const int64_t least = min_chunk(n_tiles * num_kv_heads * kv_len,
-                                  rows_kv * num_kv_heads * kv_len, kv_len);
   if (ks < least) ks = least;
-  if (paged) {
-    const int64_t cap = chunk_cap(block_size);
-    if (ks > cap) ks = cap;
-  }
+  if (ks > cap) ks = cap;
   if (ks > kv_pad) ks = kv_pad;
   if (ks < kTileKeys) ks = kTileKeys;
   const int64_t chunks = (kv_len + ks - 1) / ks;
   return KeySplit{static_cast<int>(ks), static_cast<int>(chunks < 1 ? 1 : chunks)};
+}
+// Key-range splits of a call (dense: late = early).
+// rows_kv: flattened rows of one KV head (a row count's splits are no finer than those of fewer
+// rows in as many tiles).
+__host__ __device__ inline KeySplits key_splits(int64_t rows_kv, int64_t n_tiles,
+                                                int64_t num_kv_heads, int64_t kv_len,
+                                                int64_t block_size, bool paged,
+                                                bool planned = false) {
+  const int64_t cap =
+      paged ? chunk_cap(block_size) : (kv_len + kTileKeys - 1) / kTileKeys * kTileKeys;
+  const int64_t t = n_tiles * num_kv_heads;
+  const int64_t w = t * (kv_len / 2) / (kResidentSlots * kItemsPerSlot);
+  const int64_t least = min_chunk(t, t * kv_len, rows_kv * num_kv_heads * kv_len, kv_len);
+  int64_t early = w, late = w, from = 0;
+  if (!planned && n_tiles >= 2) {
+    early = late = item_keys(t, (t + num_kv_heads) * (kv_len / 2), t * (kv_len / 2));
+    if (paged && t < kResidentSlots && w >= 512 && w < 5500 && kv_len <= 0x7fffffff) {
+      const uint32_t each = static_cast<uint32_t>(kResidentSlots) / static_cast<uint32_t>(t);
+      const int64_t even = ((static_cast<uint32_t>(kv_len) + each - 1) / each + kTileKeys - 1) /
+                           kTileKeys * kTileKeys;
+      const bool full = even <= cap && each * t >= kResidentSlots - kResidentSlots / 8;
+      if (t <= kEvenTiles) {
+        late = full ? even : w;
+        from = kv_len / 64 * 27;
+        if (t <= kEvenAlways) early = late;
+      } else if (w >= 2304 || t <= 2 * kEvenTiles) {
+        late = full && w < 2304 ? even : w;
+        from = kv_len / 64 * 45;
+      }
+    }
+  }
+  return KeySplits{clamp_split(early, least, cap, kv_len), clamp_split(late, least, cap, kv_len),
+                   from};
 }
 // Work-item decode shared by the attention and merge kernels.
 struct Item {
@@ -559,13 +611,21 @@ __device__ __forceinline__ Item decode_item(const AttnArgs& a, int64_t n_tiles_l
 
 namespace sb {
 
-// The device-derived split of a dense call (device_split), from its row-tile count.
+// The part of the split that only the device knows: of a dense call (device_split) by its row
+// count, else by the middle row's position (n_rows > 0).
 template <bool F32>
-__device__ __forceinline__ void apply_device_split(AttnArgs& a, int64_t rows_kv,
+__device__ __forceinline__ void apply_device_split(AttnArgs& a, int64_t n_rows, int64_t rows_kv,
                                                    int64_t n_tiles_live) {
-  if (!a.device_split) return;
-  const KeySplit sp = F32 ? key_split_f32(n_tiles_live, a.num_kv_heads, a.kv_len, a.head_dim)
-                          : key_split(rows_kv, n_tiles_live, a.num_kv_heads, a.kv_len, 1, false);
+  if (!a.device_split) {
+    if (!F32 && a.late_from > 0 && a.positions[n_rows / 2] >= a.late_from) {
+      a.ksplit = a.ksplit_first = a.late_ksplit;
+      a.max_chunks = a.late_chunks;
+    }
+    return;
+  }
+  const KeySplit sp =
+      F32 ? key_split_f32(n_tiles_live, a.num_kv_heads, a.kv_len, a.head_dim)
+          : key_splits(rows_kv, n_tiles_live, a.num_kv_heads, a.kv_len, 1, false).early;
   a.ksplit = sp.ksplit;
   a.ksplit_first = sp.ksplit;
   a.max_chunks = sp.max_chunks;
@@ -617,7 +677,7 @@ attn_mfma_kernel(const AttnBatch batch) {
   const int64_t rows_kv = n_rows * a.group;
   const int64_t n_tiles_live = (rows_kv + TR - 1) / TR;
   if (n_tiles_live <= 0) return;  // no rows (uniform)
-  apply_device_split<false>(a, rows_kv, n_tiles_live);
+  apply_device_split<false>(a, n_rows, rows_kv, n_tiles_live);
   const Item item = decode_item(a, n_tiles_live, item_b);
   if (item.tile < 0 || item.chunk >= a.max_chunks) return;  // uniform, before any barrier
   const int kvh = item.kvh;
@@ -1392,13 +1452,15 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const AttnBatch batch) 
   int64_t mb = select_request(batch, a, blockIdx.x / CG, true);
   mb = mb * CG + blockIdx.x % CG;
   const int TR = a.tile_rows;
-  const int64_t rows_kv = attn_num_rows(a) * a.group;
+  const int64_t n_rows = attn_num_rows(a);
+  const int64_t rows_kv = n_rows * a.group;
   const int64_t n_tiles_live = (rows_kv + TR - 1) / TR;
+  if (n_tiles_live <= 0) return;  // no rows (uniform)
+  apply_device_split<DT == SB_DTYPE_F32>(a, n_rows, rows_kv, n_tiles_live);
   if (!STRIDED) {
     merge_unit<DT, D, CG>(a, mb, n_tiles_live, rows_kv, red);
     return;
   }
-  apply_device_split<DT == SB_DTYPE_F32>(a, rows_kv, n_tiles_live);
   const int64_t units = n_tiles_live * a.num_kv_heads * (TR / 32 * CG);
   for (int64_t u = mb; u < units; u += gridDim.x) {
     merge_unit<DT, D, CG>(a, u, n_tiles_live, rows_kv, red);
@@ -1522,16 +1584,16 @@ namespace {
 constexpr int64_t kMergeStrideGrid = 2048;  // merge workgroups of a device-split call
 // Launches the merge of split-key partials over `units` units of 32 rows. Rows of more than
 // kMergeBatch chunks spread them over four groups of lanes where the units are too few to hide a
-// row's chain of loads behind other units (22 chunks of 40 x 4 rows of 8 heads: 5.5 us); with
-// many units the chains overlap, and four groups only add idle loads (28 heads of 614 rows, 7
-// chunks: 22.5 us against 11.5 with one). A strided merge counts the units of every row that could
-// be computed, and half as many of them are the line (307 of 1024 rows of 14 heads: 6.5 us with
-// four groups, 5.2 with one).
-constexpr int64_t kMergeWideUnits = 512;
+// row's chain of loads behind other units (22 chunks of 40 x 4 rows of 8 heads: 5.5 us; 32 heads of
+// 23 rows of 6827 tokens, 256 units: the call 37.6 us, 39.9 with one group); with more units the
+// chains overlap, and four groups only add idle loads (14 / 2 heads x 64, 1056 rows of 3161, 464
+// units of 7 chunks: 33.5 us against 29.1 with one; 32 / 8 x 128, 299 of 3255, 320 units: 37.8
+// against 32.9). A strided merge counts the units of every row that could be computed.
+constexpr int64_t kMergeWideUnits = 256;
 #define SB_MERGE_LAUNCH(DT, D, STRIDED, units, max_chunks, st, args)                          \
   do {                                                                                        \
     const int64_t sb_cap = (STRIDED) ? kMergeStrideGrid : int64_t{0x7fffffff};                \
-    if ((max_chunks) > kMergeBatch && (units) * ((STRIDED) ? 2 : 1) <= kMergeWideUnits) {     \
+    if ((max_chunks) > kMergeBatch && (units) <= kMergeWideUnits) {                           \
       const dim3 sb_mg(static_cast<unsigned>(std::min<int64_t>((units) * 4, sb_cap)));        \
       SB_LAUNCH("attn_merge", (attn_merge_kernel<DT, D, STRIDED, 4>), sb_mg, dim3(256), st,   \
                 args);                                                                        \
@@ -1566,6 +1628,9 @@ struct Plan {
   int ksplit;
   int ksplit_first;
   int max_chunks;
+  KeySplit late;       // of late rows, where that is another split (max_chunks 0: the same)
+  int64_t late_from;
+  int most_chunks;     // of both
   int tile_rows;
   int64_t n_tiles;
   int64_t part_bytes;  // bytes of partials (O then m/l), 0 when no tile splits
@@ -1582,21 +1647,31 @@ Plan make_plan(int64_t rows_upper, int64_t group, int64_t num_kv_heads, int64_t 
     pl.ksplit_first = op->ks_first;
     pl.max_chunks = op->max_chunks;
   } else {
-    const KeySplit sp = f32 ? key_split_f32(pl.n_tiles, num_kv_heads, kv_len, head_dim)
-                            : key_split(rows_upper * group, pl.n_tiles, num_kv_heads, kv_len,
-                                      block_size, paged);
+    KeySplit sp;
+    if (f32) {
+      sp = key_split_f32(pl.n_tiles, num_kv_heads, kv_len, head_dim);
+    } else {
+      const KeySplits both = key_splits(rows_upper * group, pl.n_tiles, num_kv_heads, kv_len,
+                                        block_size, paged);
+      sp = both.early;
+      if (both.late.ksplit != sp.ksplit) {
+        pl.late = both.late;
+        pl.late_from = both.late_from;
+      }
+    }
     pl.ksplit = sp.ksplit;
     pl.ksplit_first = sp.ksplit;
     pl.max_chunks = sp.max_chunks;
   }
-  if (pl.max_chunks > 1)
+  pl.most_chunks = std::max(pl.max_chunks, pl.late.max_chunks);
+  if (pl.most_chunks > 1)
     pl.part_bytes =
-        num_kv_heads * pl.n_tiles * pl.max_chunks * pl.tile_rows * (head_dim + 2) * 4;
+        num_kv_heads * pl.n_tiles * pl.most_chunks * pl.tile_rows * (head_dim + 2) * 4;
   return pl;
 }
 
 // Split of a call whose row count is known only on the device (dense drop-in): the kernels
-// derive it from that count with key_split; the launch covers the largest item count and
+// derive it from that count with key_splits; the launch covers the largest item count and
 // the workspace the largest partials over every possible count of row tiles (of a count's
 // splits, the one with the fewest rows is the finest).
 struct DeviceSplitBounds {
@@ -1608,13 +1683,18 @@ DeviceSplitBounds device_split_bounds(int64_t n_tiles_upper, int64_t num_kv_head
                                       int64_t kv_len, int tile_rows, int64_t head_dim,
                                       bool f32) {
   DeviceSplitBounds b{0, 1, 0};
-  for (int64_t t = 1; t <= n_tiles_upper; ++t) {
-    const KeySplit sp = f32 ? key_split_f32(t, num_kv_heads, kv_len, head_dim)
-                            : key_split((t - 1) * tile_rows + 1, t, num_kv_heads, kv_len, 1, false);
+  auto cover = [&](int64_t t, const KeySplit& sp) {
     b.items = std::max<int64_t>(b.items, t * num_kv_heads * sp.max_chunks);
     b.most_chunks = std::max(b.most_chunks, sp.max_chunks);
     if (sp.max_chunks > 1)
       b.part_rows = std::max<int64_t>(b.part_rows, num_kv_heads * t * sp.max_chunks * tile_rows);
+  };
+  for (int64_t t = 1; t <= n_tiles_upper; ++t) {
+    if (f32) {
+      cover(t, key_split_f32(t, num_kv_heads, kv_len, head_dim));
+      continue;
+    }
+    cover(t, key_splits((t - 1) * tile_rows + 1, t, num_kv_heads, kv_len, 1, false).early);
   }
   return b;
 }
@@ -1638,7 +1718,7 @@ int launch_attention_f32(const char* fn, AttnArgs a, int64_t rows_upper, void* w
   int64_t part_rows =
       pl.part_bytes > 0 ? a.num_kv_heads * pl.n_tiles * pl.max_chunks * pl.tile_rows : 0;
   int64_t gx = pl.n_tiles * a.num_kv_heads * pl.max_chunks;
-  int most_chunks = pl.max_chunks;
+  int most_chunks = pl.most_chunks;
   if (a.device_split) {
     const DeviceSplitBounds b =
         device_split_bounds(pl.n_tiles, a.num_kv_heads, a.kv_len, pl.tile_rows, a.head_dim, true);
@@ -1699,11 +1779,16 @@ int launch_attention(const char* fn, AttnArgs a, int32_t dtype, int64_t rows_upp
     a.max_chunks = pl.max_chunks;
     a.n_tiles = pl.n_tiles;
     a.tile_rows = pl.tile_rows;
-    int64_t part_rows = pl.part_bytes > 0 ? a.num_kv_heads * pl.n_tiles * pl.max_chunks *
+    if (pl.late.max_chunks > 0 && !a.device_split) {
+      a.late_from = static_cast<int>(pl.late_from);
+      a.late_ksplit = pl.late.ksplit;
+      a.late_chunks = pl.late.max_chunks;
+    }
+    int64_t part_rows = pl.part_bytes > 0 ? a.num_kv_heads * pl.n_tiles * pl.most_chunks *
                                                 pl.tile_rows
                                           : 0;
-    int64_t gx = pl.n_tiles * a.num_kv_heads * pl.max_chunks;
-    int most_chunks = pl.max_chunks;
+    int64_t gx = pl.n_tiles * a.num_kv_heads * pl.most_chunks;
+    int most_chunks = pl.most_chunks;
     if (a.device_split) {
       // The kernels split by the device row count: cover every count that can occur.
       const DeviceSplitBounds b =
@@ -1792,7 +1877,7 @@ VarlenPlan make_varlen_plan(int64_t num_reqs, const int64_t* rows, const int64_t
   });
   int64_t ks = item_keys(tiles, whole, work);
   ks = ks / kTileKeys * kTileKeys;
-  const int64_t least = min_chunk(tile_keys, row_keys, kv_max);
+  const int64_t least = min_chunk(tiles, tile_keys, row_keys, kv_max);
   if (ks < least) ks = least;
   const int64_t cap = chunk_cap(block_size);
   if (ks > cap) ks = cap;
@@ -1962,7 +2047,7 @@ HostOrderPlan plan_paged_order(const int32_t* pos, int64_t num_rows, int64_t gro
     kend[static_cast<size_t>(t)] = m + 1;
   }
   const KeySplit base =
-      key_split(rows_kv, n_tiles, num_kv_heads, kv_len, block_size, true, true);
+      key_splits(rows_kv, n_tiles, num_kv_heads, kv_len, block_size, true, true).early;
   AttnArgs geo{};
   auto cost_of = [&](int chunk, int64_t t) -> int64_t {  // 64-key tiles of one item
     const int64_t k0 = chunk_begin(geo, chunk);

@@ -430,3 +430,48 @@ def test_key_split_rules_cover_every_key(dev, hq, hkv, d, ctx, rows):
         [rows, short], [nb, nb])
     assert_attn_close(both[:rows].cpu()[sel], want)
     assert_attn_close(both[rows:], got[:short].float().cpu())
+
+
+@pytest.mark.parametrize("hq,hkv,d,ctx,rows", [
+    (28, 4, 128, 6573, 273),    # few row tiles: even chunks longer than 512 keys
+    (28, 4, 128, 2630, 490),    # few row tiles: one round in chunks of 512
+    (32, 8, 128, 513, 300),     # one key past the contexts that stay whole
+    (28, 4, 128, 8247, 786),    # late rows: even chunks
+    (28, 4, 64, 15291, 1304)])  # late rows: the average work of a slot
+@pytest.mark.parametrize("order", ["uniform", "late", "late first"])
+def test_key_split_by_the_first_position(dev, hq, hkv, d, ctx, rows, order):
+    """Splits chosen by the row count and by the first row's position: uniform rows, the last rows
+    of the context, and a first row past 3/8 of it before rows that are not."""
+    g = gen(640 + ctx)
+    nb = -(-ctx // 16)
+    kv = randn((nb + 8, 2, hkv, 16, d), torch.bfloat16, 641)
+    bt = torch.randperm(nb + 8, generator=g)[:nb].to(torch.int32)
+    if order == "late":
+        pos = torch.arange(ctx - rows, ctx, dtype=torch.int32)
+    else:
+        pos = torch.randperm(ctx, generator=g)[:rows].sort().values.to(torch.int32)
+    if order == "late first":
+        pos = pos.flip(0)
+    q = randn((rows, hq, d), torch.bfloat16, 642)
+    got = tk.partial_prefill_attention_paged(q.to(dev), kv.to(dev), bt.to(dev), pos.to(dev)).cpu()
+    sel = torch.randperm(rows, generator=g)[:10].sort().values
+    sel[0], sel[-1] = 0, rows - 1
+    assert_attn_close(got[sel], ref.partial_attention_paged(q[sel], kv, bt, pos[sel]))
+
+
+@pytest.mark.parametrize("first,rows", [(1535, 500), (1536, 500), (3500, 596), (4095, 1), (0, 4096)])
+def test_dense_split_by_the_first_position(dev, first, rows):
+    """The device-derived split on both sides of 3/8 of the context (28 heads: 56 to 84 row tiles
+    of 2 and 3 per head)."""
+    h, s, d = 28, 4096, 64
+    q, k, v = (randn((h, s, d), torch.bfloat16, 650 + i) for i in range(3))
+    mask = torch.zeros(s, dtype=torch.bool)
+    mask[first:first + rows] = True
+    got = tk.partial_prefill_attention(q.to(dev), k.to(dev), v.to(dev), mask.to(dev)).cpu()
+    sel = torch.tensor(sorted({first, first + rows // 3, first + rows - 1}))
+    for hh in (0, h - 1):
+        for p in sel.tolist():
+            w = torch.softmax((k[hh, :p + 1].double() @ q[hh, p].double()) / math.sqrt(d), 0)
+            want = (w[:, None] * v[hh, :p + 1].double()).sum(0)
+            assert_attn_close(got[hh, p][None, None], want.float()[None, None])
+    assert not bool(got[:, ~mask].any())
