@@ -34,7 +34,7 @@
 //
 // fp32 path (fp32 tensors, head_dim 64 or 128): the fp32 matrix cores, sb_attn_f32.h.
 //
-// VALU path (any other head_dim, alignment or scale): one wave per (row, q-head), a 64-key chunk
+// VALU path (any other head_dim, alignment or scale, and the smallest fp32 calls): one wave per (row, q-head), a 64-key chunk
 // per step, one key per lane for the scores and the PV sum over the chunk per output dimension.
 
 #include "sb_common.h"
@@ -1614,6 +1614,16 @@ bool f32_path(int32_t dtype, int64_t head_dim) {
   return dtype == SB_DTYPE_F32 && (head_dim == 64 || head_dim == 128);
 }
 
+// fp32 calls that the VALU kernel's one launch finishes before the matrix-core kernel has set up,
+// loaded its first tile and (past 128 or 64 keys) merged: short contexts with few products. VALU /
+// matrix cores, us: 14 / 2 heads x 64, 20 tokens, 4 rows 5.3 / 7.9; 80 tokens, 80 rows 10.6 / 11.8
+// (5.7 million products), 100 tokens, 100 rows 12.1 / 11.9 (9.0 million); 160 tokens, 20 rows 14.2 /
+// 15.3, 200 tokens 17.5 / 15.3; 28 / 4 x 128, 80 tokens, 20 rows 14.5 / 16.0, 100 tokens 16.6 / 15.9;
+// 64 tokens, 64 rows 16.1 / 12.2 (14.7 million).
+bool f32_tiny(int64_t rows, int64_t q_heads, int64_t kv_len, int64_t head_dim) {
+  return kv_len * head_dim <= 160 * 64 && rows * q_heads * kv_len * head_dim <= (7 << 20);
+}
+
 // A host-planned launch of the single-request paged attention (sb_partial_attention_paged_plan):
 // the key split (first chunk, later chunks) and the dispatch order of the work items.
 struct OrderPlan {
@@ -1826,7 +1836,8 @@ int launch_attention(const char* fn, AttnArgs a, int32_t dtype, int64_t rows_upp
     SB_ATT_CASE(SB_DTYPE_F16, 64)
 #undef SB_ATT_CASE
   }
-  if (f32_path(dtype, a.head_dim) && aligned16 && a.scale_log2 > 0.f && a.kv_len <= 0x7fffff00)
+  if (f32_path(dtype, a.head_dim) && aligned16 && a.scale_log2 > 0.f && a.kv_len <= 0x7fffff00 &&
+      !f32_tiny(rows_upper, static_cast<int64_t>(a.num_kv_heads) * a.group, a.kv_len, a.head_dim))
     return launch_attention_f32(fn, a, rows_upper, workspace, workspace_bytes, st);
   if (a.head_dim > kValuMaxDim) return fail(fn, "head_dim above 512 is not supported");
   if (rows_upper > 0x7fffffff) return fail(fn, "too many rows");

@@ -475,3 +475,30 @@ def test_dense_split_by_the_first_position(dev, first, rows):
             want = (w[:, None] * v[hh, :p + 1].double()).sum(0)
             assert_attn_close(got[hh, p][None, None], want.float()[None, None])
     assert not bool(got[:, ~mask].any())
+
+
+@pytest.mark.parametrize("hq,hkv,d,seq,rows", [
+    (14, 2, 64, 160, 9), (14, 2, 64, 161, 9),        # the smallest calls: one launch up to 160 x 64
+    (28, 4, 128, 80, 25), (28, 4, 128, 80, 26),      # ... and 7340032 products
+    (14, 2, 64, 193, 1), (14, 2, 64, 192, 9),        # key tiles of 64, one key past and whole
+    (32, 8, 128, 97, 17)])                           # key tiles of 32, one key past
+def test_paged_fp32_smallest_calls(dev, hq, hkv, d, seq, rows):
+    from semblend_amd import _lib
+
+    q, kv, bt, _ = _paged_case(hq, hkv, d, seq, seq, torch.float32, 660 + seq)
+    pos = torch.randperm(seq, generator=gen(661))[:rows].sort().values.to(torch.int32)
+    pos[-1] = seq - 1
+    q = q[:rows]
+    want = ref.partial_attention_paged(q, kv, bt, pos)
+    args = [t.to(dev) for t in (q, kv, bt, pos)]
+    _lib.kernel_timing(True)
+    try:
+        got = tk.partial_prefill_attention_paged(*args)
+        torch.cuda.synchronize()
+        valu = _lib.kernel_time("attn_valu")[1]
+    finally:
+        _lib.kernel_timing(False)
+    keys = bt.numel() * kv.shape[3]
+    assert valu == (keys * d <= 160 * 64 and rows * hq * keys * d <= 7 << 20)
+    # two orders of summing d products and up to seq weighted values: a few 2^-24 of |out| <= 1
+    assert float((got.cpu() - want).abs().max()) <= 5e-6 * max(1.0, float(want.abs().max()))
