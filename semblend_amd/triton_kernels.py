@@ -714,9 +714,8 @@ class PartialPrefillResult:
     kv_cache: [num_layers, 2, num_heads, seq_len, head_dim] assembled target cache;
     positions_computed / positions_reused: compute-mask counts;
     computation_ratio: positions_computed / seq_len;
-    *_time_ms: HIP-event timings of the scatter (the donor rows' index and the assembly of the
-    cache), projection and attention stages (the attention without its output projection) and
-    of the whole call.
+    *_time_ms: HIP-event timings of the scatter, projection (with the compaction of the mask)
+    and attention stages (the attention without its output projection) and of the whole call.
     """
 
     output: torch.Tensor
@@ -861,7 +860,7 @@ def _prefill_stages(dev, hidden_states, donor_kv, qkv_weight, output_projection,
     part_at = ((seq_len + 1) * 4 + 255) // 256 * 256
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)  # positions, count, partials
     index = torch.empty(seq_len, dtype=torch.int32, device=dev)
-    ev = [torch.cuda.Event(enable_timing=True) for _ in range(6)]
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(5)]
     es = hidden_states.element_size()
     with _lib.on_device(dev):
         stream = torch.cuda.current_stream(dev)
@@ -870,7 +869,6 @@ def _prefill_stages(dev, hidden_states, donor_kv, qkv_weight, output_projection,
         ev[0].record(stream)
         _lib.call("sb_prefill_index", mask.data_ptr(), _lib.ptr(dpos), _lib.ptr(tpos),
                   num_pairs, seq_len, donor_kv.shape[3], index.data_ptr(), pos, st)
-        ev[1].record(stream)
         if fused:
             qkv = torch.empty((seq_len, 3 * feats), dtype=dt, device=dev)
             bias = None if qkv_bias is None else qkv_bias.contiguous()
@@ -882,13 +880,13 @@ def _prefill_stages(dev, hidden_states, donor_kv, qkv_weight, output_projection,
             qkv = torch.nn.functional.linear(
                 hidden_states.float(), qkv_weight.float(),
                 None if qkv_bias is None else qkv_bias.float()).to(dt)
-        ev[2].record(stream)
+        ev[1].record(stream)
         # (the first launches are under way while the rest is allocated)
         cache = torch.empty((num_layers, 2, num_heads, seq_len, head_dim), dtype=dt, device=dev)
         _lib.call("sb_prefill_assemble", cache.data_ptr(), donor_kv.data_ptr(), qkv.data_ptr(),
                   index.data_ptr(), num_layers, num_heads, seq_len, head_dim,
                   _lib.strides(donor_kv), 3 * feats, code, st)
-        ev[3].record(stream)
+        ev[2].record(stream)
         attn = torch.empty((seq_len, feats), dtype=torch.float32, device=dev)
         out = torch.empty((seq_len, output_projection.shape[0]), dtype=dt, device=dev)
         bias32 = None if output_bias is None else output_bias.float().contiguous()
@@ -901,27 +899,25 @@ def _prefill_stages(dev, hidden_states, donor_kv, qkv_weight, output_projection,
                   pos + part_at, ws_bytes - part_at, num_heads, seq_len, head_dim,
                   float(scale), _lib.i64_array((head_dim, 3 * feats, 1)), heads_major,
                   heads_major, _lib.i64_array((head_dim, feats, 1)), code, st)
-        ev[4].record(stream)
+        ev[3].record(stream)
         _lib.call("sb_prefill_output_projection", out.data_ptr(), attn.data_ptr(),
                   output_projection.data_ptr(), _lib.ptr(bias32), mask.data_ptr(), pos,
                   seq_len, feats, output_projection.shape[0], feats,
                   output_projection.stride(0), out.stride(0), code, st)
         count.copy_(ws[4 * seq_len:4 * seq_len + 4], non_blocking=True)
-        ev[5].record(stream)
-        ev[5].synchronize()
+        ev[4].record(stream)
+        ev[4].synchronize()
     num_computed = int(count.view(torch.int32)[0])
-    index_ms = ev[0].elapsed_time(ev[1])
-    assemble_ms = ev[2].elapsed_time(ev[3])
     return PartialPrefillResult(
         output=out,
         kv_cache=cache,
         positions_computed=num_computed,
         positions_reused=seq_len - num_computed,
         computation_ratio=num_computed / seq_len,
-        scatter_time_ms=index_ms + assemble_ms,
-        projection_time_ms=ev[1].elapsed_time(ev[2]),
-        attention_time_ms=ev[3].elapsed_time(ev[4]),
-        total_time_ms=ev[0].elapsed_time(ev[5]),
+        scatter_time_ms=ev[1].elapsed_time(ev[2]),
+        projection_time_ms=ev[0].elapsed_time(ev[1]),
+        attention_time_ms=ev[2].elapsed_time(ev[3]),
+        total_time_ms=ev[0].elapsed_time(ev[4]),
     )
 
 
