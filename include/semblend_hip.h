@@ -446,7 +446,10 @@ int sb_nope_permute_paged_kv_layers(const uint64_t* kv_layer_ptrs, int64_t num_l
  * (head, seq, dim) given in q_strides[3], k_strides[3], v_strides[3] and o_strides[3].
  * compute_mask: device uint8 array of S entries. The rows are compacted on the device, so the
  * call never synchronises with the host. Rows whose mask is 0 are written as zeros.
- * workspace: device buffer of sb_partial_prefill_attention_workspace_size(...) bytes.
+ * workspace: device buffer of sb_partial_prefill_attention_workspace_size(...) bytes: the
+ * compacted positions and the fp32 partials of the largest key split that any number of computed
+ * rows takes (the number is known on the device only), so some tens of MB also for small calls
+ * (28 heads x 512 x 128: 15 MB, 14 x 1024 x 64 fp32: 30 MB; fp32 calls at most 102 MB).
  * Replaces semblend_core/triton_kernels.py:655-734 (kernel :531-652, CPU path :717-732). */
 int64_t sb_partial_prefill_attention_workspace_size(int64_t num_heads, int64_t seq_len,
                                                     int64_t head_dim, int32_t dtype);
@@ -464,7 +467,9 @@ int sb_partial_prefill_attention(void* out, const void* q, const void* k, const 
  * kv_cache [NB, 2, Hkv, bs, D] with kv_strides[5] = (block, kv, head, pos, dim).
  * positions should be ascending (any order is correct; ascending is fastest).
  * workspace: device buffer of sb_partial_attention_paged_workspace_size(...) bytes (fp32
- * partials of the split key range; the size may be 0, then workspace may be NULL).
+ * partials of the split key range; the size may be 0, then workspace may be NULL). Calls of few
+ * rows split finest, so they need some tens of MB too (32 / 8 heads x 128: 23 MB for 40 rows of
+ * 4096 tokens, 68 MB for one row of 32768).
  * No reference counterpart: the reference attention is MHA over contiguous K/V
  * (semblend_core/triton_kernels.py:655-734); this is the GQA + paged form its callers need. */
 int64_t sb_partial_attention_paged_workspace_size(int64_t num_rows, int64_t num_q_heads,
@@ -490,7 +495,7 @@ int sb_partial_attention_paged(void* out, const void* q, const void* kv_cache,
  * written, or a negative SB_ERR_INVALID_ARGUMENT on bad arguments. For a dtype / head_dim
  * the MFMA kernel does not take, max_chunks is 0 and there are no items.
  * sb_partial_attention_paged_planned takes the device copy of the item order (plan + 3), its
- * length (refused unless it is max_chunks * ceil(num_rows * group / 128) * num_kv_heads,
+ * length (refused unless it is max_chunks * ceil(num_rows * group / 256) * num_kv_heads,
  * the launch's item count) and the three split values, otherwise the arguments of
  * sb_partial_attention_paged; its
  * workspace is sb_partial_attention_paged_planned_workspace_size(...) bytes. The order only

@@ -193,8 +193,8 @@ struct AttnArgs {
   int late_chunks;
   int64_t n_tiles;            // row tiles per kv head used for the partial layout
   int tile_rows;              // flattened query rows per workgroup tile
-  float* part_o;              // [Hkv][n_tiles][max_chunks][128][D] fp32, or nullptr
-  float* part_ml;             // [Hkv][n_tiles][max_chunks][128][2] fp32 (m, l)
+  float* part_o;              // [Hkv][n_tiles][max_chunks][tile_rows][D] fp32, or nullptr
+  float* part_ml;             // [Hkv][n_tiles][max_chunks][tile_rows][2] fp32 (m, l)
   const int32_t* item_order;  // single-request launches: work item of each workgroup (a
                               // host-planned order), or nullptr (workgroup b runs item b)
 };

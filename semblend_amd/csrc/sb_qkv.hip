@@ -737,9 +737,9 @@ int qkv_common(const char* fn, QkvArgs* a, const void* hidden, const void* weigh
 // CU) when the big tiles leave more than half the CUs idle, or leave some idle while the
 // small ones fit one round of two per CU. (BJ = 4 spilled 5-6 VGPRs and never cost less than
 // BJ = 2 in this model: at most a tie.) When even the 128 x 128 tiles number fewer than the
-// CUs (a few hundred rows at the 7B shape), the split form also splits the hidden dimension
-// over grid.y, into slices of at least kMinSplitSteps k-steps (QKV_PARTIAL and the summing
-// epilogue). Qwen2.5-7B shape (3584 -> 4608 features), graph replays on one box, interleaved:
+// CUs (a few hundred rows at the 7B shape), the split form also splits the hidden dimension over
+// the workgroups of one launch (QKV_PARTIAL and the summing epilogue): into slices of at least
+// kMinSplitSteps k-steps, or finer ones as below. Qwen2.5-7B shape (3584 -> 4608 features), graph replays on one box, interleaved:
 // slices of at least 12 steps 28-30 us at 64 rows (6 steps: 32 us, 19: 35 us), 30.5 us at 128
 // and 35.5 us at 256 (library 28, 33, 46 us); small tiles from 1024 to 1536 rows 61-72 us
 // against 75-77 us with the 256-feature tiles, which stay faster from 2048 rows (97 against
@@ -751,9 +751,11 @@ constexpr int64_t kCus = 256;
 constexpr int64_t kMinSplitSteps = SB_QKV_MIN_SPLIT_STEPS;
 // Finer slices, down to kFinestSteps, while the partial products stay below kFewPartialBytes: a
 // step's loads take about one memory latency however few products it has, so a slice's time is
-// its number of steps until the partials cost more. Qwen2.5-0.5B shape (896 -> 1152) 65 rows 14.0
-// -> 9.8 us, 300 rows 14.3 -> 11.9; the 7B shape at 200 rows in slices of 7 steps (26 MB) 27.6 us
-// against 24.0 in slices of 14, at 64 rows 6 slices (7 MB) 15.2 us against 14.5 with 4.
+// its number of steps until the partials cost more. Where the line lies: six shapes from 896 ->
+// 1152 to 5120 -> 7168 features, 8 to 400 rows, with RoPE, geometric mean of the time against 5 MB,
+// up to / above 64 rows: no finer slices 1.086 / 1.044 (at most 1.57), 3 MB 0.989 / 1.003 (0.90 to
+// 1.16), 8 MB 1.004 / 1.008 (to 1.14), 12 MB 1.002 / 1.023 (to 1.28), 20 MB 1.002 / 1.055 (to 1.42:
+// 2048 -> 2560, 160 rows 14.4 -> 20.4 us).
 // Up to 64 rows take 128 x 64 tiles with three steps of loads in flight, one workgroup per CU
 // (16 CUs left to the RoPE table). Graph replays before and after: 7B shape 1 / 16 / 64 rows
 // 17.7 / 18.8 / 20.8 -> 11.9 / 12.6 / 14.5 us, 0.5B 12.9 / 12.7 / 13.2 -> 7.7 / 8.4 / 9.5 us,

@@ -266,8 +266,14 @@ def masked_qkv_projection(
 
 
 
-# Row counts in which qkv_projection_paged(backend="auto") takes the library GEMM (measured at
-# the Qwen2.5-7B shape: the fused kernel is faster or level below and above this range).
+# Row counts in which qkv_projection_paged(backend="auto") takes the library GEMM. Graph replays,
+# fused / library, bf16 with RoPE (fp16 within 2%, at 4096 -> 6144 2% slower in the fused form):
+#   rows            384        512        513        768        1024       1100       1280
+#   4096 -> 6144    35.7/38.6  41.7/41.8  45.5/42.6  55.4/53.9  64.4/61.3  68.4/68.5  73.1/72.1
+#   3584 -> 4608    29.7/31.3  33.2/35.9  36.4/36.8  41.9/41.4  48.3/50.3  53.4/51.7  56.6/57.0
+#    896 -> 1152    12.2/14.8  13.0/15.2  13.1/15.4  14.4/16.4  15.1/18.1  16.1/18.4  16.4/19.8
+# The range is the widest shape's, where the library is 3-9% ahead; the middle one is level in it,
+# and the narrowest pays 2-3 us for it.
 _LIBRARY_PROJECTION_ROWS = (513, 1024)
 
 
@@ -300,10 +306,10 @@ def qkv_projection_paged(
     kernel of its own (bias, RoPE, one rounding, Q and the paged K/V write); "auto" takes the
     library form from 513 to 1024 rows and the fused form otherwise (which splits the hidden
     dimension when its row tiles are too few for the CUs). Qwen2.5-7B shape, graph replays on
-    one MI355X, fused / library: 14.5 / 21 us at 64 rows, 21 / 25.5 at 128, 26 / 39 at 256,
-    33.5 / 36.5 at 512, 42 / 42 at 768, 49 / 50.5 at 1024, 76 / 80 at 2048, 89 / 98 at 2458,
-    158 / 165 at 4096. The fused form needs no fp32 intermediate of rows x features. Both accumulate in
-    fp32 and round once.
+    one MI355X, fused / library: 14.5 / 21 us at 64 rows (the call itself 15.9), 21 / 25.5 at 128,
+    26 / 39 at 256, 33 / 36 at 512, 42 / 41.5 at 768, 48.5 / 50.5 at 1024, 76 / 80 at 2048, 89 / 98
+    at 2458, 158 / 165 at 4096. The fused form needs no fp32 intermediate of rows x features. Both
+    accumulate in fp32 and round once.
     Fuses the masked projection (semblend_core/triton_kernels.py:451-522) with the K/V write
     of partial_prefill (:904-909), compacted and paged; no reference counterpart.
     """
