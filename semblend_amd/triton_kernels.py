@@ -774,22 +774,29 @@ def partial_prefill(
     return _prefill_composed(dev, *args)
 
 
+# torch's own (unexported) queries of its tracer, dispatch modes and functorch transforms; a torch
+# without one of them is asked through its public form, or has no such thing.
+_tracing = getattr(torch._C, "_is_tracing", torch.jit.is_tracing)
+_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", lambda: 0)
+_functorch = getattr(torch._C, "_functorch", None)
+_transform = getattr(_functorch, "peek_interpreter_stack", lambda: None)
+_wrapped = getattr(_functorch, "is_functorch_wrapped_tensor", lambda t: True)
+
+
 def _torch_only_sees_values(tensors) -> bool:
     """Whether a call on these tensors may go to kernels that read their memory, past torch's
     operators: no tensor subclass, no forward-mode tangent among them, no functorch transform
     (vmap, jvp, grad) around a wrapped one, and no tracer or dispatch mode that follows the
     operators. (Reverse mode is looked up by the caller.)"""
-    if torch._C._is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
+    if _tracing() or _dispatch_modes() > 0:
         return False
-    if any(type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter
-           for t in tensors if t is not None):
+    given = [t for t in tensors if t is not None]
+    if any(type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter for t in given):
         return False
-    if forward_ad._current_level >= 0 and any(
-            forward_ad.unpack_dual(t).tangent is not None for t in tensors if t is not None):
+    if getattr(forward_ad, "_current_level", 0) >= 0 and any(
+            forward_ad.unpack_dual(t).tangent is not None for t in given):
         return False
-    functorch = torch._C._functorch
-    return functorch.peek_interpreter_stack() is None or not any(
-        functorch.is_functorch_wrapped_tensor(t) for t in tensors if t is not None)
+    return _transform() is None or not any(_wrapped(t) for t in given)
 
 
 def _prefill_stages_ok(hidden_states, donor_kv, qkv_weight, output_projection, donor_positions,
