@@ -302,8 +302,9 @@ def test_paged_gqa_planned_unsorted_and_fp32(dev):
     (4, 4, 64, 700, 700, 16),     # no GQA, every row
     (64, 16, 64, 2000, 1100, 16)])  # enough row tiles to run unsplit
 def test_paged_fp32_tiles_and_splits(dev, hq, hkv, d, seq, rows, bs):
-    """Row tiles of 64, key tiles of 4096 / head_dim and the key split at their edges; a call
-    whose caller sized no workspace (an empty launch plan through the C entry) runs unsplit."""
+    """Row tiles of 64, key tiles of 4096 / head_dim and the key split at their edges (the shortest
+    contexts take the one-launch kernel); a call whose caller sized no workspace (an empty launch
+    plan through the C entry) runs unsplit."""
     q, kv, bt, pos = _paged_case(hq, hkv, d, seq, rows, torch.float32, 400 + d + rows, bs=bs)
     qd, kvd, btd, posd = q.to(dev), kv.to(dev), bt.to(dev), pos.to(dev)
     want = ref.partial_attention_paged(q, kv, bt, pos)
@@ -477,15 +478,16 @@ def test_dense_split_by_the_first_position(dev, first, rows):
     assert not bool(got[:, ~mask].any())
 
 
-@pytest.mark.parametrize("hq,hkv,d,seq,rows", [
-    (14, 2, 64, 160, 9), (14, 2, 64, 161, 9),        # the smallest calls: one launch up to 160 x 64
-    (28, 4, 128, 80, 25), (28, 4, 128, 80, 26),      # ... and 7340032 products
-    (14, 2, 64, 193, 1), (14, 2, 64, 192, 9),        # key tiles of 64, one key past and whole
-    (32, 8, 128, 97, 17)])                           # key tiles of 32, one key past
-def test_paged_fp32_smallest_calls(dev, hq, hkv, d, seq, rows):
+@pytest.mark.parametrize("hq,hkv,d,seq,rows,bs", [
+    (14, 2, 64, 160, 9, 16), (14, 2, 64, 161, 9, 16),    # the smallest calls: up to 160 x 64
+    (28, 4, 128, 80, 25, 16), (28, 4, 128, 80, 26, 16),  # ... and 7340032 products
+    (14, 2, 64, 193, 1, 16), (14, 2, 64, 192, 9, 16),    # key tiles of 64, one key past and whole
+    (32, 8, 128, 97, 17, 16),                            # key tiles of 32, one key past
+    (28, 4, 128, 150, 33, 24)])                          # blocks that are no power of two
+def test_paged_fp32_smallest_calls(dev, hq, hkv, d, seq, rows, bs):
     from semblend_amd import _lib
 
-    q, kv, bt, _ = _paged_case(hq, hkv, d, seq, seq, torch.float32, 660 + seq)
+    q, kv, bt, _ = _paged_case(hq, hkv, d, seq, seq, torch.float32, 660 + seq, bs=bs)
     pos = torch.randperm(seq, generator=gen(661))[:rows].sort().values.to(torch.int32)
     pos[-1] = seq - 1
     q = q[:rows]

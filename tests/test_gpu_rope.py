@@ -367,8 +367,9 @@ def test_nope_permute_paged_kv(dev, dtype):
 @pytest.mark.parametrize("seq,pairs", [(1, 3), (1023, 1023), (1025, 2000), (3000, 32768),
                                        (3000, 32769)])
 def test_rope_k_index_edges(dev, seq, pairs):
-    """The per-position pair index at the edges of its workgroups and of the list length that one
-    launch scans: repeated donor positions rotate in pair order, out-of-range ones not at all."""
+    """The per-position pair index at the edges of its workgroups and in lists of both its forms (one
+    launch up to 24576 pairs): repeated donor positions rotate in pair order, out-of-range ones not
+    at all."""
     g = gen(60 + seq)
     k = randn((1, 1, seq, 64), torch.float32, 61)
     dp = torch.randint(-2, seq + 2, (pairs,), generator=g).to(torch.int32)
