@@ -463,10 +463,10 @@ constexpr int kItemsPerSlot = SB_ATTN_ITEMS_PER_SLOT;
 // there the time is one item's serial chain of tiles (about 1.5 us each with a CU to itself):
 // until about 256 items run (one per CU) or 40000 (row, chunk) partials are written, whichever
 // comes first, and no finer than 128 keys. Contexts of at most 384 keys, or 512 with many row
-// tiles, stay whole (a merge launch costs what the split would save: 300 tokens, 5 rows 9.5 us
-// whole, 11.4 us in 128s; 426 tokens, all rows of 64 / 8 heads 20.8 and 24.1 in 320s; dense, 28
-// heads, all of 400 rows 24.5 and 28.3 in 128s; but 467 tokens, 51 rows of 32 / 8 heads 21.4 and
-// 17.2 in 128s).
+// tiles or next to none, stay whole (a merge launch costs what the split would save: 300 tokens, 5
+// rows 9.5 us whole, 11.4 us in 128s; 426 tokens, all rows of 64 / 8 heads 20.8 and 24.1 in 320s;
+// dense, 28 heads, all of 400 rows 24.5 and 28.3 in 128s; 389 tokens, 2 uniform rows of 14 / 2 heads
+// x 64 9.4 and 11.0; but 467 tokens, 51 rows of 32 / 8 heads 21.4 and 17.2 in 128s).
 // Chunks of 512 against this rule, 28 / 4 heads x 128 and (in parentheses) 32 / 8 x 128, graph
 // replays: 10 rows of 1000 tokens 20.2 -> 13.6 us (19.6 -> 12.8); 40 of 4096 29.2 -> 24.9
 // (24.9 -> 20.7); 8 of 8000 21.6 -> 17.9 (22.1 -> 18.9); past either limit it loses: 200 rows of
@@ -477,7 +477,7 @@ constexpr int kItemsPerSlot = SB_ATTN_ITEMS_PER_SLOT;
 // t: row tiles x KV heads.
 __host__ __device__ inline int64_t min_chunk(int64_t t, int64_t tile_keys, int64_t row_keys,
                                              int64_t kv_len) {
-  if (kv_len <= 384 || (kv_len <= 512 && t > 32)) return 512;
+  if (kv_len <= 384 || (kv_len <= 512 && (t > 32 || t < 4))) return 512;
   const int64_t a = tile_keys / 256, b = row_keys / 40000;
   const int64_t ks = ((a > b ? a : b) + 63) / 64 * 64;
   return ks < 128 ? 128 : (ks > 512 ? 512 : ks);
