@@ -34,8 +34,9 @@
 //
 // fp32 path (fp32 tensors, head_dim 64 or 128): the fp32 matrix cores, sb_attn_f32.h.
 //
-// VALU path (any other head_dim, alignment or scale, and the smallest fp32 calls): one wave per (row, q-head), a 64-key chunk
-// per step, one key per lane for the scores and the PV sum over the chunk per output dimension.
+// VALU path (any other head_dim, alignment or scale, and the smallest fp32 calls): one wave per
+// (row, q-head), a 64-key chunk per step, one key per lane for the scores and the PV sum over the
+// chunk per output dimension.
 
 #include "sb_common.h"
 
@@ -1710,8 +1711,8 @@ DeviceSplitBounds device_split_bounds(int64_t n_tiles_upper, int64_t num_kv_head
 }
 
 // The fp32 kernel, on tensors of `in_dtype` (fp16 / bf16 elements are widened as they are staged:
-// the same results as on fp32 copies of them). Callers that sized no workspace for it (a launch plan is empty for fp32, and
-// a caller may hold a smaller fixed buffer) run unsplit.
+// the same results as on fp32 copies of them). Callers that sized no workspace for it (a launch
+// plan is empty for fp32) run unsplit.
 int launch_attention_f32(const char* fn, AttnArgs a, int64_t rows_upper, void* workspace,
                          int64_t workspace_bytes, hipStream_t st,
                          int32_t in_dtype = SB_DTYPE_F32) {

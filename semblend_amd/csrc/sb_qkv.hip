@@ -739,8 +739,8 @@ int qkv_common(const char* fn, QkvArgs* a, const void* hidden, const void* weigh
 // BJ = 2 in this model: at most a tie.) When even the 128 x 128 tiles number fewer than the
 // CUs (a few hundred rows at the 7B shape), the split form also splits the hidden dimension over
 // the workgroups of one launch (QKV_PARTIAL and the summing epilogue): into slices of at least
-// kMinSplitSteps k-steps, or finer ones as below. Qwen2.5-7B shape (3584 -> 4608 features), graph replays on one box, interleaved:
-// slices of at least 12 steps 28-30 us at 64 rows (6 steps: 32 us, 19: 35 us), 30.5 us at 128
+// kMinSplitSteps k-steps, or finer ones as below. Qwen2.5-7B shape (3584 -> 4608 features), graph
+// replays on one box, interleaved: slices of at least 12 steps 28-30 us at 64 rows (6 steps: 32 us, 19: 35 us), 30.5 us at 128
 // and 35.5 us at 256 (library 28, 33, 46 us); small tiles from 1024 to 1536 rows 61-72 us
 // against 75-77 us with the 256-feature tiles, which stay faster from 2048 rows (97 against
 // 113 us).
